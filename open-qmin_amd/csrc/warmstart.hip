@@ -21,6 +21,7 @@
 //    chunks' partial sums are added in a fixed order by wgrad_reduce_kernel.
 //  * Elementwise kernels: features, loss gradient, bias gradient, Adam with the
 //    BF16 (and mirrored) weight copies, writing the prediction into a lattice.
+#include <algorithm>
 #include <cstdint>
 
 #include "qmin_internal.h"
@@ -35,8 +36,8 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // BF16 pairs with the sign bit set (negative values and -0) -> +0
 __device__ __forceinline__ unsigned relu2(unsigned w) {
-    const unsigned lo = (w & 0x8000u) ? 0xffffu : 0u, hi = (w & 0x80000000u) ? 0xffff0000u : 0u;
-    return w & ~(lo | hi);
+    typedef short v2s __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(v2s, w), v2s{0, 0}));
 }
 
 constexpr int kTaps = 27;
@@ -61,6 +62,15 @@ __device__ __forceinline__ long long tap_site(int x, int y, int z, int tap, int 
     return wrapd(x + dil * dx, lx) + (long long)lx * (wrapd(y + dil * dy, ly) + (long long)ly * wrapd(z + dil * dz, lz));
 }
 
+// One tile of the forward kernel: `rows` consecutive lattice rows (y fastest),
+// of each a segment of w sites, as the host chose it (choose_conv_tile).
+struct ConvTile {
+    int w, nseg;    // segment length along x, segments per row
+    int rows;       // rows per work-group
+    int halo;       // sites staged on each side of a segment: dil, or 0
+    int fold;       // 1: a step stages the rows of one (dy, dz) for its three taps; 0: the sites of one tap
+};
+
 struct ConvArgs {
     const uint16_t* x;     // [n][cin] bf16
     const uint16_t* wt;    // [27][cout][cin] bf16
@@ -70,144 +80,281 @@ struct ConvArgs {
     float* yf;             // [n][cout] fp32 output
     long long n;
     int cin, cout, lx, ly, lz, dil, reluIn;
+    ConvTile tile;
+    int nblocks;
+    int vecX, vecW, vecOut;   // x, wt, and ybf with mask are 16-byte aligned (else x at 32 or fewer channels and
+                              // wt take 8-byte loads, and ybf element stores)
 };
 
-constexpr int kFwdMT = 4;   // 16-site row tiles per wave in the forward kernel
+constexpr int kFwdMT = 4;                                     // 16-site row tiles per wave in the forward kernel
+constexpr int kFwdSites = kWsThreads / 64 * 16 * kFwdMT;      // sites a work-group computes
+constexpr int kFwdSlots = 320;                                // sites it stages per step at most
+constexpr int kFwdRows = 32;                                  // rows it covers at most
 
-// Each wave owns 64 consecutive sites (kFwdMT tiles of 16) and all output
-// channels: per tap and 16-channel slice it gathers one 8-byte A fragment per
-// tile and reads each B fragment once from LDS for all four tiles.  The
-// work-group stages a tap's weights [cout][cin] in LDS (rows padded by 4 BF16
-// against bank conflicts), double-buffered across taps.
+// 3x3x3 dilated periodic convolution as an implicit GEMM.  A work-group owns up
+// to 256 sites of whole row segments, each wave 64 of them and all output
+// channels.  For each (dy, dz) it stages the segments' neighbour rows in LDS
+// once, ReLU applied, with the weights of the three taps that differ in dx
+// only: these read the same rows at three offsets.  The next step's rows and
+// weights are loaded into registers while the matrix instructions of the
+// current one run.  Rows in LDS are padded (8 BF16 at 64 channels, 4 below), so
+// that the 16 sites of a fragment fall on different banks.
+//
+// The matrix cores need each operand byte once per tap from LDS (64 + 64 B per
+// clock and CU of the 128 it gives at full MFMA rate); gathering every tap's
+// operand from L2 instead, as 27 separate reads of each site, left the kernel
+// waiting on those gathers: kFwdTimes
 template <int NT, int KT>
-__global__ void __launch_bounds__(kWsThreads) conv_fwd_kernel(ConvArgs a) {
+__global__ void __launch_bounds__(kWsThreads, 2) conv_fwd_kernel(ConvArgs a) {
     // K32: 32 input channels per matrix instruction (for 64 input channels; with
-    // 32, one such step per tap ran 9% slower at 128^3 than two 16-channel
-    // ones); LDS rows padded by 8 BF16 so that every lane's 16-byte weight
-    // fragment stays 16-byte aligned
+    // 32, one such step per tap ran 9% slower at 128^3 than two 16-channel ones)
     constexpr bool K32 = KT == 4;
     constexpr int CO = NT * 16, CI = KT * 16, RS = CI + (K32 ? 8 : 4);   // LDS row stride in BF16
-    __shared__ __align__(16) uint2 sW[2][CO * RS / 4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int CPS = CI / 8;                                          // 16-byte pieces of a site
+    constexpr int NA = (kFwdSlots * CPS + kWsThreads - 1) / kWsThreads;  // pieces a thread stages per step: rows,
+    constexpr int NW = (3 * CO * CPS + kWsThreads - 1) / kWsThreads;     // weights
+    constexpr int OS = CO + 8;                                           // row stride of the output tile
+    constexpr int IN = (kFwdSlots + 3 * CO) * RS, OUT = kFwdSites * OS;
+    __shared__ __align__(16) uint16_t sBuf[IN > OUT ? IN : OUT];
+    __shared__ int sSite[kFwdSites];           // site of each output row of the tile, from its first row on; -1: none
+    __shared__ long long sRow[9][kFwdRows];    // first input element of each row's neighbour row at (dy, dz)
+    uint16_t* const sX = sBuf;
+    uint16_t* const sW = sBuf + kFwdSlots * RS;
+
+    const ConvTile T = a.tile;
+    // each XCD gets a contiguous run of tiles, whose neighbour rows share its L2
+    const int qb = a.nblocks >> 3, rb = a.nblocks & 7, xcd = blockIdx.x & 7;
+    const int blk = xcd * qb + min(xcd, rb) + (blockIdx.x >> 3);
+    const int x0 = (blk % T.nseg) * T.w;
+    const long long r0 = (long long)(blk / T.nseg) * T.rows, nrows = (long long)a.ly * a.lz;
+    const int pitch = T.w + 2 * T.halo;   // staged sites of a row
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kq = lane >> 4, l16 = lane & 15;
-    const long long wbase = ((long long)blockIdx.x * (kWsThreads / 64) + wave) * (16 * kFwdMT);
-    const bool waveActive = wbase < a.n;
-    int xs[kFwdMT], ys[kFwdMT], zs[kFwdMT];
-    bool valid[kFwdMT];
+
+    {
+        const int r = tid / T.w, x = x0 + tid % T.w;
+        sSite[tid] = (r < T.rows && r0 + r < nrows && x < a.lx) ? r * a.lx + x : -1;
+    }
+    for (int e = tid; e < 9 * kFwdRows; e += kWsThreads) {
+        const int st = e / kFwdRows, r = e % kFwdRows;
+        const long long row = r0 + r < nrows ? r0 + r : 0;
+        const int y = wrapd(int(row % a.ly) + (st % 3 - 1) * a.dil, a.ly);
+        const int z = wrapd(int(row / a.ly) + (st / 3 - 1) * a.dil, a.lz);
+        sRow[st][r] = (y + (long long)a.ly * z) * a.lx * CI;
+    }
+    // slots of this lane's sites at dx = -1, 0, 1
+    int off[kFwdMT][3];
 #pragma unroll
     for (int mt = 0; mt < kFwdMT; ++mt) {
-        const long long s = wbase + 16 * mt + l16;
-        valid[mt] = s < a.n;
-        const long long sc = valid[mt] ? s : 0;
-        xs[mt] = int(sc % a.lx);
-        ys[mt] = int((sc / a.lx) % a.ly);
-        zs[mt] = int(sc / ((long long)a.lx * a.ly));
+        const int m = wave * (16 * kFwdMT) + 16 * mt + l16;
+        const int r = m / T.w, x = m % T.w;
+        const bool in = r < T.rows;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            int slot = x + T.halo;
+            if (T.fold) slot = T.halo ? x + d * a.dil : wrapd(x + (d - 1) * a.dil, a.lx);
+            off[mt][d] = in ? (r * pitch + slot) * RS : 0;
+        }
     }
+    // pieces this thread stages: LDS offset, row and first input element
+    const int pieces = T.rows * pitch * CPS;
+    int stOff[NA], stRow[NA], stX[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int e = tid + kWsThreads * i;
+        const int slot = e / CPS, c = e % CPS, r = slot / pitch, p = slot % pitch;
+        stOff[i] = e < pieces ? slot * RS + c * 8 : -1;
+        stRow[i] = e < pieces ? r : 0;
+        stX[i] = wrapd(x0 - T.halo + p, a.lx) * CI + c * 8;
+    }
+    const int steps = T.fold ? 9 : kTaps, tps = T.fold ? 3 : 1;
+    const int wpieces = tps * CO * CPS;
+
+    v4u ra[NA], rw[NW];
+    auto get = [&](const uint16_t* src, bool vec) {
+        if (vec) return *reinterpret_cast<const v4u*>(src);
+        const uint2 lo = reinterpret_cast<const uint2*>(src)[0], hi = reinterpret_cast<const uint2*>(src)[1];
+        return v4u{lo.x, lo.y, hi.x, hi.y};
+    };
+    auto load = [&](int step) {
+        const long long* base = sRow[T.fold ? step : step / 3];
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            if (stOff[i] >= 0) {
+                int x = stX[i];
+                if (!T.fold) x = wrapd(x / CI + (step % 3 - 1) * a.dil, a.lx) * CI + x % CI;
+                ra[i] = get(a.x + base[stRow[i]] + x, K32 || a.vecX);
+            }
+        const uint16_t* src = a.wt + (long long)step * tps * CO * CI;
+#pragma unroll
+        for (int i = 0; i < NW; ++i)
+            if (tid + kWsThreads * i < wpieces) rw[i] = get(src + 8 * (tid + kWsThreads * i), a.vecW);
+    };
+    auto put = [&](uint16_t* dst, v4u v) {
+        if constexpr (K32) {
+            *reinterpret_cast<v4u*>(dst) = v;
+        } else {   // rows of 8-byte alignment
+            reinterpret_cast<uint2*>(dst)[0] = uint2{v[0], v[1]};
+            reinterpret_cast<uint2*>(dst)[1] = uint2{v[2], v[3]};
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            if (stOff[i] >= 0) {
+                v4u v = ra[i];
+                if (a.reluIn) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = relu2(v[j]);
+                }
+                put(sX + stOff[i], v);
+            }
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const int e = tid + kWsThreads * i;
+            if (e < wpieces) put(sW + (e / CPS) * RS + (e % CPS) * 8, rw[i]);
+        }
+    };
+
     v4f acc[kFwdMT][NT];
 #pragma unroll
     for (int mt = 0; mt < kFwdMT; ++mt)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[mt][t] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    auto stage = [&](int tap, int buf) {
-        const uint2* src = reinterpret_cast<const uint2*>(a.wt + (long long)tap * CO * CI);
-        for (int e = threadIdx.x; e < CO * CI / 4; e += kWsThreads) {
-            const int co = e / (CI / 4), c4 = e % (CI / 4);
-            sW[buf][co * (RS / 4) + c4] = src[e];
-        }
-    };
-    stage(0, 0);
-    __syncthreads();
-    for (int tap = 0; tap < kTaps; ++tap) {
-        const int buf = tap & 1;
-        // the other buffer was last read in tap - 1, before the barrier below
-        if (tap + 1 < kTaps) stage(tap + 1, buf ^ 1);
-        if (K32 && waveActive) {
-            const uint16_t* xr[kFwdMT];
-#pragma unroll
-            for (int mt = 0; mt < kFwdMT; ++mt)
-                xr[mt] = a.x + tap_site(xs[mt], ys[mt], zs[mt], tap, a.dil, a.lx, a.ly, a.lz) * CI + kq * 8;
+    auto tap = [&](int d, const uint16_t* w) {
+        if constexpr (K32) {
 #pragma unroll
             for (int k2 = 0; k2 < KT / 2; ++k2) {
                 v8bf av[kFwdMT];
 #pragma unroll
-                for (int mt = 0; mt < kFwdMT; ++mt) {
-                    v4u raw = *reinterpret_cast<const v4u*>(xr[mt] + k2 * 32);
-                    if (a.reluIn) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) raw[j] = relu2(raw[j]);
-                    }
-                    if (!valid[mt]) raw = v4u{0u, 0u, 0u, 0u};
-                    av[mt] = __builtin_bit_cast(v8bf, raw);
-                }
+                for (int mt = 0; mt < kFwdMT; ++mt)
+                    av[mt] = __builtin_bit_cast(
+                        v8bf, *reinterpret_cast<const v4u*>(sX + off[mt][d] + k2 * 32 + kq * 8));
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    const v4u wraw =
-                        *reinterpret_cast<const v4u*>(&sW[buf][((t * 16 + l16) * RS + k2 * 32 + kq * 8) / 4]);
-                    const v8bf bv = __builtin_bit_cast(v8bf, wraw);
+                    const v8bf bv = __builtin_bit_cast(
+                        v8bf, *reinterpret_cast<const v4u*>(w + (t * 16 + l16) * RS + k2 * 32 + kq * 8));
 #pragma unroll
                     for (int mt = 0; mt < kFwdMT; ++mt)
                         acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[mt], bv, acc[mt][t], 0, 0, 0);
                 }
             }
-        } else if (waveActive) {
-            const uint16_t* xr[kFwdMT];
-#pragma unroll
-            for (int mt = 0; mt < kFwdMT; ++mt)
-                xr[mt] = a.x + tap_site(xs[mt], ys[mt], zs[mt], tap, a.dil, a.lx, a.ly, a.lz) * CI + kq * 4;
+        } else {
 #pragma unroll
             for (int kt = 0; kt < KT; ++kt) {
                 v4s av[kFwdMT];
 #pragma unroll
-                for (int mt = 0; mt < kFwdMT; ++mt) {
-                    const uint2 raw = *reinterpret_cast<const uint2*>(xr[mt] + kt * 16);
-                    av[mt][0] = short(raw.x & 0xffffu);
-                    av[mt][1] = short(raw.x >> 16);
-                    av[mt][2] = short(raw.y & 0xffffu);
-                    av[mt][3] = short(raw.y >> 16);
-                    if (a.reluIn) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) av[mt][j] = av[mt][j] < 0 ? short(0) : av[mt][j];
-                    }
-                    if (!valid[mt]) av[mt] = v4s{0, 0, 0, 0};
-                }
+                for (int mt = 0; mt < kFwdMT; ++mt)
+                    av[mt] = __builtin_bit_cast(
+                        v4s, *reinterpret_cast<const uint2*>(sX + off[mt][d] + kt * 16 + kq * 4));
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    const uint2 wraw = sW[buf][((t * 16 + l16) * RS + kt * 16 + kq * 4) / 4];
-                    v4s bv;
-                    bv[0] = short(wraw.x & 0xffffu);
-                    bv[1] = short(wraw.x >> 16);
-                    bv[2] = short(wraw.y & 0xffffu);
-                    bv[3] = short(wraw.y >> 16);
+                    const v4s bv = __builtin_bit_cast(
+                        v4s, *reinterpret_cast<const uint2*>(w + (t * 16 + l16) * RS + kt * 16 + kq * 4));
 #pragma unroll
                     for (int mt = 0; mt < kFwdMT; ++mt)
                         acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[mt], bv, acc[mt][t], 0, 0, 0);
                 }
             }
         }
+    };
+
+    const long long site0 = r0 * a.lx;
+    __syncthreads();   // sRow
+    load(0);
+    store();
+    __syncthreads();
+    for (int step = 0; step < steps; ++step) {
+        if (step + 1 < steps) load(step + 1);
+        tap(0, sW);
+        if (T.fold) {
+            tap(1, sW + CO * RS);
+            tap(2, sW + 2 * CO * RS);
+        }
+        __syncthreads();
+        if (step + 1 < steps) store();
         __syncthreads();
     }
-    if (!waveActive) return;
+
+    if (a.yf || !a.vecOut) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int co = t * 16 + l16;
+            const float b = a.bias ? a.bias[co] : 0.f;
+#pragma unroll
+            for (int mt = 0; mt < kFwdMT; ++mt) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int site = sSite[wave * (16 * kFwdMT) + 16 * mt + 4 * kq + j];
+                    if (site < 0) continue;
+                    float v = acc[mt][t][j] + b;
+                    const long long o = (site0 + site) * CO + co;
+                    if (a.mask && !(bf2f(a.mask[o]) > 0.f)) v = 0.f;
+                    if (a.yf)
+                        a.yf[o] = v;
+                    else
+                        a.ybf[o] = f2bf(v);
+                }
+            }
+        }
+        return;
+    }
+    // BF16 output through LDS, so that it is stored (and the mask read) in
+    // 16-byte pieces
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int co = t * 16 + l16;
         const float b = a.bias ? a.bias[co] : 0.f;
 #pragma unroll
-        for (int mt = 0; mt < kFwdMT; ++mt) {
+        for (int mt = 0; mt < kFwdMT; ++mt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                sBuf[(wave * (16 * kFwdMT) + 16 * mt + 4 * kq + j) * OS + co] = f2bf(acc[mt][t][j] + b);
+    }
+    __syncthreads();
+    for (int e = tid; e < kFwdSites * (CO / 8); e += kWsThreads) {
+        const int m = e / (CO / 8), c = e % (CO / 8), site = sSite[m];
+        if (site < 0) continue;
+        v4u v = *reinterpret_cast<const v4u*>(sBuf + m * OS + c * 8);
+        const long long o = (site0 + site) * CO + c * 8;
+        if (a.mask) {
+            const v4u mk = *reinterpret_cast<const v4u*>(a.mask + o);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const long long site = wbase + 16 * mt + 4 * kq + j;
-                if (site >= a.n) continue;
-                float v = acc[mt][t][j] + b;
-                const long long o = site * CO + co;
-                if (a.mask && !(bf2f(a.mask[o]) > 0.f)) v = 0.f;
-                if (a.yf)
-                    a.yf[o] = v;
-                else
-                    a.ybf[o] = f2bf(v);
+                if (!(__uint_as_float(mk[j] << 16) > 0.f)) v[j] &= 0xffff0000u;
+                if (!(__uint_as_float(mk[j] & 0xffff0000u) > 0.f)) v[j] &= 0xffffu;
             }
         }
+        *reinterpret_cast<v4u*>(a.ybf + o) = v;
     }
+}
+
+// Tile of the forward kernel for a row length and dilation: the split of a row
+// into equal segments that leaves the fewest of the work-group's site slots
+// empty, staged sites included (whole rows need no halo: their neighbours wrap
+// onto the row itself).  Where a halo of dil sites on both sides never fits,
+// each tap's sites are staged by themselves.
+inline ConvTile choose_conv_tile(int lx, int dil) {
+    ConvTile best{};
+    double bestCost = 1e300;
+    for (int fold = 1; fold >= 0 && bestCost > 1e299; --fold)
+        for (int nseg = 1; nseg <= lx; ++nseg) {
+            const int w = (lx + nseg - 1) / nseg;
+            if (w > kFwdSites) continue;
+            if (w < 16 && nseg > 1) break;
+            ConvTile t{w, (lx + w - 1) / w, 0, (fold && w < lx) ? dil : 0, fold};
+            const long long pitch = w + 2LL * t.halo;
+            if (pitch > kFwdSlots) continue;
+            t.rows = int(std::min<long long>(std::min(kFwdSites / w, kFwdRows), kFwdSlots / pitch));
+            // work-groups per row, and what their staging adds (9 reads per 27 taps of work)
+            const double cost = double(t.nseg) / t.rows * (1.0 + 0.3 * double(t.rows * pitch) / kFwdSites);
+            if (cost < bestCost) {
+                bestCost = cost;
+                best = t;
+            }
+        }
+    return best;
 }
 
 struct WgradArgs {
@@ -488,9 +635,7 @@ inline int grid_for(long long work, int per = kWsThreads) {
 
 template <int NT, int KT>
 hipError_t launch_fwd_t(const ConvArgs& a, hipStream_t s) {
-    const long long waves = (a.n + 16 * kFwdMT - 1) / (16 * kFwdMT);
-    const int blocks = int((waves + 3) / 4);
-    hipLaunchKernelGGL((conv_fwd_kernel<NT, KT>), dim3(blocks), dim3(kWsThreads), 0, s, a);
+    hipLaunchKernelGGL((conv_fwd_kernel<NT, KT>), dim3(a.nblocks), dim3(kWsThreads), 0, s, a);
     return hipGetLastError();
 }
 
@@ -551,6 +696,13 @@ int qm_ws_conv_forward(const void* x, int cin, const void* wt, const float* bias
     a.lz = lz;
     a.dil = dil;
     a.reluIn = reluIn;
+    a.tile = choose_conv_tile(lx, dil);
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    a.vecX = aligned(x);
+    a.vecW = aligned(wt);
+    a.vecOut = aligned(ybf16) && aligned(mask);
+    const long long blocks = ((long long)ly * lz + a.tile.rows - 1) / a.tile.rows * a.tile.nseg;
+    a.nblocks = int(blocks);
     HIP_TRY(launch_fwd(a, static_cast<hipStream_t>(stream)));
     return QM_OK;
 }
