@@ -69,6 +69,10 @@ struct ConvTile {
     int rows;       // rows per work-group
     int halo;       // sites staged on each side of a segment: dil, or 0
     int fold;       // 1: a step stages the rows of one (dy, dz) for its three taps; 0: the sites of one tap
+    // order of the row groups: blocks of kFwdBlock consecutive groups, and within
+    // a block the groups dil planes apart (stride groups) one after the other,
+    // so that the planes z - dil, z and z + dil are found in L2
+    int groups, stride, turns;
 };
 
 struct ConvArgs {
@@ -88,8 +92,9 @@ struct ConvArgs {
 
 constexpr int kFwdMT = 4;                                     // 16-site row tiles per wave in the forward kernel
 constexpr int kFwdSites = kWsThreads / 64 * 16 * kFwdMT;      // sites a work-group computes
-constexpr int kFwdSlots = 320;                                // sites it stages per step at most
+constexpr int kFwdSlots = 288;                                // sites it stages per step at most
 constexpr int kFwdRows = 32;                                  // rows it covers at most
+constexpr int kFwdBlock = 16;                                 // row groups taken together along z
 
 // 3x3x3 dilated periodic convolution as an implicit GEMM.  A work-group owns up
 // to 256 sites of whole row segments, each wave 64 of them and all output
@@ -100,10 +105,15 @@ constexpr int kFwdRows = 32;                                  // rows it covers 
 // current one run.  Rows in LDS are padded (8 BF16 at 64 channels, 4 below), so
 // that the 16 sites of a fragment fall on different banks.
 //
-// The matrix cores need each operand byte once per tap from LDS (64 + 64 B per
-// clock and CU of the 128 it gives at full MFMA rate); gathering every tap's
-// operand from L2 instead, as 27 separate reads of each site, left the kernel
-// waiting on those gathers: kFwdTimes
+// Bound by LDS: at the full BF16 rate a wave's 64 x 64 products would read 128 B
+// per clock and CU from it, all that it gives, before any staging.  Gathering
+// every tap's operand from L2 instead, 27 reads of each site, left the kernel
+// waiting on those gathers.  At 128^3, before and now: 64 -> 64 channels 1.46
+// and 0.65 ms (710 TFLOP/s), 64 -> 16 0.99 and 0.36, 32 -> 64 0.78 and 0.45,
+// 16 -> 32 0.43 and 0.13 ms.  Measured and not kept: 320 slots, with which the
+// 64 -> 16 kernel has two work-groups per CU instead of three (0.52 ms); three
+// waves per SIMD at 32 channels (0.54 ms: spills); the loads after the first tap
+// and a raised wave priority during the taps (no difference).
 template <int NT, int KT>
 __global__ void __launch_bounds__(kWsThreads, 2) conv_fwd_kernel(ConvArgs a) {
     // K32: 32 input channels per matrix instruction (for 64 input channels; with
@@ -126,7 +136,10 @@ __global__ void __launch_bounds__(kWsThreads, 2) conv_fwd_kernel(ConvArgs a) {
     const int qb = a.nblocks >> 3, rb = a.nblocks & 7, xcd = blockIdx.x & 7;
     const int blk = xcd * qb + min(xcd, rb) + (blockIdx.x >> 3);
     const int x0 = (blk % T.nseg) * T.w;
-    const long long r0 = (long long)(blk / T.nseg) * T.rows, nrows = (long long)a.ly * a.lz;
+    const int ord = blk / T.nseg, in = (ord / (kFwdBlock * T.turns)) * kFwdBlock + ord % kFwdBlock;
+    const int group = in + ord / kFwdBlock % T.turns * T.stride;
+    if (in >= T.stride || group >= T.groups) return;   // a partial block or turn
+    const long long r0 = (long long)group * T.rows, nrows = (long long)a.ly * a.lz;
     const int pitch = T.w + 2 * T.halo;   // staged sites of a row
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kq = lane >> 4, l16 = lane & 15;
@@ -355,6 +368,18 @@ inline ConvTile choose_conv_tile(int lx, int dil) {
             }
         }
     return best;
+}
+
+// Order of the tiles, and the work-groups to launch for it.  64 -> 64 channels
+// at 128^3 and dilation 4, where an XCD's L2 holds two planes: 0.67 ms against
+// 0.77 in plain order; blocks of 8 or 32 row groups 0.68 and 0.69 ms.
+inline int order_conv_tiles(ConvTile& t, int ly, int lz, int dil) {
+    const long long rows = (long long)ly * lz;
+    t.groups = int((rows + t.rows - 1) / t.rows);
+    const long long apart = (long long)ly * std::min(dil, lz) / t.rows;
+    t.stride = int(std::max<long long>(1, std::min<long long>(apart, t.groups)));
+    t.turns = (t.groups + t.stride - 1) / t.stride;
+    return int((long long)((t.stride + kFwdBlock - 1) / kFwdBlock) * kFwdBlock * t.turns * t.nseg);
 }
 
 struct WgradArgs {
@@ -701,8 +726,7 @@ int qm_ws_conv_forward(const void* x, int cin, const void* wt, const float* bias
     a.vecX = aligned(x);
     a.vecW = aligned(wt);
     a.vecOut = aligned(ybf16) && aligned(mask);
-    const long long blocks = ((long long)ly * lz + a.tile.rows - 1) / a.tile.rows * a.tile.nseg;
-    a.nblocks = int(blocks);
+    a.nblocks = order_conv_tiles(a.tile, ly, lz, dil);
     HIP_TRY(launch_fwd(a, static_cast<hipStream_t>(stream)));
     return QM_OK;
 }
