@@ -17,8 +17,8 @@
 //  * The input gradient is the same kernel with the taps mirrored and the
 //    weights transposed (Wbd[26 - tap][cin][cout] = Wt[tap][cout][cin]).
 //  * conv_wgrad_kernel: dWt[tap][cout][cin] = sum_site G[site][cout]
-//    X[site + dil*tap][cin], a GEMM over sites per (tap, chunk of sites); the
-//    chunks' partial sums are added in a fixed order by wgrad_reduce_kernel.
+//    X[site + dil*tap][cin], a GEMM over sites per (tap, slot of sites); the
+//    slots' partial sums are added in a fixed order by wgrad_reduce_kernel.
 //  * Elementwise kernels: features, loss gradient, bias gradient, Adam with the
 //    BF16 (and mirrored) weight copies, writing the prediction into a lattice.
 #include <algorithm>
@@ -385,120 +385,238 @@ inline int order_conv_tiles(ConvTile& t, int ly, int lz, int dil) {
 struct WgradArgs {
     const uint16_t* g;  // [n][cout] bf16 output gradient
     const uint16_t* x;  // [n][cin] bf16 layer input (before the layer's input ReLU)
-    float* part;        // [chunks][27][cout][cin]
-    long long n, chunk;
+    float* part;        // [slots][27][cout][cin]
     int cin, cout, lx, ly, lz, dil, reluIn;
+    int pieces;             // 8-site pieces of a row (the last may be shorter)
+    long long total, per;   // pieces of the lattice, and of one slot
+    int slots, vec;         // vec: part is 16-byte aligned
 };
 
-constexpr int kWgSites = 64;             // sites staged per step of the weight gradient
-constexpr int kWgLd = kWgSites + 8;      // LDS row stride (BF16) of the transposed tiles
+constexpr int kWgSplit = 4;                         // waves that share a slot's sites for one tap
+constexpr int kWgThreads = 3 * kWgSplit * 64;       // three taps
+constexpr int kWgSites = 4096;                      // sites one wave adds up in FP32 at most
+constexpr int kWgSlots = 28;                        // slots (of 9 work-groups) that 256 CUs run at once
 
-// One work-group per (chunk of sites, tap).  Per step it stages 64 sites of the
-// output gradient G and of the tap's neighbours of X (ReLU applied) in LDS,
-// transposed to [channel][site], so that both operands of
-// v_mfma_f32_16x16x32_bf16 read 8 consecutive sites (the contraction axis) as
-// one 16-byte LDS load; the four waves split the 16 x 16 output tiles of
-// dW[tap][cout][cin].
-template <int NT, int KT>
-__global__ void __launch_bounds__(kWsThreads) conv_wgrad_kernel(WgradArgs a) {
-    constexpr int CO = NT * 16, CI = KT * 16, TILES = NT * KT;
-    constexpr int TPW = (TILES + 3) / 4;    // tiles per wave
-    __shared__ __align__(16) uint16_t gT[CO * kWgLd];
-    __shared__ __align__(16) uint16_t xT[CI * kWgLd];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kq = lane >> 4, l16 = lane & 15;
-    const int tap = blockIdx.y;
-    const long long c = blockIdx.x;
-    const long long s0 = c * a.chunk, s1 = min(a.n, s0 + a.chunk);
-    v4f acc[TPW];
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) acc[k] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (long long sb = s0; sb < s1; sb += kWgSites) {
-        // stage: 8-byte loads (4 channels of one site), 2-byte transposed LDS stores
-        for (int e = threadIdx.x; e < kWgSites * CO / 4; e += kWsThreads) {
-            const int site = e / (CO / 4), c4 = (e % (CO / 4)) * 4;
-            const long long sg = sb + site;
-            uint2 raw = {0u, 0u};
-            if (sg < s1) raw = *reinterpret_cast<const uint2*>(a.g + sg * CO + c4);
-            gT[(c4 + 0) * kWgLd + site] = uint16_t(raw.x & 0xffffu);
-            gT[(c4 + 1) * kWgLd + site] = uint16_t(raw.x >> 16);
-            gT[(c4 + 2) * kWgLd + site] = uint16_t(raw.y & 0xffffu);
-            gT[(c4 + 3) * kWgLd + site] = uint16_t(raw.y >> 16);
-        }
-        for (int e = threadIdx.x; e < kWgSites * CI / 4; e += kWsThreads) {
-            const int site = e / (CI / 4), c4 = (e % (CI / 4)) * 4;
-            const long long sg = sb + site;
-            uint2 raw = {0u, 0u};
-            if (sg < s1) {
-                const int x = int(sg % a.lx), y = int((sg / a.lx) % a.ly), z = int(sg / ((long long)a.lx * a.ly));
-                const long long nb = tap_site(x, y, z, tap, a.dil, a.lx, a.ly, a.lz);
-                raw = *reinterpret_cast<const uint2*>(a.x + nb * CI + c4);
-            }
-            uint16_t v[4] = {uint16_t(raw.x & 0xffffu), uint16_t(raw.x >> 16), uint16_t(raw.y & 0xffffu),
-                             uint16_t(raw.y >> 16)};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (a.reluIn && (v[j] & 0x8000u)) v[j] = 0;   // negative BF16 (and -0) -> +0
-                xT[(c4 + j) * kWgLd + site] = v[j];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < TPW; ++k) {
-            const int tile = wave * TPW + k;
-            if (tile >= TILES) break;
-            const int mt = tile / KT, nt = tile % KT;
-#pragma unroll
-            for (int ks = 0; ks < kWgSites / 32; ++ks) {
-                const int site = ks * 32 + 8 * kq;
-                const v4u ar = *reinterpret_cast<const v4u*>(&gT[(mt * 16 + l16) * kWgLd + site]);
-                const v4u br = *reinterpret_cast<const v4u*>(&xT[(nt * 16 + l16) * kWgLd + site]);
-                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ar),
-                                                                 __builtin_bit_cast(v8bf, br), acc[k], 0, 0, 0);
-            }
-        }
-        __syncthreads();
+// C / 16 consecutive channels of one site (2, 4 or 8 bytes): a lane's share of
+// a 16-channel-group row
+template <int PC>
+struct Raw {
+    unsigned w[PC == 4 ? 2 : 1];
+};
+
+template <int PC>
+__device__ __forceinline__ Raw<PC> raw_load(const uint16_t* p) {
+    Raw<PC> r;
+    if constexpr (PC == 4) {
+        const uint2 v = *reinterpret_cast<const uint2*>(p);
+        r.w[0] = v.x;
+        r.w[1] = v.y;
+    } else if constexpr (PC == 2) {
+        r.w[0] = *reinterpret_cast<const unsigned*>(p);
+    } else {
+        r.w[0] = *p;
     }
-    // D[m = cout][n = cin]: lane l, element j = D[4 (l / 16) + j][l % 16]
-#pragma unroll
-    for (int k = 0; k < TPW; ++k) {
-        const int tile = wave * TPW + k;
-        if (tile >= TILES) break;
-        const int mt = tile / KT, nt = tile % KT;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = mt * 16 + 4 * kq + j;
-            a.part[((c * kTaps + tap) * CO + row) * CI + nt * 16 + l16] = acc[k][j];
-        }
-    }
+    return r;
 }
 
-// fixed-order sum over chunks
+// Channel c of eight sites as an operand of v_mfma_f32_16x16x32_bf16
+template <int PC>
+__device__ __forceinline__ v8bf raw_operand(const Raw<PC> (&r)[8], int c) {
+    v4u v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        v[i] = __builtin_amdgcn_perm(r[2 * i + 1].w[c >> 1], r[2 * i].w[c >> 1],
+                                     (c & 1) ? 0x07060302u : 0x05040100u);
+    return __builtin_bit_cast(v8bf, v);
+}
+
+// Weight gradient dW[tap][co][ci] = sum_site G[site][co] X[site + tap][ci]: a
+// product whose contraction runs over the sites, while a site's channels are
+// what lies together in memory.  A lane reads C / 16 consecutive channels of
+// eight consecutive sites of a row and transposes them in registers, one byte
+// permute per operand word: matrix row m of product a then stands for channel
+// C / 16 m + a, which only the final store has to know.  So no operand passes
+// through LDS, and the waves run without barriers until their sums are added.
+// A work-group takes one slot of sites and the three taps of one (dy, dz),
+// whose waves read the same G and, shifted by dil sites, the same X from the
+// L1; four waves share a slot's sites per tap, and their sums are added in a
+// fixed order through LDS.
+// 64 x 64 channels of 302k sites: 160 us (418 TFLOP/s); staged in LDS per tap and
+// transposed there by two-byte stores it took 770 us.  Bound by the operand
+// loads through the L1 (8 KB per wave and 32 sites) and the vector work beside
+// the 16 matrix instructions they feed.
+template <int NT, int KT>
+__global__ void __launch_bounds__(kWgThreads) conv_wgrad_kernel(WgradArgs a) {
+    constexpr int CO = NT * 16, CI = KT * 16;
+    __shared__ __align__(16) float red[3][NT * KT][64][4];
+    // each XCD gets whole slots: the nine (dy, dz) of a slot read the same sites
+    const int nb = gridDim.x, qb = nb >> 3, rb = nb & 7, xcd = blockIdx.x & 7;
+    const int blk = xcd * qb + min(xcd, rb) + (blockIdx.x >> 3);
+    const int slot = blk / 9, dyz = blk % 9;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int d = wave % 3, quarter = wave / 3;
+    const int kq = lane >> 4, l16 = lane & 15;
+    // the taps' offsets, wrapped into [0, length)
+    const int dx = wrapd((d - 1) * a.dil, a.lx), dy = wrapd((dyz % 3 - 1) * a.dil, a.ly),
+              dz = wrapd((dyz / 3 - 1) * a.dil, a.lz);
+
+    const long long q0 = slot * a.per, q1 = min(a.total, q0 + a.per);
+    long long q = q0 + 4 * quarter + kq;
+    // x piece, y and z of the lane's piece, advanced by 4 kWgSplit pieces a turn
+    int px = int(q % a.pieces), y = int(q / a.pieces % a.ly), z = int(q / a.pieces / a.ly);
+    constexpr int kStride = 4 * kWgSplit;
+    const int sx = kStride % a.pieces, sy = kStride / a.pieces % a.ly, sz = kStride / a.pieces / a.ly;
+
+    v4f acc[NT][KT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int k = 0; k < KT; ++k) acc[i][k] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    const long long turns = (q1 - q0 + kStride - 1) / kStride;
+    for (long long it = 0; it < turns; ++it, q += kStride) {
+        const bool have = q < q1;
+        const int x = have ? 8 * px : 0, yy = have ? y : 0, zz = have ? z : 0;
+        const int valid = have ? min(8, a.lx - x) : 0;   // sites of this piece
+        const uint16_t* gp = a.g + ((long long)x + (long long)a.lx * (yy + (long long)a.ly * zz)) * CO + NT * l16;
+        const int yn = yy + dy >= a.ly ? yy + dy - a.ly : yy + dy, zn = zz + dz >= a.lz ? zz + dz - a.lz : zz + dz;
+        const int xn = x + dx >= a.lx ? x + dx - a.lx : x + dx;
+        const uint16_t* xp = a.x + (long long)a.lx * (yn + (long long)a.ly * zn) * CI + KT * l16;
+        Raw<NT> g[8];
+        Raw<KT> xv[8];
+        if (__all(valid == 8 && xn + 8 <= a.lx)) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) g[j] = raw_load<NT>(gp + j * CO);
+            xp += (long long)xn * CI;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) xv[j] = raw_load<KT>(xp + j * CI);
+        } else {
+            // a piece that ends with its row or wraps around it: sites past the end count as zeros
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const bool in = j < valid;
+                int xs = xn + (in ? j : 0);
+                xs = xs >= a.lx ? xs - a.lx : xs;
+                g[j] = raw_load<NT>(gp + (in ? j : 0) * CO);
+                xv[j] = raw_load<KT>(xp + (long long)xs * CI);
+#pragma unroll
+                for (unsigned& w : g[j].w) w = in ? w : 0u;
+#pragma unroll
+                for (unsigned& w : xv[j].w) w = in ? w : 0u;
+            }
+        }
+        if (a.reluIn) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (unsigned& w : xv[j].w) w = relu2(w);
+        }
+        v8bf xb[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) xb[k] = raw_operand<KT>(xv, k);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const v8bf ga = raw_operand<NT>(g, i);
+#pragma unroll
+            for (int k = 0; k < KT; ++k)
+                acc[i][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, xb[k], acc[i][k], 0, 0, 0);
+        }
+        px += sx;
+        const int cx = px >= a.pieces;
+        px -= cx ? a.pieces : 0;
+        y += sy + cx;
+        const int cy = y >= a.ly;
+        y -= cy ? a.ly : 0;
+        z += sz + cy;
+    }
+    for (int h = 1; h < kWgSplit; ++h) {
+        if (quarter == h) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int k = 0; k < KT; ++k) *reinterpret_cast<v4f*>(red[d][i * KT + k][lane]) = acc[i][k];
+        }
+        __syncthreads();
+        if (quarter == 0) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int k = 0; k < KT; ++k) acc[i][k] += *reinterpret_cast<const v4f*>(red[d][i * KT + k][lane]);
+        }
+        __syncthreads();
+    }
+    if (quarter != 0) return;
+    // lane l, element j of acc[i][k] = dW[co = NT (4 (l / 16) + j) + i][ci = KT (l % 16) + k]
+    const int tap = dyz * 3 + d;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float* o = a.part + (((long long)slot * kTaps + tap) * CO + NT * (4 * kq + j) + i) * CI + KT * l16;
+            if (KT == 4 && a.vec) {
+                *reinterpret_cast<v4f*>(o) = v4f{acc[i][0][j], acc[i][1 % KT][j], acc[i][2 % KT][j], acc[i][3 % KT][j]};
+            } else {
+#pragma unroll
+                for (int k = 0; k < KT; ++k) o[k] = acc[i][k][j];
+            }
+        }
+}
+
+// Fixed-order sum over chunks.  A thread's loads are taken sixteen at a time,
+// ahead of the additions: one after the other, 74 chunks of 27 x 64 x 64
+// values took 69 us.
 __global__ void wgrad_reduce_kernel(const float* part, long long chunks, long long per, float* out) {
+    constexpr int kAhead = 16;
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < per; e += (long long)gridDim.x * blockDim.x) {
         float s = 0.f;
-        for (long long c = 0; c < chunks; ++c) s += part[c * per + e];
+        long long c = 0;
+        for (; c + kAhead <= chunks; c += kAhead) {
+            float v[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) v[k] = part[(c + k) * per + e];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) s += v[k];
+        }
+        for (; c < chunks; ++c) s += part[c * per + e];
         out[e] = s;
     }
 }
 
-// bias gradient, first stage: work-group b sums its chunk of sites for every
-// channel (consecutive threads read consecutive channels of a site: coalesced);
-// wgrad_reduce_kernel then adds the work-groups' rows in a fixed order
+// Bias gradient, first stage: work-group b sums its chunk of sites for every
+// channel, each thread eight channels of every (2048 / cout)th site (VEC; two
+// bytes at a time where g is not 16-byte aligned); wgrad_reduce_kernel then
+// adds the work-groups' rows in a fixed order.  302k sites of 64 channels:
+// 8 us, two bytes at a time 44 us.
+template <bool VEC>
 __global__ void __launch_bounds__(kWsThreads) bias_grad_kernel(const uint16_t* g, long long n, int cout,
                                                               long long chunk, float* part) {
-    __shared__ float red[kWsThreads];
-    const int rows = kWsThreads / cout, c = threadIdx.x % cout, r = threadIdx.x / cout;
+    constexpr int W = VEC ? 8 : 1;
+    __shared__ float red[kWsThreads * W];
+    const int cols = cout / W, rows = kWsThreads / cols, c = threadIdx.x % cols, r = threadIdx.x / cols;
     const long long s0 = (long long)blockIdx.x * chunk, s1 = min(n, s0 + chunk);
-    float s = 0.f;
-    if (r < rows)
-        for (long long i = s0 + r; i < s1; i += rows) s += bf2f(g[i * cout + c]);
-    red[threadIdx.x] = s;
+    float s[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) s[k] = 0.f;
+#pragma unroll 4
+    for (long long i = s0 + r; i < s1; i += rows) {
+        if constexpr (VEC) {
+            const v4u v = *reinterpret_cast<const v4u*>(g + i * cout + 8 * c);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                s[2 * k] += __uint_as_float(v[k] << 16);
+                s[2 * k + 1] += __uint_as_float(v[k] & 0xffff0000u);
+            }
+        } else {
+            s[0] += bf2f(g[i * cout + c]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < W; ++k) red[(r * cols + c) * W + k] = s[k];
     __syncthreads();
-    if (r == 0) {
+    for (int e = threadIdx.x; e < cout; e += kWsThreads) {
         float t = 0.f;
-        for (int k = 0; k < rows; ++k) t += red[k * cout + c];
-        part[(long long)blockIdx.x * cout + c] = t;
+        for (int k = 0; k < rows; ++k) t += red[k * cout + e];
+        part[(long long)blockIdx.x * cout + e] = t;
     }
 }
 
@@ -665,8 +783,8 @@ hipError_t launch_fwd_t(const ConvArgs& a, hipStream_t s) {
 }
 
 template <int NT, int KT>
-hipError_t launch_wgrad_t(const WgradArgs& a, long long chunks, hipStream_t s) {
-    hipLaunchKernelGGL((conv_wgrad_kernel<NT, KT>), dim3(unsigned(chunks), kTaps), dim3(kWsThreads), 0, s, a);
+hipError_t launch_wgrad_t(const WgradArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((conv_wgrad_kernel<NT, KT>), dim3(9 * a.slots), dim3(kWgThreads), 0, s, a);
     return hipGetLastError();
 }
 
@@ -687,8 +805,8 @@ hipError_t launch_wgrad_t(const WgradArgs& a, long long chunks, hipStream_t s) {
 
 hipError_t launch_fwd(const ConvArgs& a, hipStream_t s) { QMIN_WS_DISPATCH(launch_fwd_t, a.cout / 16, a.cin / 16, a, s) }
 
-hipError_t launch_wgrad(const WgradArgs& a, long long chunks, hipStream_t s) {
-    QMIN_WS_DISPATCH(launch_wgrad_t, a.cout / 16, a.cin / 16, a, chunks, s)
+hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
+    QMIN_WS_DISPATCH(launch_wgrad_t, a.cout / 16, a.cin / 16, a, s)
 }
 
 bool channels_ok(int c) { return c == 16 || c == 32 || c == 64; }
@@ -739,8 +857,6 @@ int qm_ws_conv_wgrad(const void* g, int cout, const void* x, int cin, int reluIn
     a.g = static_cast<const uint16_t*>(g);
     a.x = static_cast<const uint16_t*>(x);
     a.part = part;
-    a.n = (long long)lx * ly * lz;
-    a.chunk = chunk;
     a.cin = cin;
     a.cout = cout;
     a.lx = lx;
@@ -748,11 +864,20 @@ int qm_ws_conv_wgrad(const void* g, int cout, const void* x, int cin, int reluIn
     a.lz = lz;
     a.dil = dil;
     a.reluIn = reluIn;
-    const long long chunks = (a.n + chunk - 1) / chunk;
+    a.vec = (reinterpret_cast<uintptr_t>(part) & 15) == 0;
+    a.pieces = (lx + 7) / 8;
+    a.total = (long long)a.pieces * ly * lz;
+    // part holds one row of partial sums per chunk: as many slots of sites at
+    // most; fewer where a whole number of rounds over the CUs already keeps
+    // every wave's FP32 sum within kWgSites sites
+    const long long n = (long long)lx * ly * lz, chunks = (n + chunk - 1) / chunk;
+    const long long rounds = (n + (long long)kWgSites * kWgSplit * kWgSlots - 1) / ((long long)kWgSites * kWgSplit * kWgSlots);
+    a.slots = int(std::min(chunks, kWgSlots * rounds));
+    a.per = (a.total + a.slots - 1) / a.slots;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    HIP_TRY(launch_wgrad(a, chunks, s));
+    HIP_TRY(launch_wgrad(a, s));
     const long long per = (long long)kTaps * cout * cin;
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(per)), dim3(kWsThreads), 0, s, part, chunks, per, dw);
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(per)), dim3(kWsThreads), 0, s, part, (long long)a.slots, per, dw);
     HIP_TRY(hipGetLastError());
     return QM_OK;
 }
@@ -761,8 +886,9 @@ int qm_ws_bias_grad(const void* g, long long n, int cout, float* part, int block
     if (!g || !db || !part || !channels_ok(cout) || blocks < 1 || n < 1) return fail(QM_EINVAL, "bad argument");
     const long long chunk = (n + blocks - 1) / blocks;
     const auto st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(bias_grad_kernel, dim3(blocks), dim3(kWsThreads), 0, st, static_cast<const uint16_t*>(g), n, cout,
-                       chunk, part);
+    const bool vec = (reinterpret_cast<uintptr_t>(g) & 15) == 0;
+    hipLaunchKernelGGL(vec ? bias_grad_kernel<true> : bias_grad_kernel<false>, dim3(blocks), dim3(kWsThreads), 0, st,
+                       static_cast<const uint16_t*>(g), n, cout, chunk, part);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(1), dim3(64), 0, st, part, (long long)blocks, (long long)cout, db);
     HIP_TRY(hipGetLastError());

@@ -58,3 +58,28 @@ def test_forward_tiles(lx, ly, lz, dil, cin, cout, shift):
     tol = 1e-5 * np.abs(ref).max()
     np.testing.assert_allclose(yf.cpu().numpy().reshape(n, cout), ref, rtol=0, atol=tol)
     np.testing.assert_allclose(host_bf16(yb).reshape(n, cout), np.where(mask > 0, ref, 0.0), rtol=2 ** -8, atol=tol)
+
+
+@pytest.mark.parametrize("lx,ly,lz,dil", TILES + [(16, 4, 5, 8), (64, 3, 2, 4)])
+@pytest.mark.parametrize("cin,cout", [(16, 32), (32, 64), (64, 16), (64, 64)])
+@pytest.mark.parametrize("chunk,shift", [(64, 0), (4096, 1)])
+def test_weight_and_bias_gradient_pieces(lx, ly, lz, dil, cin, cout, chunk, shift):
+    """Rows that are no multiple of eight sites, pieces that wrap around a row,
+    several slots and one, and buffers of four-byte alignment."""
+    lib = qmin.library()
+    rng = np.random.default_rng(lx + dil + cout)
+    dims, n = (lx, ly, lz), lx * ly * lz
+    x, g = co.bf16_round(rng.normal(size=(n, cin))), co.bf16_round(rng.normal(size=(n, cout)))
+    ref = co.weight_grad(g, x, dims, dil, relu_in=True)
+    chunks = (n + chunk - 1) // chunk
+    part = offset(torch.empty(chunks * 27 * cout * cin, dtype=torch.float32, device="cuda"), shift)
+    dw = torch.empty(27 * cout * cin, dtype=torch.float32, device="cuda")
+    gd, xd = dev_bf16(g), dev_bf16(x)
+    check(lib.qm_ws_conv_wgrad(ptr(gd), cout, ptr(xd), cin, 1, lx, ly, lz, dil, ptr(part), chunk, ptr(dw), stream()))
+    db = torch.empty(cout, dtype=torch.float32, device="cuda")
+    bpart = torch.empty(37 * cout, dtype=torch.float32, device="cuda")
+    gb = offset(gd, shift)
+    check(lib.qm_ws_bias_grad(ptr(gb), n, cout, ptr(bpart), 37, ptr(db), stream()))
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(dw.cpu().numpy().reshape(27, cout, cin), ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+    np.testing.assert_allclose(db.cpu().numpy(), g.sum(axis=0), rtol=1e-5, atol=1e-5 * np.sqrt(n))
