@@ -3,22 +3,24 @@
 // An Adam or Nesterov iteration is one lattice pass (the fused and boundary
 // passes in mode kAdamStep / kNesterovStep, step_kernels.hip): each site's
 // force, then the minimizer's update of that site, written to the other state
-// set.  An L-BFGS iteration is the shared force pass (force mode) and
+// set.  An L-BFGS iteration is the shared force pass (force mode) and two
 // streaming kernels over the 5 n components of Q, F and the minimizer's own
 // vectors (same plane layout as Q).  Every pass reduces the dot products it
-// needs into per-work-group partials; a one-work-group finalize kernel sums
-// them in a fixed order and finishes the minimizer's scalar logic in device
-// memory (step coefficients, forceMax, the stopping test).  (A separate kernel, not a last-work-group
-// pattern: the device-wide fences that pattern needs write back each XCD's L2,
-// which the streaming kernel has just filled.)  A batch of iterations is
-// therefore queued without host round trips, every kernel after the stopping
-// test is a no-op, and the host reads the control block once per batch.
+// needs into per-work-group partials; a one-work-group kernel sums them in a
+// fixed order and finishes the minimizer's scalar logic in device memory (step
+// coefficients, forceMax, the stopping test).  (A separate kernel, not a
+// last-work-group pattern: the device-wide fences that pattern needs write back
+// each XCD's L2, which the streaming kernel has just filled.)  A batch of
+// iterations is therefore queued without host round trips, every kernel after
+// the stopping test is a no-op, and the host reads the control block once per
+// batch.
 //
 // Arithmetic follows the reference CPU steps: energyMinimizerAdam.cpp:25-54,
 // energyMinimizerNesterovAG.cpp:70-92 and energyMinimizerLoLBFGS.cpp:104-193.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "qmin_internal.h"
 
@@ -26,48 +28,11 @@ namespace qmin {
 namespace {
 
 constexpr int kVecThreads = 256;
-constexpr int kVecUnroll = 4;
-constexpr int kVecMaxBlocks = 2048;
-constexpr int kMaxDots = 4;
 
 __device__ __forceinline__ double wsum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
-}
-
-// Fixed-order work-group sum of K doubles; the result is valid in thread 0.
-template <int K>
-__device__ __forceinline__ void block_sum(double (&v)[K], double (*red)[kMaxDots]) {
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = wsum(v[k]);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) red[w][k] = v[k];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            double s = 0;
-#pragma unroll
-            for (int i = 0; i < kVecThreads / 64; ++i) s += red[i][k];
-            v[k] = s;
-        }
-    }
-    __syncthreads();
-}
-
-// Writes this work-group's K partial sums (stride kMaxDots).
-template <int K>
-__device__ __forceinline__ void write_partials(double (&v)[K], double* partials) {
-    __shared__ double red[kVecThreads / 64][kMaxDots];
-    block_sum<K>(v, red);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) partials[kMaxDots * blockIdx.x + k] = v[k];
-    }
 }
 
 // Iteration bookkeeping shared by the three minimizers (thread 0 of the last
@@ -86,240 +51,293 @@ __device__ void finish_iteration(Ctrl* ctrl, double forceMax, double fc, double*
 
 struct Common {
     Ctrl* ctrl;
-    double* partials;   // [blocks][kMaxDots]
+    double* partials;
     double* trace;      // [traceCap] forceMax per iteration
     double fc, ndof;
     long long len;      // 5 n
 };
 
 // ---------------------------------------------------------------- online L-BFGS
-// Device scalars of the two-loop recursion, per memory slot t and loop index ii:
-//   SY[t] = s_t . y_t and YY[t] = y_t . y_t, cached when y_t is completed
-//   (s_t and y_t do not change until slot t is reused),
-//   A[ii] = alpha_ii, NA[ii] = -alpha_ii, CS[ii] = alpha_ii - beta_ii (0 when
-//   s.y is 0, where the reference skips the update), K3 = the step-3 factor.
+// The direction of an iteration is a combination of the forces and the history,
+// p = F + sum_t cy_t y_t + sum_t cs_t s_t.  The two-loop recursion
+// (energyMinimizerLoLBFGS.cpp:117-163) that fixes the coefficients needs only
+// scalar products: s_t.y_u and y_t.y_u, kept between iterations with the new
+// pair's rows replaced, and s_t.F and y_t.F.  So one pass over the history takes
+// the products, one work-group runs the recursion on them, and one pass forms
+// the direction and takes the step: at m = 8, 39 vectors read or written per
+// iteration instead of the 72 of one streaming pass per two-loop stage, and 3
+// launches beside the force's instead of 34.  At 100 x 96 x 104 in FP64, m = 8:
+// 0.38 ms per iteration against 0.66 (passes 144 and 148 us, 5.3 and 5.7 TB/s;
+// recursion 13 us).
+//
+// Device scalars: SY[u m + t] = s_t.y_u, YY[u m + t] = y_t.y_u, the
+// coefficients of the next step, and the recursion's work space (the products,
+// sp, yp, alpha, F.F).
 struct LbLayout {
     int m;
-    __host__ __device__ int SY(int t) const { return t; }
-    __host__ __device__ int YY(int t) const { return m + t; }
-    __host__ __device__ int A(int i) const { return 2 * m + i; }
-    __host__ __device__ int NA(int i) const { return 3 * m + i; }
-    __host__ __device__ int CS(int i) const { return 4 * m + i; }
-    __host__ __device__ int K3() const { return 5 * m; }
-    __host__ __device__ int size() const { return 5 * m + 1; }
+    __host__ __device__ int SY(int u, int t) const { return u * m + t; }
+    __host__ __device__ int YY(int u, int t) const { return m * m + u * m + t; }
+    __host__ __device__ int CY(int t) const { return 2 * m * m + t; }
+    __host__ __device__ int CS(int t) const { return 2 * m * m + m + t; }
+    __host__ __device__ int work() const { return 2 * m * m + 2 * m; }
+    __host__ __device__ int workSize() const { return 8 * m + 1; }
+    __host__ __device__ int size() const { return work() + workSize(); }
 };
 
+constexpr int kLbBlock = 8;                       // slots whose products one launch takes
+constexpr int kLbDots = 5 * kLbBlock + 1;         // products per launch
+constexpr int kLbBlocks = 512;                    // work-groups of the passes over the history at most
 
 template <typename R>
-struct LbStageArgs {
-    R* p;
-    const R* x1;
-    const R* x2;      // may be null
-    const R* d;
-    int k1, k2;       // scalar slots of the coefficients of x1, x2
-    double* scal;
-    Common c;
-};
-
-// p = (p + k1 x1) [+ k2 x2]; then partials of d.p, finished into alpha_ii
-// (step 2, energyMinimizerLoLBFGS.cpp:117-131) or alpha_ii - beta_ii (step 4,
-// :145-163) by the finalize kernel.
-template <typename R>
-__global__ void __launch_bounds__(kVecThreads) lb_stage_kernel(LbStageArgs<R> A) {
-    Ctrl* ctrl = A.c.ctrl;
-    if (ctrl->done) return;
-    const R k1 = R(A.scal[A.k1]);
-    const R k2 = A.x2 ? R(A.scal[A.k2]) : R(0);
-    double dp = 0;
-    const long long stride = (long long)gridDim.x * kVecThreads * kVecUnroll;
-    for (long long base = (long long)blockIdx.x * kVecThreads * kVecUnroll + threadIdx.x; base < A.c.len;
-         base += stride) {
-#pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-            const long long i = base + u * kVecThreads;
-            if (i < A.c.len) {
-                R p = A.p[i] + k1 * A.x1[i];
-                if (A.x2) p = p + k2 * A.x2[i];
-                A.p[i] = p;
-                dp += double(A.d[i]) * double(p);
-            }
-        }
-    }
-    double part[1] = {dp};
-    write_partials<1>(part, A.c.partials);
-}
-
-template <typename R>
-struct LbMoveArgs {
-    const R* p;
-    const R* s0;      // s of the newest slot, added with CS[0]
-    R* sc;            // s of the slot being replaced
-    R* yc;            // y of the slot being replaced: receives F
+struct LbArgs {
+    R* hist;            // s_0 .. s_{m-1}, y_0 .. y_{m-1}, stride components apart
+    long long stride;
+    const R* f;
+    const R* p;         // the forces the products were taken of: f, but for the first step of a later call
     R* q;
-    const R* f;
     double eta;
-    int k;
+    int m, c, t0;       // memory, the slot being replaced, first slot of this launch's products
     double* scal;
-    Common c;
+    Common c0;
 };
 
-// Last step-4 update, then s_c = eta p, y_c = F (old forces), Q += s_c
-// (energyMinimizerLoLBFGS.cpp:158-176); p itself is replaced by the new forces.
+// y_c = y_c - F (the move stored the old forces there, :178-188), then the
+// products of the new pair and of F with the slots t0 .. t0 + 7, and F.F.
+// Bound by HBM: 2 m + 3 vectors.
 template <typename R>
-__global__ void __launch_bounds__(kVecThreads) lb_move_kernel(LbMoveArgs<R> A) {
-    if (A.c.ctrl->done) return;
-    const R k = R(A.scal[A.k]), eta = R(A.eta);
-    const long long stride = (long long)gridDim.x * kVecThreads * kVecUnroll;
-    for (long long base = (long long)blockIdx.x * kVecThreads * kVecUnroll + threadIdx.x; base < A.c.len;
-         base += stride) {
+__global__ void __launch_bounds__(kVecThreads) lb_dots_kernel(LbArgs<R> A) {
+    if (A.c0.ctrl->done) return;
+    double acc[kLbDots];
 #pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-            const long long i = base + u * kVecThreads;
-            if (i < A.c.len) {
-                const R p = A.p[i] + k * A.s0[i];
-                const R s = eta * p;
-                A.sc[i] = s;
-                A.yc[i] = A.f[i];
-                A.q[i] = A.q[i] + s;
-            }
+    for (int k = 0; k < kLbDots; ++k) acc[k] = 0;
+    const R* s0 = A.hist;
+    const R* y0 = A.hist + A.m * A.stride;
+    R* yc = A.hist + (A.m + A.c) * A.stride;
+    const R* sc = A.hist + A.c * A.stride;
+    const int count = min(kLbBlock, A.m - A.t0);
+    auto site = [&](long long i, auto width) {
+        constexpr int W = decltype(width)::value;
+        using V = R __attribute__((ext_vector_type(W)));
+        auto at = [&](const R* p) { return *reinterpret_cast<const V*>(p + i); };
+        const V f = at(A.f), so = at(sc);
+        V yn = at(yc);
+        if (A.t0 == 0) {
+            yn = yn - f;
+            *reinterpret_cast<V*>(yc + i) = yn;
         }
+        V sv[kLbBlock], yv[kLbBlock];
+#pragma unroll
+        for (int k = 0; k < kLbBlock; ++k)
+            if (k < count) {
+                sv[k] = at(s0 + (A.t0 + k) * A.stride);
+                yv[k] = A.t0 + k == A.c ? yn : at(y0 + (A.t0 + k) * A.stride);
+            }
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const double fd = double(f[w]), yd = double(yn[w]), sd = double(so[w]);
+            acc[kLbDots - 1] += fd * fd;
+#pragma unroll
+            for (int k = 0; k < kLbBlock; ++k)
+                if (k < count) {
+                    const double a = double(sv[k][w]), b = double(yv[k][w]);
+                    acc[5 * k + 0] += a * fd;
+                    acc[5 * k + 1] += b * fd;
+                    acc[5 * k + 2] += a * yd;
+                    acc[5 * k + 3] += b * yd;
+                    acc[5 * k + 4] += sd * b;
+                }
+        }
+    };
+    const long long pairs = A.c0.len / 2, step = (long long)gridDim.x * kVecThreads;
+    for (long long j = (long long)blockIdx.x * kVecThreads + threadIdx.x; j < pairs; j += step)
+        site(2 * j, std::integral_constant<int, 2>{});
+    if ((A.c0.len & 1) && blockIdx.x == 0 && threadIdx.x == 0) site(A.c0.len - 1, std::integral_constant<int, 1>{});
+    // work-group sums in a fixed order; partials[k][work-group]
+    __shared__ double red[kVecThreads / 64][kLbDots];
+#pragma unroll
+    for (int k = 0; k < kLbDots; ++k) {
+        const double v = wsum(acc[k]);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < kLbDots) {
+        double v = 0;
+#pragma unroll
+        for (int w = 0; w < kVecThreads / 64; ++w) v += red[w][threadIdx.x];
+        A.c0.partials[((long long)(A.t0 / kLbBlock) * kLbDots + threadIdx.x) * kLbBlocks + blockIdx.x] = v;
     }
 }
 
-template <typename R>
-struct LbFinishArgs {
-    R* p;
-    const R* f;
-    const R* s;       // s of the newest slot
-    R* y;             // y of the newest slot (null on the first call: no update)
-    Common c;
-};
-
-// p = F; y_t = y_t - F (:178-188); partials of F.F, s_t.y_t, y_t.y_t and s_t.p,
-// from which the finalize kernel takes forceMax = sqrt(F.F)/N, caches s_t.y_t
-// and y_t.y_t, and starts the next two-loop pass: alpha_0 = s_t.p / s_t.y_t and
-// the step-3 factor (s.y)/(y.y) of the same slot (:117-142).
-template <typename R>
-__global__ void __launch_bounds__(kVecThreads) lb_finish_kernel(LbFinishArgs<R> A) {
-    Ctrl* ctrl = A.c.ctrl;
+// Sums the products in a fixed order (a wave per product), replaces the new
+// pair's rows of SY and YY, runs the two-loop recursion on the products (sp_t =
+// s_t.p and yp_t = y_t.p as p grows), and ends the iteration.  Its length is
+// that of the recursion's 2 m dependent steps: with LDS they read SY, YY and
+// the work space from there (up to kLbLdsMemory slots), else from memory.
+constexpr int kLbCoefThreads = 512;
+constexpr int kLbLdsMemory = 32;
+template <bool LDS>
+__global__ void __launch_bounds__(kLbCoefThreads) lb_coef_kernel(Common c, double* scal, LbLayout lay, int slot,
+                                                                int blocks) {
+    __shared__ double lds[LDS ? 2 * kLbLdsMemory * kLbLdsMemory + 8 * kLbLdsMemory + 1 : 1];
+    Ctrl* ctrl = c.ctrl;
     if (ctrl->done) return;
-    double pp = 0, sy = 0, yy = 0, sp = 0;
-    const long long stride = (long long)gridDim.x * kVecThreads * kVecUnroll;
-    for (long long base = (long long)blockIdx.x * kVecThreads * kVecUnroll + threadIdx.x; base < A.c.len;
-         base += stride) {
-#pragma unroll
-        for (int u = 0; u < kVecUnroll; ++u) {
-            const long long i = base + u * kVecThreads;
-            if (i < A.c.len) {
-                const R f = A.f[i];
-                const double s = double(A.s[i]);
-                A.p[i] = f;
-                pp += double(f) * double(f);
-                sp += s * double(f);
-                if (A.y) {
-                    const R y = A.y[i] - f;
-                    A.y[i] = y;
-                    sy += s * double(y);
-                    yy += double(y) * double(y);
-                }
-            }
+    const int m = lay.m, tid = threadIdx.x, mm = m * m;
+    double* SY = LDS ? lds : scal;
+    double* YY = SY + mm;
+    double* dots = LDS ? lds + 2 * mm : scal + lay.work();
+    double* sp = dots + 5 * m;
+    double* yp = sp + m;
+    double* alpha = yp + m;
+    double* ff = alpha + m;
+    if constexpr (LDS)
+        for (int k = tid; k < 2 * mm; k += kLbCoefThreads) lds[k] = scal[k];
+    for (int k = tid >> 6; k <= 5 * m; k += kLbCoefThreads / 64) {
+        const int block = k == 5 * m ? 0 : k / (5 * kLbBlock), row = k == 5 * m ? kLbDots - 1 : k % (5 * kLbBlock);
+        const double* part = c.partials + ((long long)block * kLbDots + row) * kLbBlocks;
+        double v = 0;
+#pragma unroll 8
+        for (int j = tid & 63; j < blocks; j += 64) v += part[j];
+        v = wsum(v);
+        if ((tid & 63) == 0) *(k == 5 * m ? ff : dots + k) = v;
+    }
+    __syncthreads();
+    for (int t = tid; t < m; t += kLbCoefThreads) {
+        sp[t] = dots[5 * t + 0];
+        yp[t] = dots[5 * t + 1];
+        const double sy = dots[5 * t + 2], yy = dots[5 * t + 3], ys = dots[5 * t + 4];
+        SY[slot * m + t] = sy;
+        YY[slot * m + t] = yy;
+        YY[t * m + slot] = yy;
+        SY[t * m + slot] = ys;
+        if constexpr (LDS) {
+            scal[lay.SY(slot, t)] = sy;
+            scal[lay.YY(slot, t)] = yy;
+            scal[lay.YY(t, slot)] = yy;
+            scal[lay.SY(t, slot)] = ys;
         }
     }
-    double part[4] = {pp, sy, yy, sp};
-    write_partials<4>(part, A.c.partials);
+    __syncthreads();
+    // newest slot first (:117-131); a pair with s.y = 0 is skipped
+    for (int i = 0; i < m; ++i) {
+        const int t = (slot - i + m) % m;
+        const double sy = SY[t * m + t];
+        const double a = sy != 0 ? sp[t] / sy : 0.0;
+        __syncthreads();
+        for (int u = tid; u < m; u += kLbCoefThreads) {
+            sp[u] -= a * SY[t * m + u];
+            yp[u] -= a * YY[t * m + u];
+        }
+        if (tid == 0) alpha[i] = a;
+        __syncthreads();
+    }
+    // step 3 (:133-142): p += (s.y / y.y) y of the newest slot
+    const double yy = YY[slot * m + slot];
+    const double k3 = yy != 0 ? SY[slot * m + slot] / yy : 0.0;
+    for (int u = tid; u < m; u += kLbCoefThreads) yp[u] += k3 * YY[slot * m + u];
+    __syncthreads();
+    // oldest first (:145-163)
+    for (int i = m - 1; i >= 0; --i) {
+        const int t = (slot - i + m) % m;
+        const double sy = SY[t * m + t];
+        const double d = sy != 0 ? alpha[i] - yp[t] / sy : 0.0;
+        __syncthreads();
+        for (int u = tid; u < m; u += kLbCoefThreads) yp[u] += d * SY[u * m + t];
+        if (tid == 0) {
+            scal[lay.CS(t)] = d;
+            scal[lay.CY(t)] = (i == 0 ? k3 : 0.0) - alpha[i];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) finish_iteration(ctrl, sqrt(*ff) / c.ndof, c.fc, c.trace);
+}
+
+// p = F + sum_t cy_t y_t + sum_t cs_t s_t in FP64; then s_c = eta p, y_c = F (the old forces), Q += s_c (:158-176).  Runs from the end of
+// the vectors to their start: the last of what the products' pass read is still
+// in the memory-side cache.  Bound by HBM: 2 m + 5 vectors.
+template <typename R>
+__global__ void __launch_bounds__(kVecThreads) lb_move_kernel(LbArgs<R> A) {
+    if (A.c0.ctrl->done) return;
+    const LbLayout lay{A.m};
+    auto site = [&](long long i, auto width) {
+        constexpr int W = decltype(width)::value;
+        using V = R __attribute__((ext_vector_type(W)));
+        auto at = [&](const R* p) { return *reinterpret_cast<const V*>(p + i); };
+        const V f = at(A.f), pv = at(A.p), q = at(A.q);
+        double p[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) p[w] = double(pv[w]);
+        for (int t0 = 0; t0 < A.m; t0 += kLbBlock) {
+            V sv[kLbBlock], yv[kLbBlock];
+#pragma unroll
+            for (int k = 0; k < kLbBlock; ++k)
+                if (t0 + k < A.m) {
+                    sv[k] = at(A.hist + (t0 + k) * A.stride);
+                    yv[k] = at(A.hist + (A.m + t0 + k) * A.stride);
+                }
+#pragma unroll
+            for (int k = 0; k < kLbBlock; ++k)
+                if (t0 + k < A.m) {
+                    const double cy = A.scal[lay.CY(t0 + k)], cs = A.scal[lay.CS(t0 + k)];
+#pragma unroll
+                    for (int w = 0; w < W; ++w) p[w] += cy * double(yv[k][w]) + cs * double(sv[k][w]);
+                }
+        }
+        V s;
+#pragma unroll
+        for (int w = 0; w < W; ++w) s[w] = R(A.eta * p[w]);
+        *reinterpret_cast<V*>(A.hist + A.c * A.stride + i) = s;
+        *reinterpret_cast<V*>(A.hist + (A.m + A.c) * A.stride + i) = f;
+        *reinterpret_cast<V*>(A.q + i) = q + s;
+    };
+    const long long pairs = A.c0.len / 2, step = (long long)gridDim.x * kVecThreads;
+    if ((A.c0.len & 1) && blockIdx.x == 0 && threadIdx.x == 0) site(A.c0.len - 1, std::integral_constant<int, 1>{});
+    for (long long j = pairs - 1 - ((long long)blockIdx.x * kVecThreads + threadIdx.x); j >= 0; j -= step)
+        site(2 * j, std::integral_constant<int, 2>{});
 }
 
 // ---------------------------------------------------------------- finalize
-enum FinOp { kFinAdam, kFinNesterov, kFinAlpha, kFinBeta, kFinLbFinish, kFinLbStart };
+enum FinOp { kFinAdam, kFinNesterov };
 
 struct FinArgs {
     int op;
-    int blocks;       // partial-sum slots to sum
-    int stride;       // doubles per slot: kMaxDots for the streaming kernels, 3 for the lattice passes
-    int flip;         // the pass wrote the other state set: make it current
-    int ii, t;        // two-loop index and memory slot
-    LbLayout lay;
+    int blocks;       // partial-sum slots of the lattice passes to sum (3 doubles each, the first |F|^2)
     double b1, b2;    // Adam
     int scheduled;    // Nesterov
     double* scal;
     Common c;
 };
 
-// One work-group: fixed-order sums of the streaming kernel's partials, then the
-// minimizer's scalar step in thread 0.
+// One work-group: fixed-order sum of the lattice passes' partials of |F|^2, then
+// the minimizer's scalar step in thread 0 and the flip to the state set that
+// the passes wrote.
 __global__ void __launch_bounds__(kVecThreads) vec_finalize_kernel(FinArgs A) {
-    __shared__ double red[kVecThreads / 64][kMaxDots];
+    __shared__ double red[kVecThreads / 64];
     Ctrl* ctrl = A.c.ctrl;
     if (ctrl->done) return;
-    double tot[kMaxDots] = {0, 0, 0, 0};
-    const int stride = A.stride;
-    for (int j = threadIdx.x; j < A.blocks; j += kVecThreads) {
-#pragma unroll
-        for (int k = 0; k < kMaxDots; ++k)
-            if (k < stride) tot[k] += A.c.partials[(long long)stride * j + k];
-    }
-    block_sum<kMaxDots>(tot, red);
+    double tot = 0;
+    for (int j = threadIdx.x; j < A.blocks; j += kVecThreads) tot += A.c.partials[3LL * j];
+    tot = wsum(tot);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = tot;
+    __syncthreads();
     if (threadIdx.x != 0) return;
+    tot = 0;
+#pragma unroll
+    for (int w = 0; w < kVecThreads / 64; ++w) tot += red[w];
     double* scal = A.scal;
-    const LbLayout& L = A.lay;
-    switch (A.op) {
-        case kFinAdam:
-            // beta^t advances once per executed step (energyMinimizerAdam.cpp:52-53)
-            scal[0] = scal[0] * A.b1;
-            scal[1] = scal[1] * A.b2;
-            finish_iteration(ctrl, sqrt(tot[0]) / A.c.ndof, A.c.fc, A.c.trace);
-            if (A.flip) ctrl->cur ^= 1;
-            break;
-        case kFinNesterov: {
-            // the same lambda and momentum the step kernel computed from scal[0]
-            const double oldLambda = scal[0];
-            const double lambda = 0.5 * (1.0 + sqrt(1.0 + 4.0 * oldLambda * oldLambda));
-            const double gamma = (1 - oldLambda) / lambda;
-            if (A.scheduled) scal[1] = 1. + gamma;
-            scal[0] = lambda;
-            finish_iteration(ctrl, sqrt(tot[0]) / A.c.ndof, A.c.fc, A.c.trace);
-            if (A.flip) ctrl->cur ^= 1;
-            break;
-        }
-        case kFinAlpha: {
-            const double sy = scal[L.SY(A.t)];
-            double a = 0;
-            if (sy != 0) a = tot[0] / sy;
-            scal[L.A(A.ii)] = a;
-            scal[L.NA(A.ii)] = -a;
-            break;
-        }
-        case kFinBeta: {
-            const double sy = scal[L.SY(A.t)];
-            double cs = 0;
-            if (sy != 0) {
-                const double beta = tot[0] / sy;
-                cs = scal[L.A(A.ii)] - beta;
-            }
-            scal[L.CS(A.ii)] = cs;
-            break;
-        }
-        case kFinLbFinish:
-        case kFinLbStart: {
-            if (A.op == kFinLbFinish) {
-                scal[L.SY(A.t)] = tot[1];
-                scal[L.YY(A.t)] = tot[2];
-            }
-            const double syt = scal[L.SY(A.t)], yyt = scal[L.YY(A.t)];
-            double a = 0;
-            if (syt != 0) a = tot[3] / syt;
-            scal[L.A(0)] = a;
-            scal[L.NA(0)] = -a;
-            scal[L.K3()] = yyt != 0 ? syt / yyt : 0.0;
-            if (A.op == kFinLbFinish) finish_iteration(ctrl, sqrt(tot[0]) / A.c.ndof, A.c.fc, A.c.trace);
-            break;
-        }
+    if (A.op == kFinAdam) {
+        // beta^t advances once per executed step (energyMinimizerAdam.cpp:52-53)
+        scal[0] = scal[0] * A.b1;
+        scal[1] = scal[1] * A.b2;
+    } else {
+        // the same lambda and momentum the step kernel computed from scal[0]
+        const double oldLambda = scal[0];
+        const double lambda = 0.5 * (1.0 + sqrt(1.0 + 4.0 * oldLambda * oldLambda));
+        const double gamma = (1 - oldLambda) / lambda;
+        if (A.scheduled) scal[1] = 1. + gamma;
+        scal[0] = lambda;
     }
-}
-
-int vec_blocks(long long len) {
-    const long long per = (long long)kVecThreads * kVecUnroll;
-    return (int)std::max<long long>(1, std::min<long long>((len + per - 1) / per, kVecMaxBlocks));
+    finish_iteration(ctrl, sqrt(tot) / A.c.ndof, A.c.fc, A.c.trace);
+    ctrl->cur ^= 1;
 }
 
 }  // namespace
@@ -335,7 +353,8 @@ struct VecMinimizer {
     uint64_t bound = 0;   // serial of the lattice the vectors belong to (0: none)
     long long boundN = 0;
     int boundPrecision = -1;
-    std::vector<void*> vecs;
+    std::vector<void*> vecs;     // in one allocation, stride reals apart
+    long long stride = 0;
     double* dScal = nullptr;
     int scalCount = 0;
     double* dPartials = nullptr;
@@ -353,7 +372,7 @@ struct VecMinimizer {
     }
     // drops the device history (the trace buffer stays)
     void release() {
-        for (void* p : vecs) (void)hipFree(p);
+        if (!vecs.empty()) (void)hipFree(vecs[0]);
         vecs.clear();
         if (dScal) (void)hipFree(dScal);
         if (dPartials) (void)hipFree(dPartials);
@@ -366,23 +385,22 @@ struct VecMinimizer {
     bool needs_bind(const qm_lattice* L) const {
         return bound != L->serial || boundN != L->n || boundPrecision != L->precision;
     }
-    // (re)allocates nv zeroed vectors and nscal zeroed scalars for lattice L
-    int bind(qm_lattice* L, int nv, int nscal) {
+    // (re)allocates nv zeroed vectors, nscal zeroed scalars and nparts partial
+    // sums of its own for lattice L
+    int bind(qm_lattice* L, int nv, int nscal, size_t nparts = 0) {
         release();
-        const size_t bytes = 5 * (size_t)L->n * L->realSize;
-        for (int k = 0; k < nv; ++k) {
-            void* p = nullptr;
-            if (hipMalloc(&p, bytes) != hipSuccess) {
-                release();
-                return fail(QM_ENOMEM, "minimizer vectors: out of device memory");
-            }
-            vecs.push_back(p);
-            HIP_TRY(hipMemsetAsync(p, 0, bytes, L->stream));
-        }
+        const size_t align = 256 / L->realSize;   // each vector on a 256-byte boundary
+        stride = (long long)((5 * (size_t)L->n + align - 1) / align * align);
+        const size_t bytes = (size_t)stride * L->realSize;
+        char* base = nullptr;
+        if (hipMalloc(&base, nv * bytes) != hipSuccess)
+            return fail(QM_ENOMEM, "minimizer vectors: out of device memory");
+        for (int k = 0; k < nv; ++k) vecs.push_back(base + k * bytes);
+        HIP_TRY(hipMemsetAsync(base, 0, nv * bytes, L->stream));
         HIP_TRY(hipMalloc(&dScal, std::max(nscal, 1) * sizeof(double)));
         HIP_TRY(hipMemsetAsync(dScal, 0, std::max(nscal, 1) * sizeof(double), L->stream));
         scalCount = nscal;
-        HIP_TRY(hipMalloc(&dPartials, (size_t)kVecMaxBlocks * kMaxDots * sizeof(double)));
+        if (nparts) HIP_TRY(hipMalloc(&dPartials, nparts * sizeof(double)));
         bound = L->serial;
         boundN = L->n;
         boundPrecision = L->precision;
@@ -410,15 +428,12 @@ struct VecMinimizer {
         HIP_TRY(hipMemcpyAsync(dScal + offset, v, count * sizeof(double), hipMemcpyHostToDevice, L->stream));
         return QM_OK;
     }
-    // the finalize kernel for a streaming kernel of `blocks` work-groups, or
-    // (partials given) for a lattice pass of `blocks` slots of 3 doubles
-    int finalize(const qm_lattice* L, FinArgs a, long long blocks, double* partials = nullptr) const {
+    // the finalize kernel for a lattice pass of `blocks` partial-sum slots
+    int finalize(const qm_lattice* L, FinArgs a, long long blocks) const {
         a.blocks = (int)blocks;
-        a.stride = partials ? 3 : kMaxDots;
-        a.flip = partials ? 1 : 0;
         a.scal = dScal;
         a.c = common(L);
-        if (partials) a.c.partials = partials;
+        a.c.partials = L->dPartials;
         vec_finalize_kernel<<<1, kVecThreads, 0, L->stream>>>(a);
         HIP_TRY(hipGetLastError());
         return QM_OK;
@@ -506,7 +521,7 @@ static int adam_enqueue(qm_adam* m, qm_lattice* L, const qm_ldg* f) {
     fa.op = kFinAdam;
     fa.b1 = m->b1;
     fa.b2 = m->b2;
-    return m->finalize(L, fa, slots, L->dPartials);
+    return m->finalize(L, fa, slots);
 }
 
 extern "C" {
@@ -594,7 +609,7 @@ static int nesterov_enqueue(qm_nesterov* m, qm_lattice* L, const qm_ldg* f) {
     FinArgs fa{};
     fa.op = kFinNesterov;
     fa.scheduled = m->scheduled;
-    return m->finalize(L, fa, slots, L->dPartials);
+    return m->finalize(L, fa, slots);
 }
 
 extern "C" {
@@ -675,107 +690,48 @@ struct qm_lolbfgs : VecMinimizer {
     int scheduled = 0;
     int cur = 0;   // currentIterationInMLoop
     bool fresh = true;   // p must be (re)started from the forces: new or re-initialised history
-    // vecs: [0] p, [1 .. m] s, [m+1 .. 2m] y
-    void* p() const { return vecs[0]; }
-    void* s(int t) const { return vecs[1 + t]; }
-    void* y(int t) const { return vecs[1 + m + t]; }
+    // vecs: [0 .. m-1] s, [m .. 2m-1] y, [2m] the direction a call ended with: p = F,
+    // of which the coefficients kept for the next call are
 };
 
 template <typename R>
-static int lb_enqueue(qm_lolbfgs* M, qm_lattice* L, const qm_ldg* f, int iteration) {
+static int lb_enqueue(qm_lolbfgs* M, qm_lattice* L, const qm_ldg* f, int iteration, bool first) {
     const int m = M->m, c = M->cur;
-    const LbLayout lay{m};
     const StateSet<R> st = state_set<R>(L, L->hCtrl.cur);
-    const Common com = M->common(L);
-    const int blocks = vec_blocks(com.len);
-    auto slot = [&](int ii) { return (c - ii - 1 + m) % m; };
-    if (iteration == 0 || M->fresh) {
-        // step 1 (energyMinimizerLoLBFGS.cpp:107-114): p = F(Q); then alpha_0 and
-        // the step-3 factor of the (empty) newest slot.  A history re-initialised
-        // after iterations also restarts here: its direction vector is new.
+    LbArgs<R> a{};
+    a.hist = rp<R>(M->vecs[0]);
+    a.stride = M->stride;
+    a.f = st.f;
+    a.p = first ? rp<R>(M->vecs[2 * m]) : st.f;
+    a.q = st.q;
+    a.m = m;
+    a.c = c;
+    a.scal = M->dScal;
+    a.c0 = M->common(L);
+    if (M->fresh) {
+        // step 1 (energyMinimizerLoLBFGS.cpp:107-114): p = F(Q); the history is
+        // empty and its coefficients are zero.  A history re-initialised after
+        // iterations also starts here.
         M->fresh = false;
         if (int rc = force_pass(L, f, true)) return rc;
-        LbFinishArgs<R> a{};
-        a.p = rp<R>(M->p());
-        a.f = st.f;
-        a.s = rp<R>(M->s(slot(0)));
-        a.y = nullptr;
-        a.c = com;
-        lb_finish_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
-        HIP_TRY(hipGetLastError());
-        FinArgs fa{};
-        fa.op = kFinLbStart;
-        fa.t = slot(0);
-        fa.lay = lay;
-        if (int rc = M->finalize(L, fa, blocks)) return rc;
+        a.p = st.f;
     }
-    auto stage = [&](const R* x1, int k1, const R* x2, int k2, const R* d, int op, int ii, int t) {
-        LbStageArgs<R> a{};
-        a.p = rp<R>(M->p());
-        a.x1 = x1;
-        a.x2 = x2;
-        a.d = d;
-        a.k1 = k1;
-        a.k2 = k2;
-        a.scal = M->dScal;
-        a.c = com;
-        lb_stage_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
-        HIP_TRY(hipGetLastError());
-        FinArgs fa{};
-        fa.op = op;
-        fa.ii = ii;
-        fa.t = t;
-        fa.lay = lay;
-        return M->finalize(L, fa, blocks);
-    };
-    // step 2: p -= alpha_ii y; alpha_{ii+1} = s.p / s.y (newest first)
-    for (int ii = 0; ii + 1 < m; ++ii)
-        if (int rc = stage(rp<R>(M->y(slot(ii))), lay.NA(ii), nullptr, 0, rp<R>(M->s(slot(ii + 1))), kFinAlpha,
-                           ii + 1, slot(ii + 1)))
-            return rc;
-    // last step-2 update fused with step 3 (p += (s.y / y.y) y of the newest
-    // slot), then beta of the oldest slot
-    if (int rc = stage(rp<R>(M->y(slot(m - 1))), lay.NA(m - 1), rp<R>(M->y(slot(0))), lay.K3(),
-                       rp<R>(M->y(slot(m - 1))), kFinBeta, m - 1, slot(m - 1)))
-        return rc;
-    // step 4: p += (alpha_ii - beta_ii) s; beta_{ii-1} = y.p / s.y (oldest first)
-    for (int ii = m - 1; ii >= 1; --ii)
-        if (int rc = stage(rp<R>(M->s(slot(ii))), lay.CS(ii), nullptr, 0, rp<R>(M->y(slot(ii - 1))), kFinBeta,
-                           ii - 1, slot(ii - 1)))
-            return rc;
+    const long long pairs = (a.c0.len + 1) / 2;
+    const int blocks = (int)std::min<long long>((pairs + kVecThreads - 1) / kVecThreads, kLbBlocks);
     // update step: eta as minimize() sets it (energyMinimizerLoLBFGS.cpp:203-209)
-    const double eta = M->scheduled ? M->tau / (M->tau + iteration) * M->dt : M->dt;
-    {
-        LbMoveArgs<R> a{};
-        a.p = rp<R>(M->p());
-        a.s0 = rp<R>(M->s(slot(0)));
-        a.sc = rp<R>(M->s(c));
-        a.yc = rp<R>(M->y(c));
-        a.q = st.q;
-        a.f = st.f;
-        a.eta = eta;
-        a.k = lay.CS(0);
-        a.scal = M->dScal;
-        a.c = com;
-        lb_move_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
-        HIP_TRY(hipGetLastError());
-    }
+    a.eta = M->scheduled ? M->tau / (M->tau + iteration) * M->dt : M->dt;
+    lb_move_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
+    HIP_TRY(hipGetLastError());
     if (int rc = force_pass(L, f, true)) return rc;
-    {
-        LbFinishArgs<R> a{};
-        a.p = rp<R>(M->p());
-        a.f = st.f;
-        a.s = rp<R>(M->s(c));
-        a.y = rp<R>(M->y(c));
-        a.c = com;
-        lb_finish_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
+    for (a.t0 = 0; a.t0 < m; a.t0 += kLbBlock) {
+        lb_dots_kernel<R><<<blocks, kVecThreads, 0, L->stream>>>(a);
         HIP_TRY(hipGetLastError());
-        FinArgs fa{};
-        fa.op = kFinLbFinish;
-        fa.t = c;
-        fa.lay = lay;
-        if (int rc = M->finalize(L, fa, blocks)) return rc;
     }
+    if (m <= kLbLdsMemory)
+        lb_coef_kernel<true><<<1, kLbCoefThreads, 0, L->stream>>>(a.c0, M->dScal, LbLayout{m}, c, blocks);
+    else
+        lb_coef_kernel<false><<<1, kLbCoefThreads, 0, L->stream>>>(a.c0, M->dScal, LbLayout{m}, c, blocks);
+    HIP_TRY(hipGetLastError());
     M->cur = (c + 1) % m;
     return QM_OK;
 }
@@ -819,7 +775,8 @@ int qm_lolbfgs_minimize(qm_lolbfgs* M, qm_ldg* f, qm_lattice* L) {
     if (!M || !f || !L) return fail(QM_EINVAL, "null handle");
     if (M->needs_bind(L)) {
         // initializeFromModel (energyMinimizerLoLBFGS.cpp:32-52): zero history
-        if (int rc = M->bind(L, 1 + 2 * M->m, LbLayout{M->m}.size())) return rc;
+        const int launches = (M->m + kLbBlock - 1) / kLbBlock;
+        if (int rc = M->bind(L, 2 * M->m + 1, LbLayout{M->m}.size(), (size_t)launches * kLbDots * kLbBlocks)) return rc;
         M->fresh = true;
         M->iterations = 0;
         M->cur = 0;
@@ -828,11 +785,15 @@ int qm_lolbfgs_minimize(qm_lolbfgs* M, qm_ldg* f, qm_lattice* L) {
     if (int rc = begin_run(*M, L, f, false)) return rc;
     const int cur0 = M->cur, it0 = M->iterations;
     auto enq = [&](int iteration) {
-        return L->precision == QM_FP64 ? lb_enqueue<double>(M, L, f, iteration)
-                                       : lb_enqueue<float>(M, L, f, iteration);
+        return L->precision == QM_FP64 ? lb_enqueue<double>(M, L, f, iteration, iteration == it0)
+                                       : lb_enqueue<float>(M, L, f, iteration, iteration == it0);
     };
     int rc = drive(*M, L, enq);
     M->cur = (cur0 + (M->iterations - it0)) % M->m;
+    // the next call's first direction: whatever computes forces on the lattice in
+    // between, it starts from these
+    HIP_TRY(hipMemcpyAsync(M->vecs[2 * M->m], static_cast<char*>(L->dSet[L->hCtrl.cur]) + 10 * (size_t)L->n * L->realSize,
+                           5 * (size_t)L->n * L->realSize, hipMemcpyDeviceToDevice, L->stream));
     return rc;
 }
 
