@@ -69,14 +69,16 @@ int qm_lattice_set_stream(qm_lattice* lat, void* stream);
  * knob of this implementation; it has no counterpart in the reference. */
 int qm_lattice_set_zchunk(qm_lattice* lat, int zchunk);
 /* tile shape of the fused lattice pass: -1 (default) picks by precision, 0 is
- * 32x8 sites per work-group, 1 is 64x4, 2 is 32x16, 3 is 64x8.  A tuning knob of this
- * implementation. */
+ * 32x8 sites per work-group, 1 is 64x4, 2 is 32x16, 3 is 64x8.  -1 also lets small
+ * lattices take a pass over 16x4x4 blocks.  A tuning knob of this implementation. */
 int qm_lattice_set_tile(qm_lattice* lat, int tile);
 /* tile autotuner, the role of kernelTuner (src/utilities/kernelTuner.cpp:5-125):
  * times the fused FIRE pass with HIP events for every tile shape and z chunks
  * {automatic, 8, 16, 32, 64} on the lattice's current state (which it leaves
  * unchanged), keeps the fastest on the lattice and returns it (any output may be
- * NULL).  Explicit, so that a run's reduction order does not depend on timing. */
+ * NULL).  Where a small lattice's own choice, the block pass, is faster than all
+ * of them, the lattice keeps that, and ms is its time.  Explicit, so that a run's
+ * reduction order does not depend on timing. */
 int qm_lattice_autotune(qm_lattice* lat, qm_ldg* f, int* tile, int* zchunk, double* ms);
 /* converts the device state (Q, v, F) to the other storage precision, e.g. for an
  * FP64 polish after an FP32 minimization; minimizers bound to the lattice other

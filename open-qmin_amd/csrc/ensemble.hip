@@ -85,7 +85,9 @@ static int ensemble_tile(const qm_ensemble* E, const qm_lattice* L) {
         return w32 < w64 ? kTile32x8 : kTile64x8;
     }
     // batched passes have the tiles of the fused pass only
-    return active_tile(E->lats[0], kForce);
+    const qm_lattice* first = E->lats[0];
+    const int set = first->tileOverride;
+    return set >= 0 && set < kNumMarchTiles ? set : march_tile(first, kForce);
 }
 
 template <typename R>
@@ -105,7 +107,7 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
         // whole columns (or chunks of 32 planes): an ensemble has work-groups enough
         L->zchunk = E->zchunk > 0 ? E->zchunk : L->zchunkOverride > 0 ? L->zchunkOverride : std::min(L->lz, 32);
         FireConst fc = fire_const(params, L);
-        fill_args<R>(L, f, md[k], bd[k], fc, tile);
+        fill_args<R>(L, f, md[k], bd[k], fc, tile, true);
         L->tileOverride = ownTile;
         L->zchunk = ownZ;
         md[k].gate = 0;

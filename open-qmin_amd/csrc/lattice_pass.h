@@ -252,13 +252,40 @@ __device__ __forceinline__ void wait_plane(const R (&a)[5], const R (&b)[5], int
     asm volatile("" ::"v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]) : "memory");
 }
 
+// The pending FIRE velocity mix v = ck u + cf F, (1, 0) when none is pending and
+// (0, 0) after a reset (energyMinimizerFIRE.cpp:117-144), and the step.
+template <typename R>
+struct FireMove {
+    R dt, hdt, hdt2, ck, cf;
+};
+
+template <typename R>
+__device__ __forceinline__ FireMove<R> fire_move(const Ctrl* ctrl) {
+    const double dtd = ctrl->dt;
+    const int reset = ctrl->reset, identity = ctrl->identity;
+    return {R(dtd), R(0.5 * dtd), R(0.5 * dtd * dtd), reset ? R(0) : (identity ? R(1) : R(ctrl->cKeep)),
+            (reset || identity) ? R(0) : R(ctrl->cForce)};
+}
+
+// Velocity-Verlet drift of one site with the pending mix: q + dt v + dt^2/2 F, and
+// the half-kicked velocity v + dt/2 F (velocityVerlet.cpp:8-40).  The products
+// are contracted by hand, so that every pass that drifts a site rounds alike.
+template <typename R>
+__device__ __forceinline__ R fire_drift(const FireMove<R>& m, R q, R u, R f, R& vh) {
+    const R v = __builtin_elementwise_fma(m.ck, u, m.cf * f);
+    vh = __builtin_elementwise_fma(m.hdt, f, v);
+    return q + __builtin_elementwise_fma(m.dt, v, m.hdt2 * f);
+}
+
 // One work-group's share of the fused pass: the column of tile `logical` (x
 // tile fastest, then y tile, then z chunk) of the lattice described by A; its
 // partial sums go to slot `slot`.
-template <typename R, int MODE, int TERMS, int TILE>
+// NARROW: the tile is A.tw x A.th sites (an ensemble's lattices, whose rows may
+// be shorter than TX), else TX x TY.
+template <typename R, int MODE, int TERMS, int TILE, bool NARROW>
 __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logical, const int slot) {
-    using T = Tile<kTileTX[TILE], kTileTY[TILE]>;
-    constexpr int kTX = T::TX, kTY = T::TY, kHX = T::HX, kHY = T::HY, kHP = T::HP, kHalo = T::Halo;
+    using T = Tile<kTileTX[TILE], kTileTY[TILE], NARROW ? tile_rows<R>(TILE) : kTileTY[TILE]>;
+    constexpr int kHX = T::HX, kHP = T::HP;
     __shared__ R sQ[3][5][kHP];
     __shared__ double sRed[T::Threads / 64][3];
 
@@ -267,18 +294,8 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     const int cur = ctrl->cur;
     const StateSet<R> in = A.set[cur];
     const StateSet<R> out = A.set[MODE == kForce ? cur : cur ^ 1];
-    // pending FIRE velocity mix v = ck u + cf F: (1, 0) when none is pending,
-    // (0, 0) after a reset (energyMinimizerFIRE.cpp:117-144)
-    R dt = 0, hdt = 0, hdt2 = 0, ck = 0, cf = 0;
-    if (MODE == kFire) {
-        const double dtd = ctrl->dt;
-        dt = R(dtd);
-        hdt = R(0.5 * dtd);
-        hdt2 = R(0.5 * dtd * dtd);
-        const int reset = ctrl->reset, identity = ctrl->identity;
-        ck = reset ? R(0) : (identity ? R(1) : R(ctrl->cKeep));
-        cf = (reset || identity) ? R(0) : R(ctrl->cForce);
-    }
+    FireMove<R> mv{};
+    if (MODE == kFire) mv = fire_move<R>(ctrl);
     StepCoef<R> sk{};
     if constexpr (is_step_mode(MODE)) sk = step_coef<R, MODE>(A.step);
 
@@ -293,74 +310,71 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     const long long n = A.n;
     const long long plane = (long long)lx * ly;
     const int tid = threadIdx.x;
-    const int ox = tid % kTX, oy = tid / kTX;
-    const int x = txi * kTX + ox, y = tyi * kTY + oy;
-    const bool active = x < lx && y < ly;
-    const int hOwn = (oy + 1) * kHX + (ox + 1);
-    const long long colOwn = wrapi(x, lx) + (long long)lx * wrapi(y, ly);
+    const int tw = NARROW ? A.tw : T::TX, th = NARROW ? A.th : T::TY;
+    const int ox = tid % tw, oy = tid / tw;
+    const bool own = !NARROW || oy < th;   // a narrow tile may leave threads over
+    const int x = txi * tw + ox, y = tyi * th + oy;
+    const bool active = own && x < lx && y < ly;
+    const int hOwn = own ? (oy + 1) * kHX + (ox + 1) : 0;
+    const long long colOwn = own ? wrapi(x, lx) + (long long)lx * wrapi(y, ly) : 0;
     int hHalo = -1;
     long long colHalo = 0;
-    if (tid < kHalo) {
-        const int k = tid;
-        if (k < kHX)
-            hHalo = k;
-        else if (k < 2 * kHX)
-            hHalo = (kHY - 1) * kHX + (k - kHX);
-        else if (k < 2 * kHX + (kHY - 2))
-            hHalo = (1 + k - 2 * kHX) * kHX;
-        else
-            hHalo = (1 + k - 2 * kHX - (kHY - 2)) * kHX + (kHX - 1);
-        const int hx = hHalo % kHX, hy = hHalo / kHX;
-        colHalo = wrapi(txi * kTX - 1 + hx, lx) + (long long)lx * wrapi(tyi * kTY - 1 + hy, ly);
+    if (tid < 2 * (tw + 2) + 2 * th) {
+        const int k = tid, w = tw + 2;
+        int hx, hy;
+        if (k < 2 * w) {
+            hx = k < w ? k : k - w;
+            hy = k < w ? 0 : th + 1;
+        } else {
+            const int m = k - 2 * w;
+            hx = m < th ? 0 : tw + 1;
+            hy = 1 + (m < th ? m : m - th);
+        }
+        hHalo = hy * kHX + hx;
+        colHalo = wrapi(txi * tw - 1 + hx, lx) + (long long)lx * wrapi(tyi * th - 1 + hy, ly);
     }
 
     // Stage plane z into slot s (FIRE: pending mix, drift and first half kick);
-    // returns the owner's half-kicked velocity and class.
+    // returns the owner's half-kicked velocity and class.  The own and the halo
+    // site are loaded together in the FP32 passes that read Q alone (150^3 Adam:
+    // 130 against 141 us per iteration); elsewhere that gains nothing (FIRE, FP32,
+    // 256^3: 437 against 431 us; Nesterov, FP64, 192 x 150 x 130: 194 against 189).
+    constexpr bool kTogether = sizeof(R) == 4 && MODE != kFire;
+    auto load_site = [&](long long i, R* q, R* u, R* f) {
+#pragma unroll
+        for (int c = 0; c < 5; ++c) q[c] = in.q[c * n + i];
+        if (MODE == kFire) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                u[c] = in.u[c * n + i];
+                f[c] = in.f[c * n + i];
+            }
+        }
+    };
+    auto put_site = [&](int s, int h, R* q, const R* u, const R* f, R* vh) {
+        if (MODE == kFire) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) {
+                R half;
+                q[c] = fire_drift(mv, q[c], u[c], f[c], half);
+                if (vh) vh[c] = half;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 5; ++c) sQ[s][c][h] = q[c];
+    };
     auto stage = [&](int z, int s, R* vh, int& cOwn) {
         const long long zoff = plane * wrapi(z, lz);
-        {
-            const long long i = colOwn + zoff;
-            cOwn = A.cls[i];
-            R q[5];
-#pragma unroll
-            for (int c = 0; c < 5; ++c) q[c] = in.q[c * n + i];
-            if (MODE == kFire) {
-                R u[5], f[5];
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    u[c] = in.u[c * n + i];
-                    f[c] = in.f[c * n + i];
-                }
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    const R v = ck * u[c] + cf * f[c];
-                    q[c] = q[c] + (dt * v + hdt2 * f[c]);
-                    vh[c] = v + hdt * f[c];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 5; ++c) sQ[s][c][hOwn] = q[c];
+        R q[5], u[5], f[5], hq[5], hu[5], hf[5];
+        if (own) {
+            cOwn = A.cls[colOwn + zoff];
+            load_site(colOwn + zoff, q, u, f);
         }
+        if (kTogether && hHalo >= 0) load_site(colHalo + zoff, hq, hu, hf);
+        if (own) put_site(s, hOwn, q, u, f, vh);
         if (hHalo >= 0) {
-            const long long i = colHalo + zoff;
-            R q[5];
-#pragma unroll
-            for (int c = 0; c < 5; ++c) q[c] = in.q[c * n + i];
-            if (MODE == kFire) {
-                R u[5], f[5];
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    u[c] = in.u[c * n + i];
-                    f[c] = in.f[c * n + i];
-                }
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    const R v = ck * u[c] + cf * f[c];
-                    q[c] = q[c] + (dt * v + hdt2 * f[c]);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 5; ++c) sQ[s][c][hHalo] = q[c];
+            if (!kTogether) load_site(colHalo + zoff, hq, hu, hf);
+            put_site(s, hHalo, hq, hu, hf, nullptr);
         }
     };
 
@@ -370,9 +384,11 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     auto fetch = [&](int z) {
         const long long zoff = plane * wrapi(z, lz);
         const long long i = colOwn + zoff;
-        pc = A.cls[i];
+        if (own) {
+            pc = A.cls[i];
 #pragma unroll
-        for (int c = 0; c < 5; ++c) pq[c] = in.q[c * n + i];
+            for (int c = 0; c < 5; ++c) pq[c] = in.q[c * n + i];
+        }
         if (hHalo >= 0) {
             const long long j = colHalo + zoff;
 #pragma unroll
@@ -393,8 +409,10 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     for (int z = z0; z < z1; ++z) {
         const int sm = (z - z0) % 3, sc = (z - z0 + 1) % 3, sp = (z - z0 + 2) % 3;
         if constexpr (kPF) {
+            if (own) {
 #pragma unroll
-            for (int c = 0; c < 5; ++c) sQ[sp][c][hOwn] = pq[c];
+                for (int c = 0; c < 5; ++c) sQ[sp][c][hOwn] = pq[c];
+            }
             if (hHalo >= 0) {
 #pragma unroll
                 for (int c = 0; c < 5; ++c) sQ[sp][c][hHalo] = ph[c];
@@ -438,7 +456,7 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
                 if (MODE == kFire) {
                     R u[5];
 #pragma unroll
-                    for (int c = 0; c < 5; ++c) u[c] = vhCur[c] + hdt * F[c];
+                    for (int c = 0; c < 5; ++c) u[c] = __builtin_elementwise_fma(mv.hdt, F[c], vhCur[c]);
 #pragma unroll
                     for (int c = 0; c < 5; ++c) {
                         st_out(&out.q[c * n + i], q[c]);
@@ -498,6 +516,175 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     }
 }
 
+// The fused pass on a small lattice: a work-group owns a block of up to 16 x 4 x
+// 4 sites, one thread per site, and stages the block with its one-site halo in
+// LDS at once, so that a pass lasts one load latency and one force computation
+// instead of marching through planes that each wait for their loads.  The halo
+// is 1.5 sites per site, read mostly from L2.  FIRE iteration at 24^3, L1, FP64:
+// 12 against 20 us, at 50^3, L1..L3: 21 against 28 us (three launches each).
+template <typename R, int MODE, int TERMS>
+__device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logical, const int slot) {
+    using B = Block;
+    constexpr int kHX = B::HX, kHP = B::HP;
+    __shared__ R sQ[B::HZ][5][kHP];
+    __shared__ double sRed[B::Threads / 64][3];
+
+    Ctrl* ctrl = A.ctrl;
+    if ((MODE != kForce || A.gate) && ctrl->done) return;
+    const int cur = ctrl->cur;
+    const StateSet<R> in = A.set[cur];
+    const StateSet<R> out = A.set[MODE == kForce ? cur : cur ^ 1];
+    FireMove<R> mv{};
+    if (MODE == kFire) mv = fire_move<R>(ctrl);
+    StepCoef<R> sk{};
+    if constexpr (is_step_mode(MODE)) sk = step_coef<R, MODE>(A.step);
+
+    const int lx = A.lx, ly = A.ly, lz = A.lz, tw = A.tw, th = A.th, td = A.zchunk;
+    const long long n = A.n;
+    const int x0 = logical % A.nbx * tw, y0 = logical / A.nbx % A.nby * th, z0 = logical / A.nbx / A.nby * td;
+    const int tid = threadIdx.x;
+    auto site = [&](int hx, int hy, int hz) {
+        return wrapi(x0 - 1 + hx, lx) + (long long)lx * (wrapi(y0 - 1 + hy, ly) + (long long)ly * wrapi(z0 - 1 + hz, lz));
+    };
+    // the own site, then the halo: the planes below and above, the rims of the others
+    const int ox = tid % tw, oy = tid / tw % th, oz = tid / tw / th;
+    const bool own = oz < td, active = own && x0 + ox < lx && y0 + oy < ly && z0 + oz < lz;
+    const long long i = own ? site(ox + 1, oy + 1, oz + 1) : 0;
+    const int w = tw + 2, face = w * (th + 2), rim = 2 * w + 2 * th, halo = 2 * face + td * rim;
+    constexpr int kRounds = (B::Halo + B::Threads - 1) / B::Threads;
+    R q[5], u[5], f[5], hq[kRounds][5], hu[kRounds][5], hf[kRounds][5];
+    int hAt[kRounds], hZ[kRounds];
+    int cls = 1;
+    auto load_site = [&](long long j, R* a, R* b, R* c) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) a[k] = in.q[k * n + j];
+        if (MODE == kFire) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                b[k] = in.u[k * n + j];
+                c[k] = in.f[k * n + j];
+            }
+        }
+    };
+    if (own) {
+        cls = A.cls[i];
+        load_site(i, q, u, f);
+    }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int k = tid + r * B::Threads;
+        hAt[r] = -1;
+        if (k < halo) {
+            int hx, hy, hz;
+            if (k < 2 * face) {
+                const int m = k < face ? k : k - face;
+                hx = m % w;
+                hy = m / w;
+                hz = k < face ? 0 : td + 1;
+            } else {
+                const int m = (k - 2 * face) % rim;
+                hz = 1 + (k - 2 * face) / rim;
+                if (m < 2 * w) {
+                    hx = m < w ? m : m - w;
+                    hy = m < w ? 0 : th + 1;
+                } else {
+                    hx = m - 2 * w < th ? 0 : tw + 1;
+                    hy = 1 + (m - 2 * w < th ? m - 2 * w : m - 2 * w - th);
+                }
+            }
+            hAt[r] = hy * kHX + hx;
+            hZ[r] = hz;
+            load_site(site(hx, hy, hz), hq[r], hu[r], hf[r]);
+        }
+    }
+    R pre[2][5];
+    if constexpr (is_step_mode(MODE))
+        if (active && cls >= 0) step_load<R, MODE>(A.step, n, i, pre);
+    const int h = (oy + 1) * kHX + ox + 1;
+    R vh[5];
+    auto drift = [&](R* a, const R* b, const R* c, R* v2) {
+        if (MODE == kFire) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                R half;
+                a[k] = fire_drift(mv, a[k], b[k], c[k], half);
+                if (v2) v2[k] = half;
+            }
+        }
+    };
+    if (own) {
+        drift(q, u, f, vh);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) sQ[oz + 1][k][h] = q[k];
+    }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (hAt[r] >= 0) {
+            drift(hq[r], hu[r], hf[r], nullptr);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) sQ[hZ[r]][k][hAt[r]] = hq[r][k];
+        }
+    __syncthreads();
+    double pF = 0, pP = 0, pV = 0;
+    if (active && cls >= 0) {
+        R F[5];
+        if (cls == 0) {
+            fast_raw_force<R, TERMS, kHX, kHP>(A.fc, reinterpret_cast<ConstPtr<R>>(reinterpret_cast<uint64_t>(A.W)), sQ,
+                                               oz, oz + 1, oz + 2, h, q, F);
+            if (A.hvar) {
+                R fv[5];
+                varying_field_force(A.hvar, n, i, A.hvarP, fv);
+                finish_bulk(A.fc, F, fv);
+            } else {
+                finish_bulk<R>(A.fc, F, nullptr);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) F[k] = R(0);
+        }
+        if (MODE == kFire) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) vh[k] = __builtin_elementwise_fma(mv.hdt, F[k], vh[k]);
+            pF = qt_dot(F, F);
+            pP = qt_dot(F, vh);
+            pV = qt_dot(vh, vh);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                out.q[k * n + i] = q[k];
+                out.u[k * n + i] = vh[k];
+                out.f[k * n + i] = F[k];
+            }
+        } else if constexpr (is_step_mode(MODE)) {
+            R qn[5];
+            step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
+            pF = sq5(F);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                out.q[k * n + i] = qn[k];
+                out.f[k * n + i] = F[k];
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) out.f[k * n + i] = F[k];
+        }
+    } else if (MODE == kFire && active) {
+        // the boundary pass finishes U and F of this site
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            out.q[k * n + i] = q[k];
+            out.u[k * n + i] = vh[k];
+        }
+    }
+    if (MODE != kForce) {
+        block_sum3<B::Threads>(pF, pP, pV, sRed);
+        if (tid == 0) {
+            A.partials[3 * (long long)slot + 0] = pF;
+            A.partials[3 * (long long)slot + 1] = pP;
+            A.partials[3 * (long long)slot + 2] = pV;
+        }
+    }
+}
+
 // XCD-aware work-group order: consecutive hardware ids go round-robin over the
 // 8 XCDs; each XCD gets a contiguous run of logical tiles, so that tiles sharing
 // halos share an L2.  With PAIR, within each run of 64 tiles of an XCD its
@@ -531,7 +718,7 @@ constexpr int march_min_waves() {
 
 template <typename R, int MODE, int TERMS, int TILE>
 __global__ void __launch_bounds__(kTileThreads[TILE], (march_min_waves<R, MODE, TERMS, TILE>())) march_kernel(MarchArgs<R> A) {
-    march_body<R, MODE, TERMS, TILE>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
+    march_body<R, MODE, TERMS, TILE, false>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
 // The 512-thread tiles (32 x 16, 64 x 8; 8 waves): two work-groups per CU need
@@ -540,7 +727,20 @@ template <typename R, int MODE, int TERMS, int TILE>
 __global__ void __launch_bounds__(kTileThreads[TILE], 4) march_wide_kernel(MarchArgs<R> A) {
     static_assert(kTileThreads[TILE] == 512, "512-thread tiles only");
     constexpr bool kPair = sizeof(R) == 4 && TILE == kTile64x8;
-    march_body<R, MODE, TERMS, TILE>(A, xcd_logical<kPair>(blockIdx.x, A.nblocks), blockIdx.x);
+    march_body<R, MODE, TERMS, TILE, false>(A, xcd_logical<kPair>(blockIdx.x, A.nblocks), blockIdx.x);
+}
+
+// Waves per SIMD asked of the compiler for the block pass: left alone it holds
+// the operands of a whole stencil in registers (213 to 256 in FP64, one or two
+// waves); at four, 52 to 120 do without spills, with FP64 L6 138 at three.
+template <typename R, int TERMS>
+constexpr int block_min_waves() {
+    return TERMS == kMultiL6 && sizeof(R) == 8 ? 2 : 4;
+}
+
+template <typename R, int MODE, int TERMS>
+__global__ void __launch_bounds__(Block::Threads, (block_min_waves<R, TERMS>())) block_kernel(MarchArgs<R> A) {
+    block_body<R, MODE, TERMS>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
 // The fused pass over many lattices in one launch: map[b] = {lattice, logical
@@ -551,7 +751,7 @@ __global__ void __launch_bounds__(kTileThreads[TILE]) march_batch_kernel(const M
     // uniform over the work-group: read once, keep in scalar registers
     const int lat = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
     const int logical = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
-    march_body<R, MODE, TERMS, TILE>(descs[lat], logical, logical);
+    march_body<R, MODE, TERMS, TILE, true>(descs[lat], logical, logical);
 }
 
 template <typename R, int MODE, int TERMS, int TILE>
@@ -560,7 +760,7 @@ __global__ void __launch_bounds__(kTileThreads[TILE], 4) march_wide_batch_kernel
     static_assert(kTileThreads[TILE] == 512, "512-thread tiles only");
     const int lat = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
     const int logical = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
-    march_body<R, MODE, TERMS, TILE>(descs[lat], logical, logical);
+    march_body<R, MODE, TERMS, TILE, true>(descs[lat], logical, logical);
 }
 
 // ---------------------------------------------------------------- boundary pass

@@ -361,6 +361,7 @@ static const void* march_fn_tile(int tile) {
         case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4>);
         case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16>);
         case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8>);
+        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
         default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8>);
     }
 }
@@ -438,7 +439,7 @@ hipError_t launch_fire_finalize_batch(const FinalizeDesc* descs, EnsembleStatus*
 template <typename R>
 hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hipStream_t s) {
     void* args[] = {const_cast<MarchArgs<R>*>(&a)};
-    return hipLaunchKernel(march_fn<R>(mode, terms, tile), dim3(a.nblocks), dim3(kTileThreads[tile]), args, 0, s);
+    return hipLaunchKernel(march_fn<R>(mode, terms, tile), dim3(a.nblocks), dim3(tile_threads(tile)), args, 0, s);
 }
 
 template <typename R>
@@ -478,7 +479,7 @@ void launch_move_q(R* q, long long n, const int64_t* src, const int64_t* dst, lo
 template <typename R>
 int march_blocks_per_cu(int mode, int terms, int tile) {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, march_fn<R>(mode, terms, tile), kTileThreads[tile], 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, march_fn<R>(mode, terms, tile), tile_threads(tile), 0) !=
         hipSuccess)
         return 1;
     return blocks < 1 ? 1 : blocks;

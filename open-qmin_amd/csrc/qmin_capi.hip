@@ -990,10 +990,30 @@ static int upload_weights(qm_lattice* L, const qm_ldg* f) {
 // The tiles of the FIRE pass that keeps only Q and v (4..6) serve FIRE passes
 // without the L6 term; a force-only pass, or one with L6, then takes the
 // default of its kind.
+//
+// Small lattices take the block pass (block_body), unless a tile or z chunk is
+// set: up to 1.2 million sites with L6, 0.9 million for other FIRE passes, 0.4
+// million for other force passes and the Adam and Nesterov passes, which the
+// block's halo costs more.  Per iteration, marching and in blocks (us, FP64):
+// FIRE L1..L3 40^3 27 and 18, 64^3 33 and 27, 80^3 51 and 43, 96^3 65 and 64,
+// 112^3 103 and 128; FIRE L6 96^3 68 and 67, 104^3 101 and 91, 112^3 111 and 127;
+// Nesterov L1..L3 40^3 23 and 16, 64^3 26 and 21, 96^3 48 and 50; Adam L1 64^3
+// 24 and 25, 80^3 40 and 41; Nesterov L6 104^3 91 and 73.  FP32 crosses at the
+// same sizes or above.
+static bool takes_blocks(const qm_lattice* L, int mode) {
+    const long long most = L->terms == kMultiL6 ? 1200000 : (mode == kFire ? 900000 : 400000);
+    return L->tileOverride < 0 && L->zchunkOverride == 0 && L->n <= most;
+}
+
 int qmin::active_tile(const qm_lattice* L, int mode) {
     // the 64 x 8 FIRE tile that keeps only Q and v needs more LDS than a CU has in FP64
     const int t = (L->tileOverride == kStream64x8 && L->precision == QM_FP64) ? kStream32x16 : L->tileOverride;
     if (t >= 0 && !(is_stream_tile(t) && (mode != kFire || L->terms == kMultiL6))) return t;
+    if (takes_blocks(L, mode)) return kBlock;
+    return march_tile(L, mode);
+}
+
+int qmin::march_tile(const qm_lattice* L, int mode) {
     if (L->terms != kMultiL6 && L->lx >= 128 && L->ly >= 128) {
         if (L->precision == QM_FP64) return mode == kFire ? kStream32x16 : kTile32x16;
         return kTile64x8;
@@ -1002,12 +1022,13 @@ int qmin::active_tile(const qm_lattice* L, int mode) {
 }
 
 long long qmin::tile_columns(const qm_lattice* L, int tile) {
-    return (long long)((L->lx + kTileTX[tile] - 1) / kTileTX[tile]) * ((L->ly + kTileTY[tile] - 1) / kTileTY[tile]);
+    const TileGrid g = tile_grid(L->lx, L->ly, tile);
+    return (long long)g.nbx * g.nby;
 }
 
 template <typename R>
 void qmin::fill_args(qm_lattice* L, const qm_ldg* f, MarchArgs<R>& ma, BoundaryArgs<R>& ba, const FireConst& fire,
-                     int tile) {
+                     int tile, bool narrow) {
     ma.set[0] = state_set<R>(L, 0);
     ma.set[1] = state_set<R>(L, 1);
     ma.cls = L->dClass;
@@ -1017,8 +1038,11 @@ void qmin::fill_args(qm_lattice* L, const qm_ldg* f, MarchArgs<R>& ma, BoundaryA
     ma.lz = L->lz;
     ma.zchunk = std::min(L->zchunk, L->lz);
     ma.n = L->n;
-    ma.nbx = (L->lx + kTileTX[tile] - 1) / kTileTX[tile];
-    ma.nby = (L->ly + kTileTY[tile] - 1) / kTileTY[tile];
+    const TileGrid g = tile_grid(L->lx, L->ly, tile, narrow, narrow ? tile_rows<R>(tile) : 0);
+    ma.nbx = g.nbx;
+    ma.nby = g.nby;
+    ma.tw = g.tw;
+    ma.th = g.th;
     const int nbz = (L->lz + ma.zchunk - 1) / ma.zchunk;
     ma.nblocks = ma.nbx * ma.nby * nbz;
     ma.fc = force_const(f);
@@ -1047,9 +1071,9 @@ void qmin::fill_args(qm_lattice* L, const qm_ldg* f, MarchArgs<R>& ma, BoundaryA
 }
 
 template void qmin::fill_args<double>(qm_lattice*, const qm_ldg*, MarchArgs<double>&, BoundaryArgs<double>&,
-                                      const FireConst&, int);
+                                      const FireConst&, int, bool);
 template void qmin::fill_args<float>(qm_lattice*, const qm_ldg*, MarchArgs<float>&, BoundaryArgs<float>&,
-                                     const FireConst&, int);
+                                     const FireConst&, int, bool);
 
 // z chunk of the fused pass: as long as possible while the grid still fills
 // every CU to its occupancy, so that the whole grid is resident at once, all
@@ -1068,6 +1092,11 @@ static void choose_zchunk(qm_lattice* L, int mode, int terms) {
         if (L->numCUs <= 0) L->numCUs = 256;
     }
     const int tile = active_tile(L, mode);
+    if (tile == kBlock) {
+        const int nbz = (L->lz + Block::BZ - 1) / Block::BZ;
+        L->zchunk = (L->lz + nbz - 1) / nbz;
+        return;
+    }
     int perCU;
     if (is_stream_tile(tile))
         perCU = L->precision == QM_FP64 ? stream_blocks_per_cu<double>(terms, tile)
@@ -1185,8 +1214,17 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
         if (int rc = push_ctrl(L)) return rc;
     }
     const int reps = L->n >= (1 << 22) ? 5 : 20;
-    double best = 1e30;
+    double best = 1e30, blocks = 1e30;
     int bestTile = 0, bestZ = 0;
+    // the block pass of a small lattice is no tile that can be set: where it is
+    // the fastest, the lattice goes on choosing by itself
+    L->tileOverride = -1;
+    L->zchunkOverride = 0;
+    if (active_tile(L, kFire) == kBlock) {
+        const int rc = L->precision == QM_FP64 ? time_march<double>(L, f, reps, &blocks)
+                                               : time_march<float>(L, f, reps, &blocks);
+        if (rc) return rc;
+    }
     for (int tile = 0; tile < kNumTiles; ++tile) {
         for (int zc : {0, 8, 16, 32, 64}) {
             if (zc > L->lz) continue;
@@ -1203,15 +1241,15 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
             }
         }
     }
-    L->tileOverride = bestTile;
-    L->zchunkOverride = bestZ;
+    L->tileOverride = blocks < best ? -1 : bestTile;
+    L->zchunkOverride = blocks < best ? 0 : bestZ;
     if (savedDone) {
         L->hCtrl.done = savedDone;
         if (int rc = push_ctrl(L)) return rc;
     }
     if (tileOut) *tileOut = bestTile;
     if (zchunkOut) *zchunkOut = bestZ;
-    if (msOut) *msOut = best;
+    if (msOut) *msOut = std::min(best, blocks);
     return QM_OK;
 }
 
@@ -1225,6 +1263,8 @@ int qmin::prepare(qm_lattice* L, const qm_ldg* f) {
     // room for the smallest z chunk (4 planes) the fused pass may pick
     long long worst = 0;
     for (int t = 0; t < kNumTiles; ++t) worst = std::max(worst, tile_columns(L, t) * ((L->lz + 3) / 4));
+    if (takes_blocks(L, kFire) || takes_blocks(L, kForce))
+        worst = std::max(worst, tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ));
     const size_t need = 3 * (size_t)(worst + boundary_blocks(L->nBoundary));
     return ensure_partials(L, need);
 }

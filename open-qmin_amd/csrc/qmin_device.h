@@ -17,22 +17,72 @@ namespace qmin {
 constexpr int kThreads = 256;   // work-group size of the streaming kernels
 enum TileId {
     kTile32x8 = 0, kTile64x4 = 1, kTile32x16 = 2, kTile64x8 = 3, kNumMarchTiles = 4,
-    kStream32x16 = 4, kStream32x8 = 5, kStream64x8 = 6, kNumTiles = 7
+    kStream32x16 = 4, kStream32x8 = 5, kStream64x8 = 6, kNumTiles = 7,
+    kBlock = 7
 };
 constexpr int kTileTX[kNumTiles] = {32, 64, 32, 64, 32, 32, 64};
 constexpr int kTileTY[kNumTiles] = {8, 4, 16, 8, 16, 8, 8};
 constexpr int kTileThreads[kNumMarchTiles] = {32 * 8, 64 * 4, 32 * 16, 64 * 8};
-__host__ __device__ constexpr bool is_stream_tile(int tile) { return tile >= kNumMarchTiles; }
+__host__ __device__ constexpr bool is_stream_tile(int tile) { return tile >= kNumMarchTiles && tile < kNumTiles; }
 
-template <int TX_, int TY_>
+// Block of the fused pass on small lattices (kBlock, automatic only): sites a
+// work-group owns in x, y and z at most, one thread per site.
+struct Block {
+    static constexpr int BX = 16, BY = 4, BZ = 4;
+    static constexpr int Threads = BX * BY * BZ;
+    static constexpr int HX = BX + 2, HP = HX * (BY + 2), HZ = BZ + 2;   // halo-padded rows, planes and planes' count
+    static constexpr int Halo = HP * HZ - Threads;
+};
+
+// Rows of a tile at most in an ensemble's pass.  Where a lattice's rows are
+// shorter than TX, the threads this leaves over take more rows: a quarter more
+// than TY in FP32 (40 lattices of 24 to 96 sites, 64 x 4 tiles: 246 against 287
+// us per iteration).  In FP64 the planes of those rows would cost a work-group
+// per CU in LDS, and TY is the most.
+template <typename R>
+constexpr int tile_rows(int tile) {
+    return sizeof(R) == 4 ? kTileTY[tile] * 5 / 4 : kTileTY[tile];
+}
+
+// threads of a work-group of the fused pass
+inline int tile_threads(int tile) { return tile == kBlock ? Block::Threads : kTileThreads[tile]; }
+
+struct TileGrid {
+    int tw, th;      // sites of a tile in x and y
+    int nbx, nby;    // tiles in x and y
+};
+
+// Tiles of one lattice plane; narrow: rows shorter than TX make room for more of
+// them, up to rowsMax.
+inline TileGrid tile_grid(int lx, int ly, int tile, bool narrow = false, int rowsMax = 0) {
+    auto parts = [](int l, int most) { return (l + most - 1) / most; };
+    if (tile == kBlock) {
+        TileGrid g{0, 0, parts(lx, Block::BX), parts(ly, Block::BY)};
+        g.tw = parts(lx, g.nbx);
+        g.th = parts(ly, g.nby);
+        return g;
+    }
+    const int tx = kTileTX[tile], ty = kTileTY[tile];
+    TileGrid g{tx, ty, parts(lx, tx), parts(ly, ty)};
+    // (Longer rows are not cut into equal parts: 203 sites in tiles of 51 instead
+    // of 64 took 316 against 285 us in FP32, with a fifth fewer tiles, as more
+    // cache lines are shared between tiles and written in parts.)
+    if (!narrow || g.nbx > 1) return g;
+    g.tw = lx;
+    g.th = tx * ty / g.tw < rowsMax ? tx * ty / g.tw : rowsMax;
+    g.nby = parts(ly, g.th);
+    g.th = parts(ly, g.nby);
+    return g;
+}
+
+template <int TX_, int TY_, int Rows>
 struct Tile {
     static constexpr int TX = TX_, TY = TY_;
-    static constexpr int Threads = TX * TY;     // one site per thread
-    static constexpr int HX = TX + 2, HY = TY + 2;
-    static constexpr int HP = HX * HY;          // sites of one halo-padded plane
-    static constexpr int Halo = HP - TX * TY;   // perimeter sites of one plane
+    static constexpr int Threads = TX * TY;        // one site per thread
+    static constexpr int HX = TX + 2;              // row pitch of one halo-padded plane
+    static constexpr int HP = HX * (Rows + 2);     // sites of it
     static_assert(Threads % 64 == 0, "whole wave64s");
-    static_assert(Halo <= Threads, "one halo site per thread at most");
+    static_assert(2 * HX + 2 * Rows <= Threads, "one halo site per thread at most");
 };
 
 using SiteType = int16_t;                // site types on the device (reference encoding)
@@ -124,6 +174,7 @@ struct MarchArgs {
     int lx, ly, lz, zchunk;
     long long n;
     int nbx, nby, nblocks;
+    int tw, th;             // sites of a tile in x and y (tile_grid)
     ForceConst fc;
     Ctrl* ctrl;
     double* partials;   // [nblocks + boundary blocks][3]

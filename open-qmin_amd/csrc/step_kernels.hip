@@ -17,6 +17,7 @@ const void* step_fn_tile(int tile) {
         case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4>);
         case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16>);
         case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8>);
+        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
         default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8>);
     }
 }
@@ -41,16 +42,17 @@ const void* step_boundary_fn(int terms) {
 
 }  // namespace
 
-// Queues the fused pass (tile `tile`, one of the four halo-padded tiles) and
+// Queues the fused pass (tile `tile`, one of the halo-padded ones or kBlock) and
 // the boundary pass of one Adam or Nesterov iteration.
 template <typename R>
 hipError_t launch_step(const MarchArgs<R>& ma, const BoundaryArgs<R>& ba, int mode, int terms, int tile,
                        hipStream_t s) {
-    if (tile < 0 || tile >= kNumMarchTiles || !is_step_mode(mode)) return hipErrorInvalidValue;
+    if (!(tile >= 0 && tile < kNumMarchTiles) && tile != kBlock) return hipErrorInvalidValue;
+    if (!is_step_mode(mode)) return hipErrorInvalidValue;
     const void* fn = mode == kAdamStep ? step_fn_terms<R, kAdamStep>(terms, tile)
                                        : step_fn_terms<R, kNesterovStep>(terms, tile);
     void* margs[] = {const_cast<MarchArgs<R>*>(&ma)};
-    hipError_t e = hipLaunchKernel(fn, dim3(ma.nblocks), dim3(kTileThreads[tile]), margs, 0, s);
+    hipError_t e = hipLaunchKernel(fn, dim3(ma.nblocks), dim3(tile_threads(tile)), margs, 0, s);
     if (e != hipSuccess) return e;
     long long blocks = (ba.nsites + kBoundaryThreads - 1) / kBoundaryThreads;
     if (blocks < 1) blocks = 1;
