@@ -19,7 +19,7 @@ hipError_t launch_march_batch(const MarchArgs<R>* descs, const int2* map, int bl
                               hipStream_t s);
 template <typename R>
 hipError_t launch_boundary_batch(const BoundaryArgs<R>* descs, const int2* map, int blocks, int mode, int terms,
-                                 hipStream_t s);
+                                 bool lanes, hipStream_t s);
 hipError_t launch_fire_finalize_batch(const FinalizeDesc* descs, EnsembleStatus* status, int count, hipStream_t s);
 }  // namespace qmin
 
@@ -38,6 +38,7 @@ struct qm_ensemble {
     int2* dBoundaryMap = nullptr;
     EnsembleStatus* dStatus = nullptr;
     int boundaryBlocks = 0;
+    bool lanes = true;   // the batched boundary pass gives a site eight lanes
     // work-groups of the batched fused pass per tile shape, in one map: entries
     // [segOff[t], segOff[t] + segCount[t]) run with tile t (one launch each)
     int segOff[kNumMarchTiles] = {0, 0, 0, 0}, segCount[kNumMarchTiles] = {0, 0, 0, 0};
@@ -97,6 +98,9 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
     std::vector<BoundaryArgs<R>> bd(count);
     std::vector<FinalizeDesc> fd(count);
     std::vector<int2> mlog[kNumMarchTiles], blog;
+    long long sites = 0;
+    for (const qm_lattice* L : E->lats) sites += L->nBoundary;
+    E->lanes = boundary_lanes(terms_of(f), sites);
     for (int k = 0; k < count; ++k) {
         qm_lattice* L = E->lats[k];
         const int tile = ensemble_tile(E, L);
@@ -112,7 +116,7 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
         L->zchunk = ownZ;
         md[k].gate = 0;
         bd[k].gate = 0;
-        const int bb = boundary_blocks(L->nBoundary);
+        const int bb = boundary_blocks(L->nBoundary, E->lanes);
         for (int j = 0; j < md[k].nblocks; ++j) mlog[tile].push_back(make_int2(k, j));
         for (int j = 0; j < bb; ++j) blog.push_back(make_int2(k, j));
         fd[k].ctrl = L->dCtrl;
@@ -135,7 +139,7 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
     HIP_TRY(hipMalloc(&E->dBoundaryDescs, count * sizeof(BoundaryArgs<R>)));
     HIP_TRY(hipMalloc(&E->dFinal, count * sizeof(FinalizeDesc)));
     HIP_TRY(hipMalloc(&E->dMarchMap, mmap.size() * sizeof(int2)));
-    HIP_TRY(hipMalloc(&E->dBoundaryMap, blog.size() * sizeof(int2)));
+    if (!blog.empty()) HIP_TRY(hipMalloc(&E->dBoundaryMap, blog.size() * sizeof(int2)));
     HIP_TRY(hipMalloc(&E->dStatus, count * sizeof(EnsembleStatus)));
     // ordered on the ensemble's stream, before the launches that read them
     HIP_TRY(hipMemcpyAsync(E->dMarchDescs, md.data(), count * sizeof(MarchArgs<R>), hipMemcpyHostToDevice, E->stream));
@@ -143,8 +147,9 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
                            E->stream));
     HIP_TRY(hipMemcpyAsync(E->dFinal, fd.data(), count * sizeof(FinalizeDesc), hipMemcpyHostToDevice, E->stream));
     HIP_TRY(hipMemcpyAsync(E->dMarchMap, mmap.data(), mmap.size() * sizeof(int2), hipMemcpyHostToDevice, E->stream));
-    HIP_TRY(hipMemcpyAsync(E->dBoundaryMap, blog.data(), blog.size() * sizeof(int2), hipMemcpyHostToDevice,
-                           E->stream));
+    if (!blog.empty())
+        HIP_TRY(hipMemcpyAsync(E->dBoundaryMap, blog.data(), blog.size() * sizeof(int2), hipMemcpyHostToDevice,
+                               E->stream));
     // the host vectors end with this function
     HIP_TRY(hipStreamSynchronize(E->stream));
     return QM_OK;
@@ -166,7 +171,7 @@ template <typename R>
 static int enqueue_pass(qm_ensemble* E, int mode, int terms) {
     HIP_TRY(launch_march_segments<R>(E, mode, terms));
     HIP_TRY(launch_boundary_batch<R>(static_cast<const BoundaryArgs<R>*>(E->dBoundaryDescs), E->dBoundaryMap,
-                                     E->boundaryBlocks, mode, terms, E->stream));
+                                     E->boundaryBlocks, mode, terms, E->lanes, E->stream));
     if (mode == kFire)
         HIP_TRY(launch_fire_finalize_batch(E->dFinal, E->dStatus, (int)E->lats.size(), E->stream));
     return QM_OK;

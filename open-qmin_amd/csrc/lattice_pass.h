@@ -176,37 +176,41 @@ __device__ __forceinline__ void step_load(const StepArgs& S, long long n, long l
     }
 }
 
-// The update of site i from its force F and its entries pre (step_load):
-// energyMinimizerAdam::adamStepCPU (energyMinimizerAdam.cpp:25-54; epsilon
-// replaces sqrt(vc) where that is 0) or energyMinimizerNesterovAG::
-// nesterovStepCPU (energyMinimizerNesterovAG.cpp:75-92).  Stores the site's
-// advanced entries (no other work-item reads them in the pass) and returns the
-// new Q in qn.
+// The update of component j (of site or lattice index j) from its q, force and
+// entries (step_load): energyMinimizerAdam::adamStepCPU
+// (energyMinimizerAdam.cpp:25-54; epsilon replaces sqrt(vc) where that is 0) or
+// energyMinimizerNesterovAG::nesterovStepCPU (energyMinimizerNesterovAG.cpp:75-92).
+// Stores the advanced entries (no other work-item reads them in the pass) and
+// returns the new q.
+template <typename R, int MODE>
+__device__ __forceinline__ R step_component(const StepArgs& S, const StepCoef<R>& k, long long j, R q, R F, R m0,
+                                            R v0) {
+    R* m = static_cast<R*>(S.m);
+    if constexpr (MODE == kAdamStep) {
+        R* v = static_cast<R*>(S.v);
+        const R mm = k.b1 * m0 + k.b1m1 * F;
+        const R vv = k.b2 * v0 + k.omb2 * (F * F);
+        const R mc = mm * k.inv1;
+        const R vc = vv * k.inv2;
+        R root = sqrt(vc);
+        if (root == R(0)) root = k.eps;
+        st_out(&m[j], mm);
+        st_out(&v[j], vv);
+        return q + k.mdt * mc / root;
+    } else {
+        const R alt = q + k.dt * F;
+        st_out(&m[j], alt);
+        return alt + k.mu * (alt - m0);
+    }
+}
+
 template <typename R, int MODE>
 __device__ __forceinline__ void step_site(const StepArgs& S, const StepCoef<R>& k, long long n, long long i,
                                           const R* q, const R* F, const R (&pre)[2][5], R* qn) {
-    R* m = static_cast<R*>(S.m);
 #pragma unroll
-    for (int c = 0; c < 5; ++c) {
-        const long long j = c * n + i;
-        if constexpr (MODE == kAdamStep) {
-            R* v = static_cast<R*>(S.v);
-            const R mm = k.b1 * pre[0][c] + k.b1m1 * F[c];
-            const R vv = k.b2 * pre[1][c] + k.omb2 * (F[c] * F[c]);
-            const R mc = mm * k.inv1;
-            const R vc = vv * k.inv2;
-            R root = sqrt(vc);
-            if (root == R(0)) root = k.eps;
-            st_out(&m[j], mm);
-            st_out(&v[j], vv);
-            qn[c] = q[c] + k.mdt * mc / root;
-        } else {
-            const R old = pre[0][c];
-            const R alt = q[c] + k.dt * F[c];
-            st_out(&m[j], alt);
-            qn[c] = alt + k.mu * (alt - old);
-        }
-    }
+    for (int c = 0; c < 5; ++c)
+        qn[c] = step_component<R, MODE>(S, k, c * n + i, q[c], F[c], pre[0][c],
+                                        MODE == kAdamStep ? pre[1][c] : R(0));
 }
 
 // Sum of squares of the five stored components (the minimizers' |F|^2).
@@ -771,9 +775,10 @@ __device__ __forceinline__ void gload(const R* base, long long n, long long i, R
     for (int c = 0; c < 5; ++c) v[c] = base[c * n + i];
 }
 
-// Work-group `blk` of the boundary pass of the lattice described by A.
+// Work-group `blk` of the boundary pass of the lattice described by A, one lane
+// per site: the stencils of many sites (boundary_lanes has the rule).
 template <typename R, int MODE, int TERMS>
-__device__ __forceinline__ void boundary_body(const BoundaryArgs<R>& A, const int blk) {
+__device__ __forceinline__ void boundary_site_body(const BoundaryArgs<R>& A, const int blk) {
     __shared__ double sRed[kBoundaryThreads / 64][3];
     Ctrl* ctrl = A.ctrl;
     if ((MODE != kForce || A.gate) && ctrl->done) return;
@@ -955,17 +960,232 @@ __device__ __forceinline__ void boundary_body(const BoundaryArgs<R>& A, const in
     }
 }
 
+// The same for few sites: eight lanes evaluate one site.  Lane d < 6 loads the neighbour in direction d (x-,
+// x+, y-, y+, z-, z+) and the four sites beside it that its transverse
+// derivatives need, takes its share of the L1 term and, if the neighbour is an
+// object, the anchoring on it; then all lanes take turns at the terms of the
+// site's stencil, whose inputs the six have put in LDS, and their sums are added.
+//
+// The pass is bound by the length of one wave's path, not by throughput: one
+// lane per site loaded 155 values and ran through up to 27 straight-line
+// stencils (80 KB of code in FP64).  50^3 with walls and a sphere, L1..L3, FP64:
+// 8 against 24 us; four spheres with L1..L6 17 against 54 us.
 template <typename R, int MODE, int TERMS>
-__global__ void __launch_bounds__(kBoundaryThreads) boundary_kernel(BoundaryArgs<R> A) {
-    boundary_body<R, MODE, TERMS>(A, blockIdx.x);
+__device__ __forceinline__ void boundary_lanes_body(const BoundaryArgs<R>& A, const int blk) {
+    constexpr bool kMulti = TERMS != kOneConstant;
+    constexpr int kOne = 125, kRow = kMulti ? 127 : 1;   // inputs of a site in LDS, odd row length
+    __shared__ R sx[kBoundaryGroup][kRow];
+    __shared__ double sRed[kBoundaryThreads / 64][3];
+    Ctrl* ctrl = A.ctrl;
+    if ((MODE != kForce || A.gate) && ctrl->done) return;
+    const int cur = ctrl->cur;
+    // FIRE: the drifted state the fused pass has written; otherwise the current one
+    const StateSet<R> st = A.set[MODE == kFire ? cur ^ 1 : cur];
+    const R hdt = MODE == kFire ? R(0.5 * ctrl->dt) : R(0);
+    StepCoef<R> sk{};
+    if constexpr (is_step_mode(MODE)) sk = step_coef<R, MODE>(A.step);
+    const long long n = A.n;
+    const int lx = A.lx, ly = A.ly, lz = A.lz;
+    // a wave takes eight consecutive entries of the site list, whose lanes of one
+    // direction are neighbours: where the sites are, their loads share lines
+    constexpr int kPer = 64 / kBoundaryLanes;
+    const int d = (threadIdx.x & 63) / kPer, g = (threadIdx.x >> 6) * kPer + threadIdx.x % kPer;
+    const int axis = d >> 1;
+    // index offset to the next site up or down an axis of m sites from coordinate v
+    auto step = [](int v, int m, int stride, bool up) {
+        return up ? (v == m - 1 ? -(m - 1) * stride : stride) : (v == 0 ? (m - 1) * stride : -stride);
+    };
+    double pF = 0, pP = 0, pV = 0;
+
+    {
+        const long long k = (long long)blk * kBoundaryGroup + g;
+        const bool have = k < A.nsites;
+        const int i = A.sites[have ? k : A.nsites - 1];   // site indices fit 31 bits
+        const int self = A.types[i];
+        const unsigned row = unsigned(i) / unsigned(lx);
+        const int x = i - int(row) * lx, z = int(row / unsigned(ly)), y = int(row) - z * ly;
+        // the entries that lane d < 5 finishes component d with
+        const long long own = (d < 5 ? d : 0) * n + i;
+        R pre0 = R(0), pre1 = R(0);
+        if constexpr (MODE == kFire) pre0 = st.u[own];
+        if constexpr (is_step_mode(MODE)) pre0 = static_cast<const R*>(A.step.m)[own];
+        if constexpr (MODE == kAdamStep) pre1 = static_cast<const R*>(A.step.v)[own];
+        R q[5], nq[5];
+        gload(st.q, n, i, q);
+        int tn = 0;
+        if (d < 6) {
+            // coordinate, length and stride of the neighbour's axis and of the two others
+            const int v0 = axis == 0 ? x : (axis == 1 ? y : z), m0 = axis == 0 ? lx : (axis == 1 ? ly : lz);
+            const int plane = lx * ly;
+            const int nb = i + step(v0, m0, axis == 0 ? 1 : (axis == 1 ? lx : plane), d & 1);
+            tn = A.types[nb];
+            gload(st.q, n, nb, nq);
+            if constexpr (kMulti) {
+                int tu[2], td[2];
+                R qu[2][5], qd[2][5];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const int ax = axis + 1 + t >= 3 ? axis - 2 + t : axis + 1 + t;
+                    const int v = ax == 0 ? x : (ax == 1 ? y : z), m = ax == 0 ? lx : (ax == 1 ? ly : lz),
+                              stride = ax == 0 ? 1 : (ax == 1 ? lx : plane);
+                    const int iu = nb + step(v, m, stride, true), id = nb + step(v, m, stride, false);
+                    tu[t] = A.types[iu];
+                    td[t] = A.types[id];
+                    gload(st.q, n, iu, qu[t]);
+                    gload(st.q, n, id, qd[t]);
+                }
+#pragma unroll
+                for (int c = 0; c < 5; ++c) sx[g][5 + 5 * d + c] = nq[c];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const int ax = axis + 1 + t >= 3 ? axis - 2 + t : axis + 1 + t;
+                    R out[5];
+                    nbr_derivative(tn, tu[t], td[t], nq, qu[t], qd[t], out);
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) sx[g][35 + 15 * d + 5 * ax + c] = out[c];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) nq[c] = q[c];
+            if constexpr (kMulti) {
+                if (d == 6) {
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) sx[g][c] = q[c];
+                } else {
+                    sx[g][kOne] = R(1);
+                }
+            }
+        }
+        // which neighbours are objects, bit d per direction
+        const unsigned long long facing = __ballot(d < 6 && tn > 0) >> (threadIdx.x % kPer);
+        unsigned faces = 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) faces |= unsigned(facing >> (kPer * k) & 1) << k;
+        // this lane's share of what is added to the phase force.  L1: the bulk
+        // Laplacian, or next to an object (boundaryL1Force, lcForces.h:39-63) only
+        // the neighbours opposite to one
+        R P[5];
+        const bool l1 = d < 6 && (self == -1 ? (faces >> (d ^ 1)) & 1 : true);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) P[c] = l1 ? R(A.fc.L1) * (nq[c] - q[c]) : R(0);
+        l1_shape(P);
+        if (self == -1 && tn > 0) add_anchoring_force(A.objects[tn - 1], q, nq, P);
+        if constexpr (kMulti) {
+            // boundary case: an object above (1) or below (2, taking precedence) on
+            // each axis (lcForces.h:13-25)
+            const int ox = (faces & 1) ? 2 : (faces >> 1) & 1, oy = (faces & 4) ? 2 : (faces >> 3) & 1,
+                      oz = (faces & 16) ? 2 : (faces >> 5) & 1;
+            const int bcase = self == -1 ? ox + 3 * oy + 9 * oz : 0;
+            __syncthreads();
+            auto terms = [&](const BoundaryTerm<R>* t, int rounds) {
+                t += bcase * 5 * rounds * kBoundaryLanes + d;
+#pragma unroll 4
+                for (int r = 0; r < rounds; ++r)
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) {
+                        const BoundaryTerm<R> e = t[(c * rounds + r) * kBoundaryLanes];
+                        P[c] -= e.coef * (sx[g][e.ab & 255] * sx[g][e.ab >> 8]);
+                    }
+            };
+            terms(A.terms, kBoundaryLinRounds);
+            if constexpr (TERMS == kMultiL6)
+                terms(A.terms + kBoundaryCases * 5 * kBoundaryLinRounds * kBoundaryLanes, kBoundaryQuadRounds);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int o = kPer; o < 64; o <<= 1)
+#pragma unroll
+            for (int c = 0; c < 5; ++c) P[c] += __shfl_xor(P[c], o, 64);
+        R F[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) F[c] = R(0);
+        phase_force(R(A.fc.a), R(A.fc.b), R(A.fc.c), q, F);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) F[c] += P[c];
+        R fv[5] = {R(0), R(0), R(0), R(0), R(0)};
+        if (A.hvar) varying_field_force(A.hvar, n, i, A.hvarP, fv);
+        // a bulk site with a one-sided neighbour derivative has bulk semantics
+        if (self == 0 && A.fc.semantics == 0) metric(F);
+        if (A.fc.hasField) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) F[c] += R(A.fc.field[c]);
+        }
+        if (A.hvar) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) F[c] += fv[c];
+        }
+        metric(F);
+        R Fd = F[0], qd = q[0];
+#pragma unroll
+        for (int c = 1; c < 5; ++c) {
+            Fd = d == c ? F[c] : Fd;
+            qd = d == c ? q[c] : qd;
+        }
+        const bool put = have && d < 5;
+        if (MODE == kFire) {
+            const R ud = pre0 + hdt * Fd;
+            const R u0 = __shfl(ud, threadIdx.x % kPer, 64);   // component 0's, for the QT products' F_0 u_3 and u_0 u_3
+            if (put) {
+                st.u[own] = ud;
+                st.f[own] = Fd;
+                const double f = double(Fd), u = double(ud);
+                pF += f * f + (d == 3 ? double(F[0]) * f : 0.0);
+                pP += f * u + (d == 3 ? double(F[0]) * u : 0.0);
+                pV += u * u + (d == 3 ? double(u0) * u : 0.0);
+            }
+        } else if constexpr (is_step_mode(MODE)) {
+            if (put) {
+                const StateSet<R> out = A.set[cur ^ 1];
+                out.q[own] = step_component<R, MODE>(A.step, sk, own, qd, Fd, pre0, pre1);
+                out.f[own] = Fd;
+                pF += double(Fd) * double(Fd);
+            }
+        } else {
+            if (put) st.f[own] = Fd;
+        }
+    }
+    if (MODE == kForce) return;
+    block_sum3<kBoundaryThreads>(pF, pP, pV, sRed);
+    if (threadIdx.x == 0) {
+        const long long slot = A.marchBlocks + blk;
+        A.partials[3 * slot + 0] = pF;
+        A.partials[3 * slot + 1] = pP;
+        A.partials[3 * slot + 2] = pV;
+    }
 }
 
-template <typename R, int MODE, int TERMS>
+template <typename R, int MODE, int TERMS, bool LANES>
+__device__ __forceinline__ void boundary_body(const BoundaryArgs<R>& A, const int blk) {
+    if constexpr (LANES)
+        boundary_lanes_body<R, MODE, TERMS>(A, blk);
+    else
+        boundary_site_body<R, MODE, TERMS>(A, blk);
+}
+
+template <typename R, int MODE, int TERMS, bool LANES>
+__global__ void __launch_bounds__(kBoundaryThreads) boundary_kernel(BoundaryArgs<R> A) {
+    boundary_body<R, MODE, TERMS, LANES>(A, blockIdx.x);
+}
+
+template <typename R, int MODE, int TERMS, bool LANES>
 __global__ void __launch_bounds__(kBoundaryThreads) boundary_batch_kernel(
     const BoundaryArgs<R>* __restrict__ descs, const int2* __restrict__ map) {
     const int lat = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
     const int blk = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
-    boundary_body<R, MODE, TERMS>(descs[lat], blk);
+    boundary_body<R, MODE, TERMS, LANES>(descs[lat], blk);
+}
+
+// The kernels of a force's stencil variant; neither pass distinguishes L1..L3
+// from L1..L4, and the one-constant pass always takes the lanes.
+template <typename R, int MODE>
+const void* boundary_fn(int terms, bool lanes) {
+    if (terms == kOneConstant) return reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kOneConstant, true>);
+    if (terms == kMultiL6)
+        return lanes ? reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiL6, true>)
+                     : reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiL6, false>);
+    return lanes ? reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiLinear, true>)
+                 : reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiLinear, false>);
 }
 
 }  // namespace qmin

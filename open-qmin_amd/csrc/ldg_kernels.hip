@@ -382,11 +382,6 @@ static const void* march_fn(int mode, int terms, int tile) {
 }
 
 template <typename R, int MODE, int TERMS>
-static void launch_boundary_t(const BoundaryArgs<R>& a, int blocks, hipStream_t s) {
-    hipLaunchKernelGGL((boundary_kernel<R, MODE, TERMS>), dim3(blocks), dim3(kBoundaryThreads), 0, s, a);
-}
-
-template <typename R, int MODE, int TERMS>
 static const void* march_batch_fn_tile(int tile) {
     switch (tile) {
         case kTile64x4: return reinterpret_cast<const void*>(&march_batch_kernel<R, MODE, TERMS, kTile64x4>);
@@ -415,18 +410,21 @@ hipError_t launch_march_batch(const MarchArgs<R>* descs, const int2* map, int bl
     return hipLaunchKernel(fn, dim3(blocks), dim3(kTileThreads[tile]), args, 0, s);
 }
 
+template <typename R, int MODE>
+static const void* boundary_batch_fn(int terms, bool lanes) {
+    if (terms == kOneConstant) return reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kOneConstant, true>);
+    if (terms == kMultiL6)
+        return lanes ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiL6, true>)
+                     : reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiL6, false>);
+    return lanes ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiLinear, true>)
+                 : reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiLinear, false>);
+}
+
 template <typename R>
 hipError_t launch_boundary_batch(const BoundaryArgs<R>* descs, const int2* map, int blocks, int mode, int terms,
-                                 hipStream_t s) {
-    const void* fn;
-    if (mode == kFire)
-        fn = terms == kOneConstant ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, kFire, kOneConstant>)
-           : terms == kMultiL6     ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, kFire, kMultiL6>)
-                                   : reinterpret_cast<const void*>(&boundary_batch_kernel<R, kFire, kMultiLinear>);
-    else
-        fn = terms == kOneConstant ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, kForce, kOneConstant>)
-           : terms == kMultiL6     ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, kForce, kMultiL6>)
-                                   : reinterpret_cast<const void*>(&boundary_batch_kernel<R, kForce, kMultiLinear>);
+                                 bool lanes, hipStream_t s) {
+    if (blocks == 0) return hipSuccess;
+    const void* fn = mode == kFire ? boundary_batch_fn<R, kFire>(terms, lanes) : boundary_batch_fn<R, kForce>(terms, lanes);
     void* args[] = {&descs, &map};
     return hipLaunchKernel(fn, dim3(blocks), dim3(kBoundaryThreads), args, 0, s);
 }
@@ -444,19 +442,12 @@ hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hi
 
 template <typename R>
 void launch_boundary(const BoundaryArgs<R>& a, int mode, int terms, hipStream_t s) {
-    long long blocks = (a.nsites + kBoundaryThreads - 1) / kBoundaryThreads;
-    if (blocks < 1) blocks = 1;
-    // the boundary pass does not distinguish L1..L3 from L1..L4
-    if (mode == kFire) {
-        if (terms == kOneConstant) launch_boundary_t<R, kFire, kOneConstant>(a, int(blocks), s);
-        else if (terms == kMultiL6) launch_boundary_t<R, kFire, kMultiL6>(a, int(blocks), s);
-        else launch_boundary_t<R, kFire, kMultiLinear>(a, int(blocks), s);
-    } else {
-        if (a.nsites == 0) return;
-        if (terms == kOneConstant) launch_boundary_t<R, kForce, kOneConstant>(a, int(blocks), s);
-        else if (terms == kMultiL6) launch_boundary_t<R, kForce, kMultiL6>(a, int(blocks), s);
-        else launch_boundary_t<R, kForce, kMultiLinear>(a, int(blocks), s);
-    }
+    const bool lanes = boundary_lanes(terms, a.nsites);
+    const int blocks = boundary_blocks(a.nsites, lanes);
+    if (blocks == 0) return;
+    const void* fn = mode == kFire ? boundary_fn<R, kFire>(terms, lanes) : boundary_fn<R, kForce>(terms, lanes);
+    void* args[] = {const_cast<BoundaryArgs<R>*>(&a)};
+    (void)hipLaunchKernel(fn, dim3(blocks), dim3(kBoundaryThreads), args, 0, s);   // the caller reads the error
 }
 
 template <typename R>
@@ -488,11 +479,6 @@ int march_blocks_per_cu(int mode, int terms, int tile) {
 void launch_fire_finalize(Ctrl* ctrl, const FireConst& fp, const double* partials, long long total, double* trace,
                           hipStream_t s) {
     hipLaunchKernelGGL(fire_finalize_kernel, dim3(1), dim3(kReduceThreads), 0, s, ctrl, fp, partials, total, trace);
-}
-
-int boundary_blocks(long long nsites) {
-    long long b = (nsites + kBoundaryThreads - 1) / kBoundaryThreads;
-    return b < 1 ? 1 : int(b);
 }
 
 template <typename R>
@@ -541,7 +527,7 @@ void launch_defects(const R* q, const SiteType* types, long long n, int kind, do
                                            const EnergyConst&, double*, hipStream_t);                            \
     template int march_blocks_per_cu<R>(int, int, int);                                                          \
     template hipError_t launch_march_batch<R>(const MarchArgs<R>*, const int2*, int, int, int, int, hipStream_t);  \
-    template hipError_t launch_boundary_batch<R>(const BoundaryArgs<R>*, const int2*, int, int, int, hipStream_t);  \
+    template hipError_t launch_boundary_batch<R>(const BoundaryArgs<R>*, const int2*, int, int, int, bool, hipStream_t);  \
     template void launch_object_force<R>(const R*, const SiteType*, const DevObject*, int, int, int, const EnergyConst&, \
                                          double, const int64_t*, long long, double*, hipStream_t);                 \
     template void launch_move_q<R>(R*, long long, const int64_t*, const int64_t*, long long, R*, hipStream_t);

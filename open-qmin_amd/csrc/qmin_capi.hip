@@ -21,11 +21,30 @@
 #include "gen/ldg_fast_host.inc"
 
 namespace qmin {
+#include "gen/ldg_boundary_tables.inc"
+
+constexpr int kBoundaryLinTerms = int(sizeof(kBoundaryLin) / sizeof(kBoundaryLin[0]));
+constexpr int kBoundaryQuadTerms = int(sizeof(kBoundaryQuad) / sizeof(kBoundaryQuad[0]));
+
+// Boundary stencils for a force's constants (boundary_body).
+template <typename R>
+__global__ void compose_boundary_kernel(double L2, double L3, double L4, double L6, BoundaryTerm<R>* out) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < kBoundaryLinTerms) {
+        const BoundaryLinTerm t = kBoundaryLin[k];
+        out[k] = {R(L2 * t.c2 + L3 * t.c3 + L4 * t.c4), t.a + 256 * t.b};
+    } else if (k < kBoundaryLinTerms + kBoundaryQuadTerms) {
+        const BoundaryQuadTerm t = kBoundaryQuad[k - kBoundaryLinTerms];
+        out[k] = {R(L6 * t.c6), t.a + 256 * t.b};
+    }
+}
+}  // namespace qmin
+
+namespace qmin {
 template <typename R>
 hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hipStream_t s);
 template <typename R>
 void launch_boundary(const BoundaryArgs<R>& a, int mode, int terms, hipStream_t s);
-int boundary_blocks(long long nsites);
 void launch_fire_finalize(Ctrl* ctrl, const FireConst& fp, const double* partials, long long total, double* trace,
                           hipStream_t s);
 template <typename R>
@@ -259,6 +278,7 @@ int qm_lattice_create(int lx, int ly, int lz, int precision, qm_lattice** out) {
     HIP_TRY(hipMalloc(&L->dTypes, n * sizeof(SiteType)));
     HIP_TRY(hipMalloc(&L->dClass, n));
     HIP_TRY(hipMalloc(&L->dW, sizeof(double) * 2 * kFastWeights));
+    HIP_TRY(hipMalloc(&L->dTerms, sizeof(BoundaryTerm<double>) * (kBoundaryLinTerms + kBoundaryQuadTerms)));
     HIP_TRY(hipMalloc(&L->dObjects, sizeof(DevObject) * kMaxObjects));
     for (int s = 0; s < 2; ++s) {
         HIP_TRY(hipMalloc(&L->dSet[s], 15 * n * L->realSize));
@@ -279,6 +299,7 @@ int qm_lattice_destroy(qm_lattice* L) {
     (void)hipFree(L->dTypes);
     (void)hipFree(L->dClass);
     (void)hipFree(L->dW);
+    (void)hipFree(L->dTerms);
     (void)hipFree(L->dObjects);
     (void)hipFree(L->dSet[0]);
     (void)hipFree(L->dSet[1]);
@@ -965,16 +986,30 @@ static void weight_buffer(const qm_ldg* f, R* w) {
     }
 }
 
-static int upload_weights(qm_lattice* L, const qm_ldg* f) {
-    if (L->precision == QM_FP64) {
-        double w[2 * kFastWeights];
-        weight_buffer<double>(f, w);
-        HIP_TRY(copy_on(L, L->dW, w, sizeof(w), hipMemcpyHostToDevice));
-    } else {
-        float w[2 * kFastWeights];
-        weight_buffer<float>(f, w);
-        HIP_TRY(copy_on(L, L->dW, w, sizeof(w), hipMemcpyHostToDevice));
+// Composes the operators of the passes for the force's constants, unless the
+// lattice holds those of the same constants already.
+template <typename R>
+static int compose(qm_lattice* L, const qm_ldg* f) {
+    R w[2 * kFastWeights];
+    weight_buffer<R>(f, w);
+    HIP_TRY(copy_on(L, L->dW, w, sizeof(w), hipMemcpyHostToDevice));
+    if (f->multi) {
+        constexpr int kTerms = kBoundaryLinTerms + kBoundaryQuadTerms;
+        compose_boundary_kernel<R><<<(kTerms + 255) / 256, 256, 0, L->stream>>>(
+            f->L2, f->L3, f->L4, f->L6, static_cast<BoundaryTerm<R>*>(L->dTerms));
+        HIP_TRY(hipGetLastError());
     }
+    return QM_OK;
+}
+
+static int upload_weights(qm_lattice* L, const qm_ldg* f) {
+    const double want[7] = {f->L1, f->L2, f->L3, f->L4, f->L6, (double)terms_of(f), (double)L->precision};
+    bool same = true;
+    for (int k = 0; k < 7; ++k) same = same && want[k] == L->composed[k];
+    if (same) return QM_OK;
+    for (double& v : L->composed) v = NAN;
+    if (int rc = L->precision == QM_FP64 ? compose<double>(L, f) : compose<float>(L, f)) return rc;
+    std::copy(want, want + 7, L->composed);
     return QM_OK;
 }
 
@@ -1054,6 +1089,7 @@ void qmin::fill_args(qm_lattice* L, const qm_ldg* f, MarchArgs<R>& ma, BoundaryA
     ba.objects = L->dObjects;
     ba.sites = L->dSites;
     ba.nsites = L->nBoundary;
+    ba.terms = static_cast<const BoundaryTerm<R>*>(L->dTerms);
     ba.lx = L->lx;
     ba.ly = L->ly;
     ba.lz = L->lz;
@@ -1151,7 +1187,7 @@ static int run_pass(qm_lattice* L, const qm_ldg* f, int mode, const FireConst& f
     launch_boundary<R>(ba, mode, terms, L->stream);
     HIP_TRY(hipGetLastError());
     if (mode == kFire) {
-        launch_fire_finalize(L->dCtrl, fire, ma.partials, (long long)ma.nblocks + boundary_blocks(L->nBoundary),
+        launch_fire_finalize(L->dCtrl, fire, ma.partials, (long long)ma.nblocks + boundary_slots(L),
                              L->dTrace, L->stream);
         HIP_TRY(hipGetLastError());
     }
@@ -1265,7 +1301,7 @@ int qmin::prepare(qm_lattice* L, const qm_ldg* f) {
     for (int t = 0; t < kNumTiles; ++t) worst = std::max(worst, tile_columns(L, t) * ((L->lz + 3) / 4));
     if (takes_blocks(L, kFire) || takes_blocks(L, kForce))
         worst = std::max(worst, tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ));
-    const size_t need = 3 * (size_t)(worst + boundary_blocks(L->nBoundary));
+    const size_t need = 3 * (size_t)(worst + boundary_slots(L));
     return ensure_partials(L, need);
 }
 
@@ -1287,7 +1323,7 @@ static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs&
     ma.step = step;
     ba.step = step;
     HIP_TRY(launch_step<R>(ma, ba, mode, terms_of(f), tile, L->stream));
-    *slots = (long long)ma.nblocks + boundary_blocks(L->nBoundary);
+    *slots = (long long)ma.nblocks + boundary_slots(L);
     return QM_OK;
 }
 
@@ -1545,9 +1581,11 @@ FireConst qmin::fire_const(const qm_fire* m, const qm_lattice* L) {
 // library runs on holds its own copy until the process ends.  Every slot a pass
 // reads is written by that pass first, so nothing has to start at zero; calls
 // that overlap on one GPU share the array and race.
-constexpr long long kScratchSlots = 65536;   // partial-sum slots of 3 doubles: 1.5 MiB
+constexpr long long kScratchSlots = 65536;   // partial-sum slots of 3 doubles: 1.5 MiB, a boundary pass
+constexpr long long kScratchSites = 128;     // counted with one slot per 128 sites; where its work-groups take
+constexpr long long kScratchMore = 1 << 17;  // fewer, they have room of their own
 constexpr int kScratchDevices = 64;
-static __device__ __align__(256) double scratch[3 * kScratchSlots];
+static __device__ __align__(256) double scratch[3 * (kScratchSlots + kScratchMore)];
 static std::mutex g_scratchMutex;
 static double* g_scratchPtr[kScratchDevices] = {};
 
@@ -1582,9 +1620,11 @@ static int prepare_noalloc(qm_lattice* L, const qm_ldg* f, double** partials) {
     long long need = 0;
     for (int mode : {kForce, kFire}) {
         choose_zchunk(L, mode, L->terms);
-        need = std::max(need, (long long)march_blocks(L, mode) + boundary_blocks(L->nBoundary));
+        const long long boundary = std::max(1LL, (L->nBoundary + kScratchSites - 1) / kScratchSites);
+        need = std::max(need, march_blocks(L, mode) + boundary);
     }
-    if (need > kScratchSlots)
+    const long long slots = need + boundary_slots(L);
+    if (need > kScratchSlots || slots > kScratchSlots + kScratchMore)
         return fail(QM_EINVAL, "the lattice needs " + std::to_string(need) + " partial-sum slots; the "
                                "allocation-free call holds at most " + std::to_string(kScratchSlots));
     if (int rc = upload_weights(L, f)) return rc;

@@ -88,6 +88,48 @@ struct Tile {
 using SiteType = int16_t;                // site types on the device (reference encoding)
 constexpr int kMaxObjects = 32767;      // object ids a SiteType holds
 constexpr int kBoundaryThreads = 128;
+constexpr int kBoundaryLanes = 8;   // lanes that evaluate one site together, where the pass does so
+constexpr int kBoundaryGroup = kBoundaryThreads / kBoundaryLanes;   // sites of such a work-group
+constexpr int kBoundaryCases = 27;
+
+// Whether the boundary pass gives a site eight lanes (boundary_lanes_body) or one
+// (boundary_site_body).  FIRE iterations with lanes and with one lane per site
+// (us, FP64 unless noted): L1..L3 50^3, 6,500 sites, 27 and 40; 96^3, 23,000
+// sites, 78 and 83; L1..L6 144 x 128 x 100, 38,000 sites, 167 and 176; L1..L3
+// Nesterov 192 x 150 x 130, 60,000 sites, 196 and 187; FP32 203 x 176 x 161,
+// 73,000 sites, 332 and 322; 256^3, 135,000 sites, 903 and 866: there the
+// loads, which eight lanes scatter over more lines, set the pace.  The
+// one-constant pass loads little and is never slower with lanes.
+constexpr long long kLanesSites = 40960;
+__host__ __device__ inline bool boundary_lanes(int terms, long long nsites) {
+    return terms == 0 || nsites <= kLanesSites;
+}
+// work-groups of the boundary pass over nsites sites
+__host__ __device__ inline int boundary_blocks(long long nsites, bool lanes) {
+    const int per = lanes ? kBoundaryGroup : kBoundaryThreads;
+    return int((nsites + per - 1) / per);
+}
+
+// One term of a boundary stencil, at unit constants: coefficient(s) and the
+// inputs multiplied (the 125 of a site, then the constant 1).
+struct BoundaryLinTerm {
+    double c2, c3, c4;
+    short a, b;
+};
+struct BoundaryQuadTerm {
+    double c6;
+    short a, b;
+};
+
+// The same composed for a force's constants in the lattice's precision, as the
+// boundary pass reads it: [case][component][round][lane], the terms of L2..L4
+// first, those of L6 behind them.
+template <typename R>
+struct BoundaryTerm {
+    R coef;
+    int ab;   // a + 256 b
+};
+
 constexpr int kReduceThreads = 256;
 constexpr int kMaxEnergyBlocks = 4096;
 constexpr int kFastWeights = 160;  // >= entries of the composed L1..L4 operator
@@ -195,6 +237,7 @@ struct BoundaryArgs {
     long long nsites;
     int lx, ly, lz;
     long long n;
+    const BoundaryTerm<R>* terms;   // stencils of the 27 cases for the force's constants
     int marchBlocks;        // partial slots used by the fused pass
     ForceConst fc;
     FireConst fire;

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -36,6 +37,10 @@ struct qm_lattice {
     qmin::SiteType* dTypes = nullptr;
     int8_t* dClass = nullptr;             // 0 composed bulk formula, > 0 object, < 0 boundary pass
     void* dW = nullptr;                   // composed bulk operator weights (Real)
+    void* dTerms = nullptr;               // composed boundary stencils (BoundaryTerm<Real>)
+    // the constants dW and dTerms were composed for: L1, L2, L3, L4, L6, the
+    // stencil variant and the precision (NaN: none yet)
+    double composed[7] = {NAN, NAN, NAN, NAN, NAN, NAN, NAN};
     DevObject* dObjects = nullptr;
     void* dSet[2] = {nullptr, nullptr};   // each 15 n reals: Q, U, F planes
     int32_t* dSites = nullptr;            // compacted sites finished by the boundary pass
@@ -118,7 +123,10 @@ template <typename R>
 void fill_args(qm_lattice* L, const qm_ldg* f, MarchArgs<R>& ma, BoundaryArgs<R>& ba, const FireConst& fire,
                int tile, bool narrow = false);
 FireConst fire_const(const qm_fire* m, const qm_lattice* L);
-int boundary_blocks(long long nsites);
+// work-groups of a lattice's boundary pass
+inline int boundary_slots(const qm_lattice* L) {
+    return boundary_blocks(L->nBoundary, boundary_lanes(L->terms, L->nBoundary));
+}
 template <typename R>
 inline StateSet<R> state_set(const qm_lattice* L, int s) {
     R* base = static_cast<R*>(L->dSet[s]);

@@ -32,14 +32,6 @@ const void* step_fn_terms(int terms, int tile) {
     }
 }
 
-// the boundary pass does not distinguish L1..L3 from L1..L4
-template <typename R, int MODE>
-const void* step_boundary_fn(int terms) {
-    if (terms == kOneConstant) return reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kOneConstant>);
-    if (terms == kMultiL6) return reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiL6>);
-    return reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiLinear>);
-}
-
 }  // namespace
 
 // Queues the fused pass (tile `tile`, one of the halo-padded ones or kBlock) and
@@ -54,9 +46,10 @@ hipError_t launch_step(const MarchArgs<R>& ma, const BoundaryArgs<R>& ba, int mo
     void* margs[] = {const_cast<MarchArgs<R>*>(&ma)};
     hipError_t e = hipLaunchKernel(fn, dim3(ma.nblocks), dim3(tile_threads(tile)), margs, 0, s);
     if (e != hipSuccess) return e;
-    long long blocks = (ba.nsites + kBoundaryThreads - 1) / kBoundaryThreads;
-    if (blocks < 1) blocks = 1;
-    const void* bfn = mode == kAdamStep ? step_boundary_fn<R, kAdamStep>(terms) : step_boundary_fn<R, kNesterovStep>(terms);
+    const bool lanes = boundary_lanes(terms, ba.nsites);
+    const int blocks = boundary_blocks(ba.nsites, lanes);
+    if (blocks == 0) return hipGetLastError();
+    const void* bfn = mode == kAdamStep ? boundary_fn<R, kAdamStep>(terms, lanes) : boundary_fn<R, kNesterovStep>(terms, lanes);
     void* bargs[] = {const_cast<BoundaryArgs<R>*>(&ba)};
     e = hipLaunchKernel(bfn, dim3((unsigned)blocks), dim3(kBoundaryThreads), bargs, 0, s);
     if (e != hipSuccess) return e;

@@ -12,10 +12,14 @@ Output: ../csrc/gen/ldg_stencils.inc with
   ldg_boundary_l6(bcase, x, out)          the 27 boundary-case L6 forms
 
 acc[t][c] accumulates term t (0 = L2, 1 = L3, 2 = L4) of component c at unit
-constant; the caller scales by L.
+constant; the caller scales by L.  ../csrc/gen/ldg_boundary_tables.inc has the
+same forms as tables: per case and component the entries over the inputs, padded
+to whole rounds of eight (the lanes that evaluate a site together), with the
+coefficients of L2, L3 and L4 (kBoundaryLin) or of L6 (kBoundaryQuad; a product
+of two inputs, a second input of 125 standing for the constant 1).
 
-It also composes, for a site whose neighbours all have central derivatives,
-the bulk L1 (shaped Laplacian), L2, L3 and L4 forms with those central
+ldg_stencils.inc also composes, for a site whose neighbours all have central
+derivatives, the bulk L1 (shaped Laplacian), L2, L3 and L4 forms with those central
 differences into one linear operator on the 19-point neighbourhood (centre,
 6 faces, 12 edges).  Its weights are L1 C1 + L2 C2 + L3 C3 + L4 C4 per entry:
 
@@ -39,6 +43,9 @@ import os
 HERE = os.path.dirname(os.path.abspath(__file__))
 TABLES = os.path.join(HERE, "ldg_stencil_tables.json")
 OUT = os.path.join(os.path.dirname(HERE), "csrc", "gen", "ldg_stencils.inc")
+BOUNDARY_OUT = os.path.join(os.path.dirname(OUT), "ldg_boundary_tables.inc")
+LANES = 8    # lanes that evaluate one boundary site together
+ONE = 125    # input index of the constant 1
 LIN_TERMS = ("L2", "L3", "L4")
 
 
@@ -88,6 +95,33 @@ def gen_boundary(tables, cases):
         l6.append("    }")
     l6 += ["    default: for (int i = 0; i < 5; ++i) out[i] = R(0); break;", "    }", "}"]
     return lines + l6
+
+
+def gen_boundary_tables(tables, cases):
+    """Tables of the boundary forms, rows [case][component][round][lane], and the
+    lines that say how many rounds they have."""
+    lin, quad = [], []
+    for c in cases:
+        for r in range(5):
+            coefs = {}
+            for t, name in enumerate(LIN_TERMS):
+                for e in tables[name][str(c)]:
+                    if e[0] == r:
+                        coefs.setdefault(e[2], [0.0, 0.0, 0.0])[t] += e[1]
+            lin.append([(k, ONE) + tuple(v) for k, v in sorted(coefs.items())])
+            quad.append([(e[2], e[3], e[1]) for e in tables["L6"][str(c)] if e[0] == r])
+    assert cases == [x + 4 * y + 16 * z for z in range(3) for y in range(3) for x in range(3)]
+    lines, counts = [], []
+    for name, rows, width in (("Lin", lin, 3), ("Quad", quad, 1)):
+        rounds = max((len(row) + LANES - 1) // LANES for row in rows)
+        flat = [e for row in rows for e in row + [(ONE, ONE) + (0.0,) * width] * (rounds * LANES - len(row))]
+        counts.append("constexpr int kBoundary%sRounds = %d;" % (name, rounds))
+        lines += ["static __device__ const Boundary%sTerm kBoundary%s[%d] = {" % (name, name, len(flat))]
+        for k in range(0, len(flat), 4):
+            lines.append("    " + " ".join("{%s, %d, %d}," % (", ".join(repr(float(v)) for v in e[2:]), e[0], e[1])
+                                           for e in flat[k:k + 4]))
+        lines.append("};")
+    return lines, counts
 
 
 POINTS = [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
@@ -379,7 +413,13 @@ def main():
     tables, cases = doc["tables"], doc["cases"]
     body = ["// Generated by open-qmin_amd/stencils/gen_stencils.py from ldg_stencil_tables.json.",
             "// Do not edit by hand.", "#pragma once", ""]
+    boundary, counts = gen_boundary_tables(tables, cases)
+    boundary_text = "\n".join(body[:2] + boundary) + "\n"
+    body += ["// rounds of eight terms per component of the boundary tables"] + counts + [""]
     body += gen_boundary(tables, cases)
+    if not os.path.exists(BOUNDARY_OUT) or open(BOUNDARY_OUT).read() != boundary_text:
+        with open(BOUNDARY_OUT, "w") as fh:
+            fh.write(boundary_text)
     fast_dev, fast_host, lin_keys = gen_fast(tables)
     body += [""] + fast_dev
     body += [""] + gen_fast_l6(tables["L6"]["bulk"], lin_keys)
