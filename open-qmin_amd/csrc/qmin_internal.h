@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -59,6 +60,7 @@ struct qm_lattice {
     int terms = 0;            // distortion terms of the force last prepared on this lattice
     double* dHField = nullptr;  // spatially varying H: planes hx, hy, hz of n (FP64)
     int numCUs = 0;
+    std::mutex scratchMutex;    // held while the state set that is not current serves as work space
 };
 
 struct qm_ldg {
