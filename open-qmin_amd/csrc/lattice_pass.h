@@ -475,9 +475,10 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
                     if constexpr (!step_early_load<R, TERMS>()) step_load<R, MODE>(A.step, n, i, pre);
                     step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
 #pragma unroll
-                    for (int c = 0; c < 5; ++c) {
-                        st_out(&out.q[c * n + i], qn[c]);
-                        st_out(&out.f[c * n + i], F[c]);
+                    for (int c = 0; c < 5; ++c) st_out(&out.q[c * n + i], qn[c]);
+                    if (A.storeF) {
+#pragma unroll
+                        for (int c = 0; c < 5; ++c) st_out(&out.f[c * n + i], F[c]);
                     }
                     pF += sq5(F);
                 } else if constexpr (kPF) {
@@ -663,9 +664,10 @@ __device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logi
             step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
             pF = sq5(F);
 #pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                out.q[k * n + i] = qn[k];
-                out.f[k * n + i] = F[k];
+            for (int k = 0; k < 5; ++k) out.q[k * n + i] = qn[k];
+            if (A.storeF) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) out.f[k * n + i] = F[k];
             }
         } else {
 #pragma unroll

@@ -1347,7 +1347,7 @@ int qmin::force_pass(qm_lattice* L, const qm_ldg* f, bool gated) {
 }
 
 template <typename R>
-static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, long long* slots) {
+static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, bool storeF, long long* slots) {
     // the force pass's tile and z chunk: the update adds no staging
     choose_zchunk(L, kForce, terms_of(f));
     MarchArgs<R> ma{};
@@ -1357,14 +1357,35 @@ static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs&
     fill_args<R>(L, f, ma, ba, fire, tile);
     ma.step = step;
     ba.step = step;
+    ma.storeF = storeF ? 1 : 0;
     HIP_TRY(launch_step<R>(ma, ba, mode, terms_of(f), tile, L->stream));
     *slots = (long long)ma.nblocks + boundary_slots(L);
     return QM_OK;
 }
 
-int qmin::step_pass(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, long long* slots) {
-    return L->precision == QM_FP64 ? step_pass_t<double>(L, f, mode, step, slots)
-                                   : step_pass_t<float>(L, f, mode, step, slots);
+int qmin::step_pass(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, bool storeF, long long* slots) {
+    return L->precision == QM_FP64 ? step_pass_t<double>(L, f, mode, step, storeF, slots)
+                                   : step_pass_t<float>(L, f, mode, step, storeF, slots);
+}
+
+template <typename R>
+static int last_step_force_t(qm_lattice* L, const qm_ldg* f) {
+    choose_zchunk(L, kForce, terms_of(f));
+    MarchArgs<R> ma{};
+    BoundaryArgs<R> ba{};
+    FireConst fire{};
+    const int tile = active_tile(L, kForce);
+    fill_args<R>(L, f, ma, ba, fire, tile);
+    const int cur = L->hCtrl.cur;
+    ma.set[cur].q = ba.set[cur].q = state_set<R>(L, cur ^ 1).q;
+    HIP_TRY(launch_march<R>(ma, kForce, terms_of(f), tile, L->stream));
+    launch_boundary<R>(ba, kForce, terms_of(f), L->stream);
+    HIP_TRY(hipGetLastError());
+    return QM_OK;
+}
+
+int qmin::last_step_force(qm_lattice* L, const qm_ldg* f) {
+    return L->precision == QM_FP64 ? last_step_force_t<double>(L, f) : last_step_force_t<float>(L, f);
 }
 
 int qmin::share_velocity(qm_lattice* L) {

@@ -223,7 +223,8 @@ struct MarchArgs {
     const R* W;         // composed bulk operator weights (device buffer, read with scalar loads)
     const double* hvar; // spatially varying H, planes hx, hy, hz of n (null: none)
     double hvarP;       // deltaChi mu0
-    int storeF;         // FIRE pass that keeps only Q and v: store F of the sites it finishes as well
+    int storeF;         // FIRE pass that keeps only Q and v, and the Adam and Nesterov passes: store F of the sites
+                        // they finish as well
     StepArgs step;      // modes kAdamStep, kNesterovStep
 };
 

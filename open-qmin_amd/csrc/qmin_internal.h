@@ -100,7 +100,12 @@ int force_pass(qm_lattice* L, const qm_ldg* f, bool gated);
 // to the other state set; the partial sums of |F|^2 go to the lattice's
 // partials buffer, three doubles per slot, and *slots receives their count.
 // The caller's finalize sums them, advances the minimizer and flips the set.
-int step_pass(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, long long* slots);
+// storeF: whether the other set gets the force of all sites, or (a run's passes
+// but the last, whose forces nothing reads) of the boundary pass's alone.
+int step_pass(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs& step, bool storeF, long long* slots);
+// F of the current set = forces at the other set's Q: those the last step pass
+// moved the current Q with, where it did not store them
+int last_step_force(qm_lattice* L, const qm_ldg* f);
 // copies U of the current state set into the other one, so that passes that
 // alternate the sets without touching U keep the FIRE velocity
 int share_velocity(qm_lattice* L);
