@@ -120,12 +120,23 @@ __device__ __forceinline__ void finish_bulk(const ForceConst& fc, R* F, const R*
     metric(F);
 }
 
-// Stores of the next state: not read again in this pass, so they are streamed
-// past L2 (non-temporal), which keeps L2 for the halo rows that neighbouring
-// tiles read.
-template <typename R>
+// Stores of the next state: not read again in this pass, so with NT they are
+// streamed past L2 (non-temporal), which keeps L2 for the halo rows that
+// neighbouring tiles read (nontemporal_stores has the rule).  A template
+// parameter: of stores in the two branches of a flag, the compiler makes plain
+// ones.
+template <bool NT, typename R>
 __device__ __forceinline__ void st_out(R* p, R v) {
-    __builtin_nontemporal_store(v, p);
+    if constexpr (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
+template <bool NT, typename R>
+__device__ __forceinline__ void st_site(R* field, long long n, long long i, const R* v) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c) st_out<NT>(&field[c * n + i], v[c]);
 }
 
 // Coefficients of one Adam or Nesterov update, from the minimizer's device
@@ -182,7 +193,7 @@ __device__ __forceinline__ void step_load(const StepArgs& S, long long n, long l
 // energyMinimizerNesterovAG::nesterovStepCPU (energyMinimizerNesterovAG.cpp:75-92).
 // Stores the advanced entries (no other work-item reads them in the pass) and
 // returns the new q.
-template <typename R, int MODE>
+template <typename R, int MODE, bool NT>
 __device__ __forceinline__ R step_component(const StepArgs& S, const StepCoef<R>& k, long long j, R q, R F, R m0,
                                             R v0) {
     R* m = static_cast<R*>(S.m);
@@ -194,23 +205,23 @@ __device__ __forceinline__ R step_component(const StepArgs& S, const StepCoef<R>
         const R vc = vv * k.inv2;
         R root = sqrt(vc);
         if (root == R(0)) root = k.eps;
-        st_out(&m[j], mm);
-        st_out(&v[j], vv);
+        st_out<NT>(&m[j], mm);
+        st_out<NT>(&v[j], vv);
         return q + k.mdt * mc / root;
     } else {
         const R alt = q + k.dt * F;
-        st_out(&m[j], alt);
+        st_out<NT>(&m[j], alt);
         return alt + k.mu * (alt - m0);
     }
 }
 
-template <typename R, int MODE>
+template <typename R, int MODE, bool NT>
 __device__ __forceinline__ void step_site(const StepArgs& S, const StepCoef<R>& k, long long n, long long i,
                                           const R* q, const R* F, const R (&pre)[2][5], R* qn) {
 #pragma unroll
     for (int c = 0; c < 5; ++c)
-        qn[c] = step_component<R, MODE>(S, k, c * n + i, q[c], F[c], pre[0][c],
-                                        MODE == kAdamStep ? pre[1][c] : R(0));
+        qn[c] = step_component<R, MODE, NT>(S, k, c * n + i, q[c], F[c], pre[0][c],
+                                            MODE == kAdamStep ? pre[1][c] : R(0));
 }
 
 // Sum of squares of the five stored components (the minimizers' |F|^2).
@@ -278,15 +289,15 @@ template <typename R>
 __device__ __forceinline__ R fire_drift(const FireMove<R>& m, R q, R u, R f, R& vh) {
     const R v = __builtin_elementwise_fma(m.ck, u, m.cf * f);
     vh = __builtin_elementwise_fma(m.hdt, f, v);
-    return q + __builtin_elementwise_fma(m.dt, v, m.hdt2 * f);
+    return __builtin_elementwise_fma(m.dt, v, __builtin_elementwise_fma(m.hdt2, f, q));
 }
 
 // One work-group's share of the fused pass: the column of tile `logical` (x
 // tile fastest, then y tile, then z chunk) of the lattice described by A; its
 // partial sums go to slot `slot`.
 // NARROW: the tile is A.tw x A.th sites (an ensemble's lattices, whose rows may
-// be shorter than TX), else TX x TY.
-template <typename R, int MODE, int TERMS, int TILE, bool NARROW>
+// be shorter than TX), else TX x TY.  NT: non-temporal stores of the next state.
+template <typename R, int MODE, int TERMS, int TILE, bool NARROW, bool NT>
 __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logical, const int slot) {
     using T = Tile<kTileTX[TILE], kTileTY[TILE], NARROW ? tile_rows<R>(TILE) : kTileTY[TILE]>;
     constexpr int kHX = T::HX, kHP = T::HP;
@@ -361,7 +372,7 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
             for (int c = 0; c < 5; ++c) {
                 R half;
                 q[c] = fire_drift(mv, q[c], u[c], f[c], half);
-                if (vh) vh[c] = half;
+                vh[c] = half;
             }
         }
 #pragma unroll
@@ -369,16 +380,27 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
     };
     auto stage = [&](int z, int s, R* vh, int& cOwn) {
         const long long zoff = plane * wrapi(z, lz);
-        R q[5], u[5], f[5], hq[5], hu[5], hf[5];
-        if (own) {
-            cOwn = A.cls[colOwn + zoff];
-            load_site(colOwn + zoff, q, u, f);
-        }
-        if (kTogether && hHalo >= 0) load_site(colHalo + zoff, hq, hu, hf);
-        if (own) put_site(s, hOwn, q, u, f, vh);
-        if (hHalo >= 0) {
-            if (!kTogether) load_site(colHalo + zoff, hq, hu, hf);
-            put_site(s, hHalo, hq, hu, hf, nullptr);
+        if constexpr (kTogether) {
+            R q[5], hq[5];
+            if (own) {
+                cOwn = A.cls[colOwn + zoff];
+                load_site(colOwn + zoff, q, nullptr, nullptr);
+            }
+            if (hHalo >= 0) load_site(colHalo + zoff, hq, nullptr, nullptr);
+            if (own) put_site(s, hOwn, q, nullptr, nullptr, nullptr);
+            if (hHalo >= 0) put_site(s, hHalo, hq, nullptr, nullptr, nullptr);
+        } else {
+            if (own) {
+                R q[5], u[5], f[5];
+                cOwn = A.cls[colOwn + zoff];
+                load_site(colOwn + zoff, q, u, f);
+                put_site(s, hOwn, q, u, f, vh);
+            }
+            if (hHalo >= 0) {
+                R q[5], u[5], f[5], unused[5];
+                load_site(colHalo + zoff, q, u, f);
+                put_site(s, hHalo, q, u, f, unused);
+            }
         }
     };
 
@@ -463,9 +485,9 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
                     for (int c = 0; c < 5; ++c) u[c] = __builtin_elementwise_fma(mv.hdt, F[c], vhCur[c]);
 #pragma unroll
                     for (int c = 0; c < 5; ++c) {
-                        st_out(&out.q[c * n + i], q[c]);
-                        st_out(&out.u[c * n + i], u[c]);
-                        st_out(&out.f[c * n + i], F[c]);
+                        st_out<NT>(&out.q[c * n + i], q[c]);
+                        st_out<NT>(&out.u[c * n + i], u[c]);
+                        st_out<NT>(&out.f[c * n + i], F[c]);
                     }
                     pF += qt_dot(F, F);
                     pP += qt_dot(F, u);
@@ -473,13 +495,9 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
                 } else if constexpr (is_step_mode(MODE)) {
                     R qn[5];
                     if constexpr (!step_early_load<R, TERMS>()) step_load<R, MODE>(A.step, n, i, pre);
-                    step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
-#pragma unroll
-                    for (int c = 0; c < 5; ++c) st_out(&out.q[c * n + i], qn[c]);
-                    if (A.storeF) {
-#pragma unroll
-                        for (int c = 0; c < 5; ++c) st_out(&out.f[c * n + i], F[c]);
-                    }
+                    step_site<R, MODE, NT>(A.step, sk, n, i, q, F, pre, qn);
+                    st_site<NT>(out.q, n, i, qn);
+                    if (A.storeF) st_site<NT>(out.f, n, i, F);
                     pF += sq5(F);
                 } else if constexpr (kPF) {
 #pragma unroll
@@ -493,8 +511,8 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
                 // the boundary pass finishes U and F of this site
 #pragma unroll
                 for (int c = 0; c < 5; ++c) {
-                    st_out(&out.q[c * n + i], q[c]);
-                    st_out(&out.u[c * n + i], vhCur[c]);
+                    st_out<NT>(&out.q[c * n + i], q[c]);
+                    st_out<NT>(&out.u[c * n + i], vhCur[c]);
                 }
             }
         }
@@ -661,7 +679,7 @@ __device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logi
             }
         } else if constexpr (is_step_mode(MODE)) {
             R qn[5];
-            step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
+            step_site<R, MODE, false>(A.step, sk, n, i, q, F, pre, qn);
             pF = sq5(F);
 #pragma unroll
             for (int k = 0; k < 5; ++k) out.q[k * n + i] = qn[k];
@@ -722,18 +740,18 @@ constexpr int march_min_waves() {
     return (sizeof(R) == 8 && TERMS == kMultiL6 && MODE == kForce && TILE == kTile32x8) ? 4 : 1;
 }
 
-template <typename R, int MODE, int TERMS, int TILE>
+template <typename R, int MODE, int TERMS, int TILE, bool NT>
 __global__ void __launch_bounds__(kTileThreads[TILE], (march_min_waves<R, MODE, TERMS, TILE>())) march_kernel(MarchArgs<R> A) {
-    march_body<R, MODE, TERMS, TILE, false>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
+    march_body<R, MODE, TERMS, TILE, false, NT>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
 // The 512-thread tiles (32 x 16, 64 x 8; 8 waves): two work-groups per CU need
 // at least four waves per SIMD, i.e. at most 128 VGPRs.
-template <typename R, int MODE, int TERMS, int TILE>
+template <typename R, int MODE, int TERMS, int TILE, bool NT>
 __global__ void __launch_bounds__(kTileThreads[TILE], 4) march_wide_kernel(MarchArgs<R> A) {
     static_assert(kTileThreads[TILE] == 512, "512-thread tiles only");
     constexpr bool kPair = sizeof(R) == 4 && TILE == kTile64x8;
-    march_body<R, MODE, TERMS, TILE, false>(A, xcd_logical<kPair>(blockIdx.x, A.nblocks), blockIdx.x);
+    march_body<R, MODE, TERMS, TILE, false, NT>(A, xcd_logical<kPair>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
 // Waves per SIMD asked of the compiler for the block pass: left alone it holds
@@ -749,6 +767,37 @@ __global__ void __launch_bounds__(Block::Threads, (block_min_waves<R, TERMS>()))
     block_body<R, MODE, TERMS>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
+// The pass of one lattice with tile `tile` (a halo-padded one, or kBlock).
+template <typename R, int MODE, int TERMS, bool NT>
+const void* march_fn_tile(int tile) {
+    switch (tile) {
+        case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4, NT>);
+        case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16, NT>);
+        case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8, NT>);
+        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
+        default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8, NT>);
+    }
+}
+
+template <typename R, int MODE, bool NT>
+const void* march_fn_terms(int terms, int tile) {
+    switch (terms) {
+        case kOneConstant: return march_fn_tile<R, MODE, kOneConstant, NT>(tile);
+        case kMultiLinear: return march_fn_tile<R, MODE, kMultiLinear, NT>(tile);
+        case kMultiL4: return march_fn_tile<R, MODE, kMultiL4, NT>(tile);
+        default: return march_fn_tile<R, MODE, kMultiL6, NT>(tile);
+    }
+}
+
+// (force passes store F plainly)
+template <typename R, int MODE>
+const void* march_fn_mode(int terms, int tile, bool nt) {
+    if constexpr (MODE == kForce)
+        return march_fn_terms<R, MODE, false>(terms, tile);
+    else
+        return nt ? march_fn_terms<R, MODE, true>(terms, tile) : march_fn_terms<R, MODE, false>(terms, tile);
+}
+
 // The fused pass over many lattices in one launch: map[b] = {lattice, logical
 // tile} for hardware work-group b, laid out by the host in XCD-aware order.
 template <typename R, int MODE, int TERMS, int TILE>
@@ -757,7 +806,7 @@ __global__ void __launch_bounds__(kTileThreads[TILE]) march_batch_kernel(const M
     // uniform over the work-group: read once, keep in scalar registers
     const int lat = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
     const int logical = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
-    march_body<R, MODE, TERMS, TILE, true>(descs[lat], logical, logical);
+    march_body<R, MODE, TERMS, TILE, true, true>(descs[lat], logical, logical);
 }
 
 template <typename R, int MODE, int TERMS, int TILE>
@@ -766,7 +815,7 @@ __global__ void __launch_bounds__(kTileThreads[TILE], 4) march_wide_batch_kernel
     static_assert(kTileThreads[TILE] == 512, "512-thread tiles only");
     const int lat = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
     const int logical = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
-    march_body<R, MODE, TERMS, TILE, true>(descs[lat], logical, logical);
+    march_body<R, MODE, TERMS, TILE, true, true>(descs[lat], logical, logical);
 }
 
 // ---------------------------------------------------------------- boundary pass
@@ -940,7 +989,7 @@ __device__ __forceinline__ void boundary_site_body(const BoundaryArgs<R>& A, con
         } else if constexpr (is_step_mode(MODE)) {
             const StateSet<R> out = A.set[cur ^ 1];
             R qn[5];
-            step_site<R, MODE>(A.step, sk, n, i, q, F, pre, qn);
+            step_site<R, MODE, false>(A.step, sk, n, i, q, F, pre, qn);
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
                 out.q[c * n + i] = qn[c];
@@ -1139,7 +1188,7 @@ __device__ __forceinline__ void boundary_lanes_body(const BoundaryArgs<R>& A, co
         } else if constexpr (is_step_mode(MODE)) {
             if (put) {
                 const StateSet<R> out = A.set[cur ^ 1];
-                out.q[own] = step_component<R, MODE>(A.step, sk, own, qd, Fd, pre0, pre1);
+                out.q[own] = step_component<R, MODE, false>(A.step, sk, own, qd, Fd, pre0, pre1);
                 out.f[own] = Fd;
                 pF += double(Fd) * double(Fd);
             }

@@ -355,30 +355,9 @@ __global__ void defect_kernel(const R* q, const SiteType* types, long long n, in
 
 // ---------------------------------------------------------------- host launchers
 
-template <typename R, int MODE, int TERMS>
-static const void* march_fn_tile(int tile) {
-    switch (tile) {
-        case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4>);
-        case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16>);
-        case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8>);
-        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
-        default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8>);
-    }
-}
-
-template <typename R, int MODE>
-static const void* march_fn_terms(int terms, int tile) {
-    switch (terms) {
-        case kOneConstant: return march_fn_tile<R, MODE, kOneConstant>(tile);
-        case kMultiLinear: return march_fn_tile<R, MODE, kMultiLinear>(tile);
-        case kMultiL4: return march_fn_tile<R, MODE, kMultiL4>(tile);
-        default: return march_fn_tile<R, MODE, kMultiL6>(tile);
-    }
-}
-
 template <typename R>
-static const void* march_fn(int mode, int terms, int tile) {
-    return mode == kFire ? march_fn_terms<R, kFire>(terms, tile) : march_fn_terms<R, kForce>(terms, tile);
+static const void* march_fn(int mode, int terms, int tile, bool nt) {
+    return mode == kFire ? march_fn_mode<R, kFire>(terms, tile, nt) : march_fn_mode<R, kForce>(terms, tile, nt);
 }
 
 template <typename R, int MODE, int TERMS>
@@ -437,7 +416,7 @@ hipError_t launch_fire_finalize_batch(const FinalizeDesc* descs, EnsembleStatus*
 template <typename R>
 hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hipStream_t s) {
     void* args[] = {const_cast<MarchArgs<R>*>(&a)};
-    return hipLaunchKernel(march_fn<R>(mode, terms, tile), dim3(a.nblocks), dim3(tile_threads(tile)), args, 0, s);
+    return hipLaunchKernel(march_fn<R>(mode, terms, tile, a.nt != 0), dim3(a.nblocks), dim3(tile_threads(tile)), args, 0, s);
 }
 
 template <typename R>
@@ -470,7 +449,7 @@ void launch_move_q(R* q, long long n, const int64_t* src, const int64_t* dst, lo
 template <typename R>
 int march_blocks_per_cu(int mode, int terms, int tile) {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, march_fn<R>(mode, terms, tile), tile_threads(tile), 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, march_fn<R>(mode, terms, tile, true), tile_threads(tile), 0) !=
         hipSuccess)
         return 1;
     return blocks < 1 ? 1 : blocks;

@@ -1175,16 +1175,44 @@ static void choose_zchunk(qm_lattice* L, int mode, int terms) {
     else
         perCU = L->precision == QM_FP64 ? march_blocks_per_cu<double>(mode, terms, tile)
                                         : march_blocks_per_cu<float>(mode, terms, tile);
-    const long long columns = tile_columns(L, tile);
-    long long chunks = (long long)perCU * L->numCUs / columns;
-    if (chunks < 1) chunks = 1;
-    int zc = (int)((L->lz + chunks - 1) / chunks);
-    L->zchunk = std::max(4, std::min(zc, L->lz));
+    const long long columns = tile_columns(L, tile), slots = (long long)perCU * L->numCUs;
+    auto cost = [&](int zc) {
+        const long long groups = columns * ((L->lz + zc - 1) / zc);
+        return (double)((groups + slots - 1) / slots) * (zc + 4);   // a chunk of zc planes passes zc + 4
+    };
+    const long long chunks = std::max(1LL, slots / columns);
+    const int once = std::max(4, std::min((int)((L->lz + chunks - 1) / chunks), L->lz));
+    int best = once;
+    // The pass that keeps only Q and v has one work-group per CU: where one round
+    // of them would leave many CUs idle, several shorter ones are better (200^3
+    // FP64, 182 work-groups of 100 planes: 574 us; 455 of 40: 485; 192^3 399 and
+    // 388).  The marching passes gain nothing so (220^3 FP32: 394 and 437 us).
+    if (is_stream_tile(tile))
+        for (int zc = once - 1; zc >= 12; --zc)
+            if (cost(zc) < 0.95 * cost(once) && cost(zc) < cost(best)) best = zc;
+    L->zchunk = best;
 }
 
 static int march_blocks(const qm_lattice* L, int mode) {
     const int zc = std::min(L->zchunk, L->lz);
     return int(tile_columns(L, active_tile(L, mode)) * ((L->lz + zc - 1) / zc));
+}
+
+// Non-temporal stores of the next state (marching passes).  They pay on
+// lattices beyond the 256 MB memory-side cache, where plain ones push halo
+// rows out of L2; below it the next pass finds plain ones in that cache.  A
+// FIRE pass over rows that are no multiple of 64 bytes also stores plainly:
+// lines shared between rows then fill up in L2 before they are written.  Per
+// iteration, non-temporal and plain (us): FIRE L1..L3 FP32 128^3 68 and 59,
+// 144^3 113 and 115, 180^3 250 and 210, 192^3 203 and 204, 200^3 314 and 287,
+// 256^3 443 and 453; FP64 104^3 90 and 80; L6 FP64 128^3 138 and 144, 150^3 270
+// and 241; Nesterov FP64 128^3 78 and 68, 131^3 98 and 101, 200^3 308 and 340;
+// Adam FP32 131^3 92 and 83, 192^3 221 and 222.
+// fields: of five reals, that a pass touches.
+static int nontemporal_stores(const qm_lattice* L, int mode, int fields) {
+    const double bytes = 5.0 * fields * L->realSize * (double)L->n;
+    if (mode == kFire) return bytes > 288e6 && (L->lx * L->realSize) % 64 == 0;
+    return bytes > 256e6;
 }
 
 // One pass (force only or one FIRE iteration); kernels only, no host sync.
@@ -1206,6 +1234,7 @@ static int run_pass(qm_lattice* L, const qm_ldg* f, int mode, const FireConst& f
     ma.gate = gated ? 1 : 0;
     ba.gate = ma.gate;
     ma.storeF = storeF ? 1 : 0;
+    ma.nt = nontemporal_stores(L, mode, 6);
     const int terms = terms_of(f);
     hipEvent_t ev[3];
     if (g_timing.on && mode == kFire) {
@@ -1252,6 +1281,7 @@ static int time_march(qm_lattice* L, const qm_ldg* f, int reps, double* ms) {
     FireConst fire{};
     const int terms = terms_of(f), tile = active_tile(L, kFire);
     fill_args<R>(L, f, ma, ba, fire, tile);
+    ma.nt = nontemporal_stores(L, kFire, 6);
     auto launch = [&]() {
         return is_stream_tile(tile) ? launch_fire_stream<R>(ma, terms, tile, L->stream)
                                     : launch_march<R>(ma, kFire, terms, tile, L->stream);
@@ -1358,6 +1388,7 @@ static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs&
     ma.step = step;
     ba.step = step;
     ma.storeF = storeF ? 1 : 0;
+    ma.nt = nontemporal_stores(L, mode, mode == kAdamStep ? 4 : 3);
     HIP_TRY(launch_step<R>(ma, ba, mode, terms_of(f), tile, L->stream));
     *slots = (long long)ma.nblocks + boundary_slots(L);
     return QM_OK;

@@ -225,6 +225,7 @@ struct MarchArgs {
     double hvarP;       // deltaChi mu0
     int storeF;         // FIRE pass that keeps only Q and v, and the Adam and Nesterov passes: store F of the sites
                         // they finish as well
+    int nt;             // non-temporal stores of the next state (marching passes)
     StepArgs step;      // modes kAdamStep, kNesterovStep
 };
 

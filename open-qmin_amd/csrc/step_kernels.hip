@@ -9,31 +9,6 @@
 #include "lattice_pass.h"
 
 namespace qmin {
-namespace {
-
-template <typename R, int MODE, int TERMS>
-const void* step_fn_tile(int tile) {
-    switch (tile) {
-        case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4>);
-        case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16>);
-        case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8>);
-        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
-        default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8>);
-    }
-}
-
-template <typename R, int MODE>
-const void* step_fn_terms(int terms, int tile) {
-    switch (terms) {
-        case kOneConstant: return step_fn_tile<R, MODE, kOneConstant>(tile);
-        case kMultiLinear: return step_fn_tile<R, MODE, kMultiLinear>(tile);
-        case kMultiL4: return step_fn_tile<R, MODE, kMultiL4>(tile);
-        default: return step_fn_tile<R, MODE, kMultiL6>(tile);
-    }
-}
-
-}  // namespace
-
 // Queues the fused pass (tile `tile`, one of the halo-padded ones or kBlock) and
 // the boundary pass of one Adam or Nesterov iteration.
 template <typename R>
@@ -41,8 +16,8 @@ hipError_t launch_step(const MarchArgs<R>& ma, const BoundaryArgs<R>& ba, int mo
                        hipStream_t s) {
     if (!(tile >= 0 && tile < kNumMarchTiles) && tile != kBlock) return hipErrorInvalidValue;
     if (!is_step_mode(mode)) return hipErrorInvalidValue;
-    const void* fn = mode == kAdamStep ? step_fn_terms<R, kAdamStep>(terms, tile)
-                                       : step_fn_terms<R, kNesterovStep>(terms, tile);
+    const void* fn = mode == kAdamStep ? march_fn_mode<R, kAdamStep>(terms, tile, ma.nt != 0)
+                                       : march_fn_mode<R, kNesterovStep>(terms, tile, ma.nt != 0);
     void* margs[] = {const_cast<MarchArgs<R>*>(&ma)};
     hipError_t e = hipLaunchKernel(fn, dim3(ma.nblocks), dim3(tile_threads(tile)), margs, 0, s);
     if (e != hipSuccess) return e;
