@@ -267,29 +267,33 @@ __device__ __forceinline__ void wait_plane(const R (&a)[5], const R (&b)[5], int
     asm volatile("" ::"v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]) : "memory");
 }
 
-// The pending FIRE velocity mix v = ck u + cf F, (1, 0) when none is pending and
-// (0, 0) after a reset (energyMinimizerFIRE.cpp:117-144), and the step.
+// Velocity-Verlet drift and first half kick of one site with the pending FIRE
+// velocity mix v = ck u + cf F, (1, 0) when none is pending and (0, 0) after a
+// reset (energyMinimizerFIRE.cpp:117-144, velocityVerlet.cpp:8-40):
+//   q + dt v + dt^2/2 F = q + (du u + df F),  v + dt/2 F = vu u + vf F.
+// One rounding of q, and the products contracted by hand, so that every pass that
+// drifts a site rounds alike.
 template <typename R>
 struct FireMove {
-    R dt, hdt, hdt2, ck, cf;
+    R du, df, vu, vf, hdt;
 };
 
 template <typename R>
 __device__ __forceinline__ FireMove<R> fire_move(const Ctrl* ctrl) {
-    const double dtd = ctrl->dt;
+    const double dt = ctrl->dt;
     const int reset = ctrl->reset, identity = ctrl->identity;
-    return {R(dtd), R(0.5 * dtd), R(0.5 * dtd * dtd), reset ? R(0) : (identity ? R(1) : R(ctrl->cKeep)),
-            (reset || identity) ? R(0) : R(ctrl->cForce)};
+    const double ck = reset ? 0.0 : (identity ? 1.0 : ctrl->cKeep), cf = (reset || identity) ? 0.0 : ctrl->cForce;
+    return {R(dt * ck), R(dt * cf + 0.5 * dt * dt), R(ck), R(cf + 0.5 * dt), R(0.5 * dt)};
 }
 
-// Velocity-Verlet drift of one site with the pending mix: q + dt v + dt^2/2 F, and
-// the half-kicked velocity v + dt/2 F (velocityVerlet.cpp:8-40).  The products
-// are contracted by hand, so that every pass that drifts a site rounds alike.
 template <typename R>
-__device__ __forceinline__ R fire_drift(const FireMove<R>& m, R q, R u, R f, R& vh) {
-    const R v = __builtin_elementwise_fma(m.ck, u, m.cf * f);
-    vh = __builtin_elementwise_fma(m.hdt, f, v);
-    return __builtin_elementwise_fma(m.dt, v, __builtin_elementwise_fma(m.hdt2, f, q));
+__device__ __forceinline__ R fire_drift(const FireMove<R>& m, R q, R u, R f) {
+    return q + __builtin_elementwise_fma(m.du, u, m.df * f);
+}
+
+template <typename R>
+__device__ __forceinline__ R fire_half_kick(const FireMove<R>& m, R u, R f) {
+    return __builtin_elementwise_fma(m.vu, u, m.vf * f);
 }
 
 // One work-group's share of the fused pass: the column of tile `logical` (x
@@ -370,9 +374,8 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
         if (MODE == kFire) {
 #pragma unroll
             for (int c = 0; c < 5; ++c) {
-                R half;
-                q[c] = fire_drift(mv, q[c], u[c], f[c], half);
-                vh[c] = half;
+                q[c] = fire_drift(mv, q[c], u[c], f[c]);
+                vh[c] = fire_half_kick(mv, u[c], f[c]);
             }
         }
 #pragma unroll
@@ -629,9 +632,8 @@ __device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logi
         if (MODE == kFire) {
 #pragma unroll
             for (int k = 0; k < 5; ++k) {
-                R half;
-                a[k] = fire_drift(mv, a[k], b[k], c[k], half);
-                if (v2) v2[k] = half;
+                a[k] = fire_drift(mv, a[k], b[k], c[k]);
+                if (v2) v2[k] = fire_half_kick(mv, b[k], c[k]);
             }
         }
     };
