@@ -267,6 +267,66 @@ __device__ __forceinline__ void wait_plane(const R (&a)[5], const R (&b)[5], int
     asm volatile("" ::"v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]) : "memory");
 }
 
+// FIRE scalar step of energyMinimizerFIRE::fireStepCPU (energyMinimizerFIRE.cpp:77-145),
+// run by one thread once all partial sums are in.
+__device__ __forceinline__ void fire_scalar_step(Ctrl* ctrl, const FireConst& fp, double fnorm, double power, double vnorm,
+                                 double* trace) {
+    const int it = ctrl->iterations + 1;
+    const double forceMax = sqrt(fnorm) / fp.nTotal;
+    const double scaling = fnorm > 0. ? sqrt(vnorm / fnorm) : 0.0;
+    double alpha = ctrl->alpha, dt = ctrl->dt;
+    int nPos = ctrl->nPositive;
+    ctrl->cKeep = 1.0 - alpha;
+    ctrl->cForce = alpha * scaling;
+    ctrl->identity = 0;
+    if (power > 0 && it % 500 != 0) {
+        if (nPos > fp.nMin) {
+            dt = fmin(dt * fp.dtInc, fp.dtMax);
+            alpha = alpha * fp.alphaDec;
+            alpha = fmax(alpha, fp.alphaMin);
+        }
+        nPos += 1;
+        ctrl->reset = 0;
+    } else {
+        nPos = 0;
+        dt = dt * fp.dtDec;
+        dt = fmax(dt, fp.dtMin);
+        alpha = fp.alphaStart;
+        ctrl->reset = 1;
+    }
+    ctrl->alpha = alpha;
+    ctrl->dt = dt;
+    ctrl->nPositive = nPos;
+    ctrl->iterations = it;
+    ctrl->forceMax = forceMax;
+    ctrl->power = power;
+    ctrl->fnorm = fnorm;
+    ctrl->vnorm = vnorm;
+    ctrl->scaling = scaling;
+    if (trace && ctrl->traceLen < ctrl->traceCap) {
+        double* t = trace + 6 * (long long)ctrl->traceLen;
+        t[0] = forceMax;
+        t[1] = power;
+        t[2] = alpha;
+        t[3] = dt;
+        t[4] = scaling;
+        t[5] = nPos;
+        ctrl->traceLen += 1;
+    }
+    ctrl->cur ^= 1;
+    if (isnan(forceMax)) ctrl->nanFlag = 1;
+    ctrl->done = !(it < ctrl->maxIter && forceMax > fp.fc);
+}
+
+// This thread's share of the fixed-order sum of the partials of `total` slots.
+__device__ __forceinline__ void fire_partials(const double* part, long long total, double& s0, double& s1, double& s2) {
+    for (long long j = threadIdx.x; j < total; j += kReduceThreads) {
+        s0 += part[3 * j + 0];
+        s1 += part[3 * j + 1];
+        s2 += part[3 * j + 2];
+    }
+}
+
 // Velocity-Verlet drift and first half kick of one site with the pending FIRE
 // velocity mix v = ck u + cf F, (1, 0) when none is pending and (0, 0) after a
 // reset (energyMinimizerFIRE.cpp:117-144, velocityVerlet.cpp:8-40):
@@ -547,21 +607,24 @@ __device__ __forceinline__ void march_body(const MarchArgs<R>& A, const int logi
 // LDS at once, so that a pass lasts one load latency and one force computation
 // instead of marching through planes that each wait for their loads.  The halo
 // is 1.5 sites per site, read mostly from L2.  FIRE iteration at 24^3, L1, FP64:
-// 12 against 20 us, at 50^3, L1..L3: 21 against 28 us (three launches each).
-template <typename R, int MODE, int TERMS>
+// 12 against 20 us, at 50^3, L1..L3: 21 against 28 us (three launches each;
+// 8.7 and 18 us chained).
+// CHAIN: a FIRE pass that takes the previous iteration's scalar step (ChainArgs).
+template <typename R, int MODE, int TERMS, bool CHAIN>
 __device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logical, const int slot) {
     using B = Block;
     constexpr int kHX = B::HX, kHP = B::HP;
     __shared__ R sQ[B::HZ][5][kHP];
     __shared__ double sRed[B::Threads / 64][3];
 
+    static_assert(!CHAIN || MODE == kFire, "FIRE passes are chained");
     Ctrl* ctrl = A.ctrl;
-    if ((MODE != kForce || A.gate) && ctrl->done) return;
-    const int cur = ctrl->cur;
+    if (!CHAIN && (MODE != kForce || A.gate) && ctrl->done) return;
+    const int cur = CHAIN ? A.chain.cur : ctrl->cur;
     const StateSet<R> in = A.set[cur];
     const StateSet<R> out = A.set[MODE == kForce ? cur : cur ^ 1];
     FireMove<R> mv{};
-    if (MODE == kFire) mv = fire_move<R>(ctrl);
+    if (MODE == kFire && !CHAIN) mv = fire_move<R>(ctrl);
     StepCoef<R> sk{};
     if constexpr (is_step_mode(MODE)) sk = step_coef<R, MODE>(A.step);
 
@@ -622,6 +685,26 @@ __device__ __forceinline__ void block_body(const MarchArgs<R>& A, const int logi
             hZ[r] = hz;
             load_site(site(hx, hy, hz), hq[r], hu[r], hf[r]);
         }
+    }
+    if constexpr (CHAIN) {
+        // the previous iteration's scalar step, in every work-group while the
+        // sites' loads are in flight; the first one keeps its outcome
+        static_assert(B::Threads == kReduceThreads, "one work-group sums as fire_finalize_kernel does");
+        __shared__ Ctrl sCtrl;
+        double s0 = 0, s1 = 0, s2 = 0;
+        if (A.chain.pending) {
+            fire_partials(A.chain.prev, A.chain.total, s0, s1, s2);
+            block_sum3<kReduceThreads>(s0, s1, s2, sRed);
+        }
+        if (tid == 0) {
+            sCtrl = *ctrl;
+            if (A.chain.pending && !sCtrl.done)
+                fire_scalar_step(&sCtrl, A.chain.fire, s0, s1, s2, slot == 0 ? A.chain.trace : nullptr);
+            if (slot == 0) *A.chain.next = sCtrl;
+        }
+        __syncthreads();
+        if (sCtrl.done) return;
+        mv = fire_move<R>(&sCtrl);
     }
     R pre[2][5];
     if constexpr (is_step_mode(MODE))
@@ -758,15 +841,16 @@ __global__ void __launch_bounds__(kTileThreads[TILE], 4) march_wide_kernel(March
 
 // Waves per SIMD asked of the compiler for the block pass: left alone it holds
 // the operands of a whole stencil in registers (213 to 256 in FP64, one or two
-// waves); at four, 52 to 120 do without spills, with FP64 L6 138 at three.
-template <typename R, int TERMS>
+// waves); at four, 52 to 122 do without spills, at three 134 with FP64 L6 and 132
+// to 149 in a chained FP64 pass.
+template <typename R, int TERMS, bool CHAIN>
 constexpr int block_min_waves() {
-    return TERMS == kMultiL6 && sizeof(R) == 8 ? 2 : 4;
+    return sizeof(R) == 4 ? 4 : (TERMS == kMultiL6 ? 2 : (CHAIN ? 3 : 4));
 }
 
-template <typename R, int MODE, int TERMS>
-__global__ void __launch_bounds__(Block::Threads, (block_min_waves<R, TERMS>())) block_kernel(MarchArgs<R> A) {
-    block_body<R, MODE, TERMS>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
+template <typename R, int MODE, int TERMS, bool CHAIN>
+__global__ void __launch_bounds__(Block::Threads, (block_min_waves<R, TERMS, CHAIN>())) block_kernel(MarchArgs<R> A) {
+    block_body<R, MODE, TERMS, CHAIN>(A, xcd_logical<false>(blockIdx.x, A.nblocks), blockIdx.x);
 }
 
 // The pass of one lattice with tile `tile` (a halo-padded one, or kBlock).
@@ -776,7 +860,7 @@ const void* march_fn_tile(int tile) {
         case kTile64x4: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile64x4, NT>);
         case kTile32x16: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile32x16, NT>);
         case kTile64x8: return reinterpret_cast<const void*>(&march_wide_kernel<R, MODE, TERMS, kTile64x8, NT>);
-        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS>);
+        case kBlock: return reinterpret_cast<const void*>(&block_kernel<R, MODE, TERMS, false>);
         default: return reinterpret_cast<const void*>(&march_kernel<R, MODE, TERMS, kTile32x8, NT>);
     }
 }

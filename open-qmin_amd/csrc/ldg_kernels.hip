@@ -23,57 +23,6 @@
 
 namespace qmin {
 
-// FIRE scalar step of energyMinimizerFIRE::fireStepCPU (energyMinimizerFIRE.cpp:77-145),
-// run by one thread once all partial sums are in.
-__device__ void fire_scalar_step(Ctrl* ctrl, const FireConst& fp, double fnorm, double power, double vnorm,
-                                 double* trace) {
-    const int it = ctrl->iterations + 1;
-    const double forceMax = sqrt(fnorm) / fp.nTotal;
-    const double scaling = fnorm > 0. ? sqrt(vnorm / fnorm) : 0.0;
-    double alpha = ctrl->alpha, dt = ctrl->dt;
-    int nPos = ctrl->nPositive;
-    ctrl->cKeep = 1.0 - alpha;
-    ctrl->cForce = alpha * scaling;
-    ctrl->identity = 0;
-    if (power > 0 && it % 500 != 0) {
-        if (nPos > fp.nMin) {
-            dt = fmin(dt * fp.dtInc, fp.dtMax);
-            alpha = alpha * fp.alphaDec;
-            alpha = fmax(alpha, fp.alphaMin);
-        }
-        nPos += 1;
-        ctrl->reset = 0;
-    } else {
-        nPos = 0;
-        dt = dt * fp.dtDec;
-        dt = fmax(dt, fp.dtMin);
-        alpha = fp.alphaStart;
-        ctrl->reset = 1;
-    }
-    ctrl->alpha = alpha;
-    ctrl->dt = dt;
-    ctrl->nPositive = nPos;
-    ctrl->iterations = it;
-    ctrl->forceMax = forceMax;
-    ctrl->power = power;
-    ctrl->fnorm = fnorm;
-    ctrl->vnorm = vnorm;
-    ctrl->scaling = scaling;
-    if (trace && ctrl->traceLen < ctrl->traceCap) {
-        double* t = trace + 6 * (long long)ctrl->traceLen;
-        t[0] = forceMax;
-        t[1] = power;
-        t[2] = alpha;
-        t[3] = dt;
-        t[4] = scaling;
-        t[5] = nPos;
-        ctrl->traceLen += 1;
-    }
-    ctrl->cur ^= 1;
-    if (isnan(forceMax)) ctrl->nanFlag = 1;
-    ctrl->done = !(it < ctrl->maxIter && forceMax > fp.fc);
-}
-
 // FIRE scalar step after both lattice passes of an iteration: one work-group
 // sums every partial in a fixed order (fused-pass blocks, then boundary-pass
 // blocks) and advances the FIRE scalars.  A kernel of its own: the launch
@@ -84,18 +33,16 @@ __device__ __forceinline__ void fire_finalize_body(Ctrl* ctrl, const FireConst& 
     __shared__ double sRed[kReduceThreads / 64][3];
     if (ctrl->done) return;
     double s0 = 0, s1 = 0, s2 = 0;
-    for (long long j = threadIdx.x; j < total; j += kReduceThreads) {
-        s0 += part[3 * j + 0];
-        s1 += part[3 * j + 1];
-        s2 += part[3 * j + 2];
-    }
+    fire_partials(part, total, s0, s1, s2);
     block_sum3<kReduceThreads>(s0, s1, s2, sRed);
     if (threadIdx.x == 0) fire_scalar_step(ctrl, fp, s0, s1, s2, trace);
 }
 
+// copy: where the control block is wanted as well (or null).
 __global__ void __launch_bounds__(kReduceThreads) fire_finalize_kernel(Ctrl* ctrl, FireConst fp, const double* part,
-                                                                      long long total, double* trace) {
+                                                                      long long total, double* trace, Ctrl* copy) {
     fire_finalize_body(ctrl, fp, part, total, trace);
+    if (copy && threadIdx.x == 0) *copy = *ctrl;
 }
 
 // One work-group per lattice of an ensemble; each also copies its lattice's
@@ -356,6 +303,16 @@ __global__ void defect_kernel(const R* q, const SiteType* types, long long n, in
 // ---------------------------------------------------------------- host launchers
 
 template <typename R>
+static const void* chained_fn(int terms) {
+    switch (terms) {
+        case kOneConstant: return reinterpret_cast<const void*>(&block_kernel<R, kFire, kOneConstant, true>);
+        case kMultiLinear: return reinterpret_cast<const void*>(&block_kernel<R, kFire, kMultiLinear, true>);
+        case kMultiL4: return reinterpret_cast<const void*>(&block_kernel<R, kFire, kMultiL4, true>);
+        default: return reinterpret_cast<const void*>(&block_kernel<R, kFire, kMultiL6, true>);
+    }
+}
+
+template <typename R>
 static const void* march_fn(int mode, int terms, int tile, bool nt) {
     return mode == kFire ? march_fn_mode<R, kFire>(terms, tile, nt) : march_fn_mode<R, kForce>(terms, tile, nt);
 }
@@ -416,6 +373,8 @@ hipError_t launch_fire_finalize_batch(const FinalizeDesc* descs, EnsembleStatus*
 template <typename R>
 hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hipStream_t s) {
     void* args[] = {const_cast<MarchArgs<R>*>(&a)};
+    if (a.chain.on)
+        return hipLaunchKernel(chained_fn<R>(terms), dim3(a.nblocks), dim3(Block::Threads), args, 0, s);
     return hipLaunchKernel(march_fn<R>(mode, terms, tile, a.nt != 0), dim3(a.nblocks), dim3(tile_threads(tile)), args, 0, s);
 }
 
@@ -456,8 +415,8 @@ int march_blocks_per_cu(int mode, int terms, int tile) {
 }
 
 void launch_fire_finalize(Ctrl* ctrl, const FireConst& fp, const double* partials, long long total, double* trace,
-                          hipStream_t s) {
-    hipLaunchKernelGGL(fire_finalize_kernel, dim3(1), dim3(kReduceThreads), 0, s, ctrl, fp, partials, total, trace);
+                          Ctrl* copy, hipStream_t s) {
+    hipLaunchKernelGGL(fire_finalize_kernel, dim3(1), dim3(kReduceThreads), 0, s, ctrl, fp, partials, total, trace, copy);
 }
 
 template <typename R>

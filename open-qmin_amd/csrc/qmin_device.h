@@ -165,13 +165,10 @@ struct Ctrl {
     int reset;      // pending velocity reset (v = 0) from the last FIRE step
     int identity;   // no pending velocity mix (v = u)
     int nanFlag;
-    unsigned int arrive;
     int traceLen;
     int traceCap;
-    int pad;
     double dt, alpha;
     double cKeep, cForce;   // pending mix v = cKeep u + cForce F
-    double slot[40];        // minimizer scalars finished on the device (L-BFGS s.y, a_i, coefficients)
     double forceMax, power, fnorm, vnorm, scaling;
 };
 
@@ -208,6 +205,21 @@ struct StateSet {
     R* f;
 };
 
+// A FIRE pass that begins with the scalar step of the iteration before it, whose
+// partial sums are then still to be summed (block_body): an iteration is one
+// launch less.  The control block alternates between two places, as some
+// work-groups read the old one while the first writes the new.
+struct ChainArgs {
+    int on;                 // the pass is one of these
+    int pending;            // there is such a step (not before a run's first pass)
+    int cur;                // the current state set, unless the run is done
+    const double* prev;     // partial sums of the previous iteration
+    long long total;        // and their slots
+    Ctrl* next;             // receives the control block after the step
+    FireConst fire;
+    double* trace;
+};
+
 template <typename R>
 struct MarchArgs {
     StateSet<R> set[2];
@@ -227,6 +239,7 @@ struct MarchArgs {
                         // they finish as well
     int nt;             // non-temporal stores of the next state (marching passes)
     StepArgs step;      // modes kAdamStep, kNesterovStep
+    ChainArgs chain;    // block pass in mode kFire
 };
 
 template <typename R>

@@ -46,7 +46,7 @@ struct qm_lattice {
     void* dSet[2] = {nullptr, nullptr};   // each 15 n reals: Q, U, F planes
     int32_t* dSites = nullptr;            // compacted sites finished by the boundary pass
     long long nBoundary = 0;
-    Ctrl* dCtrl = nullptr;
+    Ctrl* dCtrl = nullptr;                 // [2]: the second is a chained run's other place (ChainArgs)
     Ctrl hCtrl{};                          // host mirror, valid after syncCtrl
     double* dPartials = nullptr;
     size_t partialsCap = 0;
