@@ -64,14 +64,45 @@ __global__ void __launch_bounds__(kReduceThreads) fire_finalize_batch_kernel(con
 
 // Materialize the pending FIRE velocity mix into U of the current set.
 template <typename R>
-__global__ void materialize_velocity_kernel(StateSet<R> s0, StateSet<R> s1, long long n, Ctrl* ctrl) {
-    const StateSet<R> st = ctrl->cur ? s1 : s0;
+__device__ __forceinline__ void materialize_velocity(const StateSet<R>& st, long long n, const Ctrl* ctrl) {
     const int mix = ctrl->reset ? 2 : (ctrl->identity ? 0 : 1);
     const R ck = R(ctrl->cKeep), cf = R(ctrl->cForce);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 5 * n; i += (long long)gridDim.x * blockDim.x) {
         const R u = st.u[i];
         st.u[i] = mix == 2 ? R(0) : (mix == 0 ? u : ck * u + cf * st.f[i]);
     }
+}
+
+template <typename R>
+__global__ void materialize_velocity_kernel(StateSet<R> s0, StateSet<R> s1, long long n, Ctrl* ctrl) {
+    materialize_velocity(ctrl->cur ? s1 : s0, n, ctrl);
+}
+
+// The same for the lattices of an ensemble, blockIdx.y each, and afterwards
+// their control blocks.
+template <typename R>
+__global__ void materialize_batch_kernel(const MarchArgs<R>* __restrict__ descs) {
+    const MarchArgs<R>& A = descs[blockIdx.y];
+    if (A.ctrl->identity) return;
+    materialize_velocity(A.set[A.ctrl->cur], A.n, A.ctrl);
+}
+
+template <typename R>
+__global__ void materialized_kernel(const MarchArgs<R>* __restrict__ descs, int count) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= count || descs[k].ctrl->identity) return;
+    descs[k].ctrl->identity = 1;
+    descs[k].ctrl->reset = 0;
+}
+
+__global__ void gather_ctrls_kernel(const FinalizeDesc* __restrict__ descs, Ctrl* all, int count) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < count) all[k] = *descs[k].ctrl;
+}
+
+__global__ void scatter_ctrls_kernel(const FinalizeDesc* __restrict__ descs, const Ctrl* all, int count) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < count) *descs[k].ctrl = all[k];
 }
 
 // Energy density of liquid-crystal site i split in its components [phase,
@@ -379,6 +410,28 @@ hipError_t launch_march(const MarchArgs<R>& a, int mode, int terms, int tile, hi
 }
 
 template <typename R>
+hipError_t launch_materialize_batch(const MarchArgs<R>* descs, int count, long long maxSites, hipStream_t s) {
+    const unsigned blocks = unsigned(std::max<long long>(1, std::min<long long>((5 * maxSites + 1023) / 1024, 256)));
+    // at most 65,535 lattices per grid row
+    for (int first = 0; first < count; first += 65535) {
+        const int m = std::min(count - first, 65535);
+        hipLaunchKernelGGL(materialize_batch_kernel<R>, dim3(blocks, m), dim3(256), 0, s, descs + first);
+    }
+    hipLaunchKernelGGL(materialized_kernel<R>, dim3((count + 63) / 64), dim3(64), 0, s, descs, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_gather_ctrls(const FinalizeDesc* descs, Ctrl* all, int count, hipStream_t s) {
+    hipLaunchKernelGGL(gather_ctrls_kernel, dim3((count + 63) / 64), dim3(64), 0, s, descs, all, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_scatter_ctrls(const FinalizeDesc* descs, const Ctrl* all, int count, hipStream_t s) {
+    hipLaunchKernelGGL(scatter_ctrls_kernel, dim3((count + 63) / 64), dim3(64), 0, s, descs, all, count);
+    return hipGetLastError();
+}
+
+template <typename R>
 void launch_boundary(const BoundaryArgs<R>& a, int mode, int terms, hipStream_t s) {
     const bool lanes = boundary_lanes(terms, a.nsites);
     const int blocks = boundary_blocks(a.nsites, lanes);
@@ -457,6 +510,7 @@ void launch_defects(const R* q, const SiteType* types, long long n, int kind, do
 #define QMIN_INSTANTIATE(R)                                                                                      \
     template hipError_t launch_march<R>(const MarchArgs<R>&, int, int, int, hipStream_t);                                   \
     template void launch_boundary<R>(const BoundaryArgs<R>&, int, int, hipStream_t);                             \
+    template hipError_t launch_materialize_batch<R>(const MarchArgs<R>*, int, long long, hipStream_t);            \
     template void launch_materialize<R>(StateSet<R>, StateSet<R>, long long, Ctrl*, hipStream_t);                \
     template int launch_energy<R>(const R*, const SiteType*, const DevObject*, int, int, int, const EnergyConst&,   \
                                   double*, hipStream_t);                                                        \
