@@ -186,8 +186,8 @@ static int enqueue_pass(qm_ensemble* E, int mode, int terms) {
 
 // The lattices' control blocks to their host copies and back, one transfer for
 // all of them (three and more transfers and their waits per lattice made a call of
-// 96 iterations over 40 lattices 29.3 ms instead of 25.5, with the velocities below, one launch for all
-// as well).  The lattices' own streams have nothing queued.
+// 96 iterations over 40 lattices 29.3 ms instead of 25.5, with one launch for the
+// velocities below).  The lattices' own streams have nothing queued.
 static int pull_ctrls(qm_ensemble* E) {
     const int count = (int)E->lats.size();
     std::vector<Ctrl> all(count);
