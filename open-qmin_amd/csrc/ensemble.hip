@@ -123,6 +123,7 @@ static int build_descs(qm_ensemble* E, const qm_ldg* f, const qm_fire* params) {
         md[k].gate = 0;
         bd[k].gate = 0;
         const int bb = boundary_blocks(L->nBoundary, E->lanes);
+        if (int rc = partials_fit(L, (long long)md[k].nblocks + bb)) return rc;
         for (int j = 0; j < md[k].nblocks; ++j) mlog[tile].push_back(make_int2(k, j));
         for (int j = 0; j < bb; ++j) blog.push_back(make_int2(k, j));
         fd[k].ctrl = L->dCtrl;

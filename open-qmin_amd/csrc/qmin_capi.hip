@@ -1070,9 +1070,12 @@ static int upload_weights(qm_lattice* L, const qm_ldg* f) {
 // Nesterov L1..L3 40^3 23 and 16, 64^3 26 and 21, 96^3 48 and 50; Adam L1 64^3
 // 24 and 25, 80^3 40 and 41; Nesterov L6 104^3 91 and 73.  FP32 crosses at the
 // same sizes or above.
+static bool block_sized(const qm_lattice* L, int mode) {
+    return L->n <= (L->terms == kMultiL6 ? 1200000 : (mode == kFire ? 900000 : 400000));
+}
+
 static bool takes_blocks(const qm_lattice* L, int mode) {
-    const long long most = L->terms == kMultiL6 ? 1200000 : (mode == kFire ? 900000 : 400000);
-    return L->tileOverride < 0 && L->zchunkOverride == 0 && L->n <= most;
+    return L->tileOverride < 0 && L->zchunkOverride == 0 && block_sized(L, mode);
 }
 
 int qmin::active_tile(const qm_lattice* L, int mode) {
@@ -1215,6 +1218,14 @@ static int nontemporal_stores(const qm_lattice* L, int mode, int fields) {
     return bytes > 256e6;
 }
 
+// Whether `slots` partial sums of three doubles fit the lattice's buffer
+// (prepare sizes it); asked before every pass that writes them there.
+int qmin::partials_fit(const qm_lattice* L, long long slots) {
+    if (3 * (size_t)slots <= L->partialsCap) return QM_OK;
+    return fail(QM_ESTATE, "a pass of " + std::to_string(slots) + " partial sums on a lattice with room for " +
+                               std::to_string(L->partialsCap / 3));
+}
+
 // One pass (force only or one FIRE iteration); kernels only, no host sync.
 // partials: the work-group partial sums (null: the lattice's own buffer)
 template <typename R>
@@ -1249,6 +1260,8 @@ static int run_pass(qm_lattice* L, const qm_ldg* f, int mode, const FireConst& f
         ma.chain.fire = fire;
         ma.chain.trace = L->dTrace;
     }
+    if (mode != kForce && !partials)
+        if (int rc = partials_fit(L, (chained >= 0 ? 2 : 1) * ((long long)ma.nblocks + boundary_slots(L)))) return rc;
     ma.gate = gated ? 1 : 0;
     ba.gate = ma.gate;
     ma.storeF = storeF ? 1 : 0;
@@ -1310,6 +1323,7 @@ static int time_march(qm_lattice* L, const qm_ldg* f, int reps, double* ms) {
     FireConst fire{};
     const int terms = terms_of(f), tile = active_tile(L, kFire);
     fill_args<R>(L, f, ma, ba, fire, tile);
+    if (int rc = partials_fit(L, ma.nblocks)) return rc;
     ma.nt = nontemporal_stores(L, kFire, 6);
     auto launch = [&]() {
         return is_stream_tile(tile) ? launch_fire_stream<R>(ma, terms, tile, L->stream)
@@ -1388,10 +1402,9 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
 // work-group.  Iteration with boundary, FP64: 24^3, L1, 16.4 against 14.2 us,
 // 50^3, L3, 27.4 against 26.5, 64^3, L3, 33.1 against 38.8 (FP32: 17.4 against
 // 15.2, 23.6 against 22.3, 27.3 against 26.9; 80^3 38 against 46).
-static bool chains_fire(const qm_lattice* L) {
-    constexpr long long kChainSites = 1 << 17;
-    return active_tile(L, kFire) == kBlock && L->n <= kChainSites;
-}
+constexpr long long kChainSites = 1 << 17;
+
+static bool chains_fire(const qm_lattice* L) { return active_tile(L, kFire) == kBlock && L->n <= kChainSites; }
 
 int qmin::prepare(qm_lattice* L, const qm_ldg* f) {
     if (!L || !f) return fail(QM_EINVAL, "null handle");
@@ -1400,13 +1413,15 @@ int qmin::prepare(qm_lattice* L, const qm_ldg* f) {
         return fail(QM_ESTATE, "the force uses a spatially varying field but the lattice has none");
     if (int rc = refresh_types(L)) return rc;
     if (int rc = upload_weights(L, f)) return rc;
-    // room for the smallest z chunk (4 planes) the fused pass may pick
+    // room for every pass a lattice of this size may take, whatever tile and z
+    // chunk are set on it now (the autotuner changes them between passes): any
+    // tile with the smallest z chunk (4 planes), blocks, and chained blocks
     long long worst = 0;
     for (int t = 0; t < kNumTiles; ++t) worst = std::max(worst, tile_columns(L, t) * ((L->lz + 3) / 4));
     size_t need = 3 * (size_t)(worst + boundary_slots(L));
-    if (takes_blocks(L, kFire) || takes_blocks(L, kForce)) {
+    if (block_sized(L, kFire) || block_sized(L, kForce)) {
         const long long blocks = tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ);
-        need = std::max(need, (chains_fire(L) ? 2 : 1) * 3 * (size_t)(blocks + boundary_slots(L)));
+        need = std::max(need, (L->n <= kChainSites ? 2 : 1) * 3 * (size_t)(blocks + boundary_slots(L)));
     }
     return ensure_partials(L, need);
 }
@@ -1430,6 +1445,7 @@ static int step_pass_t(qm_lattice* L, const qm_ldg* f, int mode, const StepArgs&
     ba.step = step;
     ma.storeF = storeF ? 1 : 0;
     ma.nt = nontemporal_stores(L, mode, mode == kAdamStep ? 4 : 3);
+    if (int rc = partials_fit(L, (long long)ma.nblocks + boundary_slots(L))) return rc;
     HIP_TRY(launch_step<R>(ma, ba, mode, terms_of(f), tile, L->stream));
     *slots = (long long)ma.nblocks + boundary_slots(L);
     return QM_OK;

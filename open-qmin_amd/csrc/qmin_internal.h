@@ -116,6 +116,7 @@ int push_ctrl(qm_lattice* L);
 // synchronous copy ordered after the work queued on the lattice's stream
 hipError_t copy_on(qm_lattice* L, void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
 int ensure_partials(qm_lattice* L, size_t count);
+int partials_fit(const qm_lattice* L, long long slots);
 int64_t n_active(const qm_lattice* L);
 // stencil variant of a force computer (kOneConstant .. kMultiL6)
 int terms_of(const qm_ldg* f);
