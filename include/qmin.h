@@ -76,9 +76,10 @@ int qm_lattice_set_tile(qm_lattice* lat, int tile);
  * times the fused FIRE pass with HIP events for every tile shape and z chunks
  * {automatic, 8, 16, 32, 64} on the lattice's current state (which it leaves
  * unchanged), keeps the fastest on the lattice and returns it (any output may be
- * NULL).  Where a small lattice's own choice, the block pass, is faster than all
- * of them, the lattice keeps that, and ms is its time.  Explicit, so that a run's
- * reduction order does not depend on timing. */
+ * NULL).  It chooses among tile shapes only: a small lattice's block pass, which
+ * qm_lattice_set_tile(lat, -1) with qm_lattice_set_zchunk(lat, 0) returns to, is
+ * mostly faster there than all of them.  Explicit, so that a run's reduction order
+ * does not depend on timing. */
 int qm_lattice_autotune(qm_lattice* lat, qm_ldg* f, int* tile, int* zchunk, double* ms);
 /* converts the device state (Q, v, F) to the other storage precision, e.g. for an
  * FP64 polish after an FP32 minimization; minimizers bound to the lattice other

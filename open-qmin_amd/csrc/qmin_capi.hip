@@ -1347,7 +1347,9 @@ static int time_march(qm_lattice* L, const qm_ldg* f, int reps, double* ms) {
 
 // Tile autotuner (the role of the reference's kernelTuner, kernelTuner.cpp:5-125,
 // measured with HIP events on the library's stream instead of host clocks):
-// every compiled tile shape x z chunks {automatic, 8, 16, 32, 64}.
+// every compiled tile shape x z chunks {automatic, 8, 16, 32, 64}.  What it keeps
+// on the lattice is what it returns.  The block pass of small lattices is no tile
+// that it could return, so it is not among them.
 int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, double* msOut) {
     if (int rc = prepare(L, f)) return rc;
     if (int rc = sync_ctrl_to_host(L)) return rc;
@@ -1357,27 +1359,18 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
         L->hCtrl.done = 0;
         if (int rc = push_ctrl(L)) return rc;
     }
+    const int savedTile = L->tileOverride, savedZ = L->zchunkOverride;
     const int reps = L->n >= (1 << 22) ? 5 : 20;
-    double best = 1e30, blocks = 1e30;
-    int bestTile = 0, bestZ = 0;
-    // the block pass of a small lattice is no tile that can be set: where it is
-    // the fastest, the lattice goes on choosing by itself
-    L->tileOverride = -1;
-    L->zchunkOverride = 0;
-    if (active_tile(L, kFire) == kBlock) {
-        const int rc = L->precision == QM_FP64 ? time_march<double>(L, f, reps, &blocks)
-                                               : time_march<float>(L, f, reps, &blocks);
-        if (rc) return rc;
-    }
-    for (int tile = 0; tile < kNumTiles; ++tile) {
+    double best = 1e30;
+    int bestTile = 0, bestZ = 0, rc = QM_OK;
+    for (int tile = 0; tile < kNumTiles && rc == QM_OK; ++tile) {
         for (int zc : {0, 8, 16, 32, 64}) {
             if (zc > L->lz) continue;
             L->tileOverride = tile;
             L->zchunkOverride = zc;
             double ms = 0;
-            int rc = L->precision == QM_FP64 ? time_march<double>(L, f, reps, &ms)
-                                             : time_march<float>(L, f, reps, &ms);
-            if (rc) return rc;
+            rc = L->precision == QM_FP64 ? time_march<double>(L, f, reps, &ms) : time_march<float>(L, f, reps, &ms);
+            if (rc) break;
             if (ms < best) {
                 best = ms;
                 bestTile = tile;
@@ -1385,15 +1378,16 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
             }
         }
     }
-    L->tileOverride = blocks < best ? -1 : bestTile;
-    L->zchunkOverride = blocks < best ? 0 : bestZ;
+    L->tileOverride = rc == QM_OK ? bestTile : savedTile;
+    L->zchunkOverride = rc == QM_OK ? bestZ : savedZ;
     if (savedDone) {
         L->hCtrl.done = savedDone;
-        if (int rc = push_ctrl(L)) return rc;
+        if (int r2 = push_ctrl(L)) return r2;
     }
+    if (rc) return rc;
     if (tileOut) *tileOut = bestTile;
     if (zchunkOut) *zchunkOut = bestZ;
-    if (msOut) *msOut = std::min(best, blocks);
+    if (msOut) *msOut = best;
     return QM_OK;
 }
 

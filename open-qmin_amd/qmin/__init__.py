@@ -231,12 +231,14 @@ class Lattice:
         _check(self.lib.qm_lattice_load_hfield(self.h, str(path).encode()))
 
     def set_tile(self, tile):
-        """Tile shape of the fused pass: -1 automatic, 0 = 32x8, 1 = 64x4, 2 = 32x16, 3 = 64x8."""
+        """Tile shape of the fused pass: -1 automatic (16x4x4 blocks on small lattices), 0 = 32x8, 1 = 64x4, 2 = 32x16, 3 = 64x8."""
         _check(self.lib.qm_lattice_set_tile(self.h, tile))
 
     def autotune(self, force):
         """Pick the fastest tile shape and z chunk of the fused FIRE pass for this
-        lattice and force (timed on the current state, which is unchanged)."""
+        lattice and force (timed on the current state, which is unchanged); they are
+        set on the lattice and returned with the pass's time in ms.  Small lattices
+        are mostly faster with the automatic choice, set_tile(-1) and set_zchunk(0)."""
         t, z, ms = ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
         _check(self.lib.qm_lattice_autotune(self.h, force.h, ctypes.byref(t), ctypes.byref(z), ctypes.byref(ms)))
         return t.value, z.value, ms.value
