@@ -1313,11 +1313,13 @@ __global__ void __launch_bounds__(kBoundaryThreads) boundary_batch_kernel(
     boundary_body<R, MODE, TERMS, LANES>(descs[lat], blk);
 }
 
-// The kernels of a force's stencil variant; neither pass distinguishes L1..L3
-// from L1..L4, and the one-constant pass always takes the lanes.
+// The kernels of a force's stencil variant; neither form distinguishes L1..L3
+// from L1..L4.
 template <typename R, int MODE>
 const void* boundary_fn(int terms, bool lanes) {
-    if (terms == kOneConstant) return reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kOneConstant, true>);
+    if (terms == kOneConstant)
+        return lanes ? reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kOneConstant, true>)
+                     : reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kOneConstant, false>);
     if (terms == kMultiL6)
         return lanes ? reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiL6, true>)
                      : reinterpret_cast<const void*>(&boundary_kernel<R, MODE, kMultiL6, false>);

@@ -379,7 +379,9 @@ hipError_t launch_march_batch(const MarchArgs<R>* descs, const int2* map, int bl
 
 template <typename R, int MODE>
 static const void* boundary_batch_fn(int terms, bool lanes) {
-    if (terms == kOneConstant) return reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kOneConstant, true>);
+    if (terms == kOneConstant)
+        return lanes ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kOneConstant, true>)
+                     : reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kOneConstant, false>);
     if (terms == kMultiL6)
         return lanes ? reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiL6, true>)
                      : reinterpret_cast<const void*>(&boundary_batch_kernel<R, MODE, kMultiL6, false>);

@@ -93,19 +93,24 @@ constexpr int kBoundaryGroup = kBoundaryThreads / kBoundaryLanes;   // sites of 
 constexpr int kBoundaryCases = 27;
 
 // Whether the boundary pass gives a site eight lanes (boundary_lanes_body) or one
-// (boundary_site_body).  FIRE iterations with lanes and with one lane per site
-// (us, FP64 unless noted): L1..L3 50^3, 6,500 sites, 27 and 40; 96^3, 23,000
-// sites, 78 and 83; L1..L6 144 x 128 x 100, 38,000 sites, 167 and 176; L1..L3
-// Nesterov 192 x 150 x 130, 60,000 sites, 196 and 187; FP32 203 x 176 x 161,
-// 73,000 sites, 332 and 322; 256^3, 135,000 sites, 903 and 866: there the
-// loads, which eight lanes scatter over more lines, set the pace.  The
-// one-constant pass loads little and is never slower with lanes.
-constexpr long long kLanesSites = 40960;
-__host__ __device__ inline bool boundary_lanes(int terms, long long nsites) {
-    return terms == 0 || nsites <= kLanesSites;
+// (boundary_site_body).  Few sites leave the chip idle, and the length of one
+// wave's path decides: lanes.  Many fill it, and the loads, which eight lanes
+// scatter over more lines, set the pace.  FIRE iterations with lanes less those
+// with one lane per site (us; walls across z, then spheres; FP64 / FP32):
+//   L1      6,400 sites  -4 / -3 (spheres), 16,200  +1 / +0.5, 18,400  +2 / +1
+//           and +1 / 0, 32,800  +4 / +3, 80,000  +11 / +9, 131,000  +19 / +15
+//   L1..L3  6,400  -10 / -11 (spheres), 16,200  0 / -1, 18,400  +2 / 0 and
+//           0 / 0, 33,000  +6 / +4, 80,000  +17 / +13 and (83,000) 0 / +9
+//   L1..L6  6,400  -27 / -23 (spheres), 16,200  -1 / -1, 18,400  +2 / +2 and
+//           -7 / -3, 22,800  +1 / +8 (spheres), 33,000  +8 / +7, 41,000  +14 / +26
+//           (spheres), 131,000  +42 / +43
+// Ensembles, by the sum of their lattices' sites: the same line, to 4%.
+constexpr long long kLanesSitesOne = 16384, kLanesSites = 18432;
+inline bool boundary_lanes(int terms, long long nsites) {
+    return nsites <= (terms == 0 ? kLanesSitesOne : kLanesSites);
 }
 // work-groups of the boundary pass over nsites sites
-__host__ __device__ inline int boundary_blocks(long long nsites, bool lanes) {
+inline int boundary_blocks(long long nsites, bool lanes) {
     const int per = lanes ? kBoundaryGroup : kBoundaryThreads;
     return int((nsites + per - 1) / per);
 }
