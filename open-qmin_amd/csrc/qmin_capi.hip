@@ -1718,9 +1718,10 @@ FireConst qmin::fire_const(const qm_fire* m, const qm_lattice* L) {
 // library runs on holds its own copy until the process ends.  Every slot a pass
 // reads is written by that pass first, so nothing has to start at zero; calls
 // that overlap on one GPU share the array and race.
-constexpr long long kScratchSlots = 65536;   // partial-sum slots of 3 doubles: 1.5 MiB, a boundary pass
-constexpr long long kScratchSites = 128;     // counted with one slot per 128 sites; where its work-groups take
-constexpr long long kScratchMore = 1 << 17;  // fewer, they have room of their own
+// A lattice is refused by its work-groups with one lane per boundary site; where
+// the boundary pass takes eight, its further work-groups have room of their own.
+constexpr long long kScratchSlots = 65536;   // partial-sum slots of 3 doubles: 1.5 MiB
+constexpr long long kScratchMore = kLanesSites / kBoundaryGroup;
 constexpr int kScratchDevices = 64;
 static __device__ __align__(256) double scratch[3 * (kScratchSlots + kScratchMore)];
 static std::mutex g_scratchMutex;
@@ -1754,17 +1755,17 @@ static int prepare_noalloc(qm_lattice* L, const qm_ldg* f, double** partials) {
     if (f->hvarOn && !L->dHField)
         return fail(QM_ESTATE, "the force uses a spatially varying field but the lattice has none");
     L->terms = terms_of(f);
-    long long need = 0;
+    long long need = 0, slots = 0;
     for (int mode : {kForce, kFire}) {
         choose_zchunk(L, mode, L->terms);
-        const long long boundary = std::max(1LL, (L->nBoundary + kScratchSites - 1) / kScratchSites);
-        need = std::max(need, march_blocks(L, mode) + boundary);
+        const long long march = march_blocks(L, mode);
+        need = std::max(need, march + std::max(1, boundary_blocks(L->nBoundary, false)));
+        slots = std::max(slots, march + boundary_slots(L));
     }
-    long long slots = need + boundary_slots(L);
     // chained passes alternate between two sets (their lattices' fit easily)
-    if (chains_fire(L)) slots = std::max<long long>(slots, 2 * (march_blocks(L, kFire) + boundary_slots(L)));
+    if (chains_fire(L)) slots = std::max(slots, 2 * ((long long)march_blocks(L, kFire) + boundary_slots(L)));
     if (need > kScratchSlots || slots > kScratchSlots + kScratchMore)
-        return fail(QM_EINVAL, "the lattice needs " + std::to_string(need) + " partial-sum slots; the "
+        return fail(QM_EINVAL, "the lattice needs " + std::to_string(std::max(need, slots)) + " partial-sum slots; the "
                                "allocation-free call holds at most " + std::to_string(kScratchSlots));
     if (int rc = upload_weights(L, f)) return rc;
     return scratch_for(L, partials);
