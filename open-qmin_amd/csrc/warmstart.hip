@@ -852,7 +852,8 @@ int qm_ws_conv_forward(const void* x, int cin, const void* wt, const float* bias
 int qm_ws_conv_wgrad(const void* g, int cout, const void* x, int cin, int reluIn, int lx, int ly, int lz, int dil,
                      float* part, long long chunk, float* dw, void* stream) {
     if (!channels_ok(cin) || !channels_ok(cout)) return fail(QM_EINVAL, "channels must be 16, 32 or 64");
-    if (!g || !x || !part || !dw || chunk < 16 || chunk % 16) return fail(QM_EINVAL, "bad weight-gradient argument");
+    if (!g || !x || !part || !dw || lx < 1 || ly < 1 || lz < 1 || chunk < 16 || chunk % 16)
+        return fail(QM_EINVAL, "bad weight-gradient argument");
     WgradArgs a{};
     a.g = static_cast<const uint16_t*>(g);
     a.x = static_cast<const uint16_t*>(x);
