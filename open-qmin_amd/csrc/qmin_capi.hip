@@ -309,6 +309,8 @@ int qm_lattice_create(int lx, int ly, int lz, int precision, qm_lattice** out) {
     L->realSize = precision == QM_FP64 ? 8 : 4;
     L->types.assign(n, 0);
     HIP_TRY(hipGetDevice(&L->device));
+    if (hipDeviceGetAttribute(&L->numCUs, hipDeviceAttributeMultiprocessorCount, L->device) != hipSuccess || L->numCUs <= 0)
+        L->numCUs = 256;
     HIP_TRY(hipStreamCreateWithFlags(&L->ownStream, hipStreamNonBlocking));
     L->stream = L->ownStream;
     HIP_TRY(hipMalloc(&L->dTypes, n * sizeof(SiteType)));
@@ -1062,20 +1064,73 @@ static int upload_weights(qm_lattice* L, const qm_ldg* f) {
 // default of its kind.
 //
 // Small lattices take the block pass (block_body), unless a tile or z chunk is
-// set: up to 1.2 million sites with L6, 0.9 million for other FIRE passes, 0.4
-// million for other force passes and the Adam and Nesterov passes, which the
-// block's halo costs more.  Per iteration, marching and in blocks (us, FP64):
-// FIRE L1..L3 40^3 27 and 18, 64^3 33 and 27, 80^3 51 and 43, 96^3 65 and 64,
-// 112^3 103 and 128; FIRE L6 96^3 68 and 67, 104^3 101 and 91, 112^3 111 and 127;
-// Nesterov L1..L3 40^3 23 and 16, 64^3 26 and 21, 96^3 48 and 50; Adam L1 64^3
-// 24 and 25, 80^3 40 and 41; Nesterov L6 104^3 91 and 73.  FP32 crosses at the
-// same sizes or above.
-static bool block_sized(const qm_lattice* L, int mode) {
-    return L->n <= (L->terms == kMultiL6 ? 1200000 : (mode == kFire ? 900000 : 400000));
+// set (blocks_pay).
+
+// z chunk of a pass over `columns` tile columns with `slots` work-groups at once,
+// and (planes) the planes that the longest sequence of them passes, halos included.
+static int z_chunk(int lz, long long columns, long long slots, bool stream, long long* planes = nullptr) {
+    auto cost = [&](int zc) {
+        const long long groups = columns * ((lz + zc - 1) / zc);
+        return (groups + slots - 1) / slots * (zc + 4);   // a chunk of zc planes passes zc + 4
+    };
+    const long long chunks = std::max(1LL, slots / columns);
+    const int once = std::max(4, std::min((int)((lz + chunks - 1) / chunks), lz));
+    int best = once;
+    // The pass that keeps only Q and v has one work-group per CU: where one round
+    // of them would leave many CUs idle, several shorter ones are better (200^3
+    // FP64, 182 work-groups of 100 planes: 574 us; 455 of 40: 485; 192^3 399 and
+    // 388).  The marching passes gain nothing so (220^3 FP32: 394 and 437 us).
+    if (stream)
+        for (int zc = once - 1; zc >= 12; --zc)
+            if (cost(zc) < 0.95 * cost(once) && cost(zc) < cost(best)) best = zc;
+    if (planes) *planes = cost(best);
+    return best;
+}
+
+// Whether the block pass is the faster one, for a lattice of B blocks of 16 x 4 x 4
+// sites.  Its time grows with B (1024 run at once, in FP64 without L6 25 to 27 us a
+// FIRE iteration, 15 us more per further 1000), that of the marching passes
+// with the planes that their z chunks pass one after the other.  FIRE iterations
+// without boundary sites, in blocks and marching (us):
+//   FP64 L1     64^3 26 and 26, 70^3 33 and 30, 86^3 52 and 43, 96^3 62 and 54;
+//        L1..L3 64^3 27 and 31, 70^3 36 and 34, 86^3 54 and 45, 96^3 65 and 55;
+//        L1..L6 64^3 31 and 36, 80^3 50 and 47, 96^3 71 and 64
+//   FP32 L1     64^3 20 and 20, 70^3 27 and 24, 96^3 42 and 33;
+//        L1..L3 64^3 21 and 23, 80^3 30 and 31, 96^3 43 and 36;
+//        L1..L6 80^3 33 and 38, 86^3 44 and 44, 96^3 48 and 45
+// Against the FP64 FIRE pass that keeps only Q and v, which takes 4.7 (L1) and
+// 5.4 us per plane, the line moves with its planes: 256 x 256 x 13 (4096 blocks, 11
+// planes) L1..L3 76 and 60, 200 x 200 x 20 (3250, 14 planes) 61 and 75, 128 x 128 x
+// 32 (2048, 8) 44 and 47, L1 40 and 38.  FP32 marching tiles are 64 sites wide, of
+// which short rows leave most idle: 17 x 150 x 150 L1 29 and 38.
+// Adam and Nesterov, whose halo costs more in blocks: Nesterov FP64 L1 70^3 23 and
+// 22, L1..L3 76^3 29 and 31, 17 x 150 x 150 33 and 30, L1..L6 80^3 37 and 41,
+// 86^3 48 and 42, 96^3 54 and 57, 150 x 150 x 30 49 and 43; FP32 L1 100 x 100 x 40
+// 21 and 18, L1..L3 22 and 21, L1..L6 96^3 37 and 42, 512 x 512 x 3 36 and 29.
+constexpr long long kBlockSites = 900000, kBlockStepSites = 400000;   // the most measured
+
+static bool blocks_pay(const qm_lattice* L, int mode) {
+    if (L->n <= 1 << 17) return true;
+    const bool one = L->terms == kOneConstant, l6 = L->terms == kMultiL6, fp32 = L->precision == QM_FP32;
+    if (L->n > (mode == kFire || l6 ? kBlockSites : kBlockStepSites)) return false;
+    long long most;
+    if (mode != kFire) {
+        most = l6 ? (fp32 ? 3600 : 2000) : one ? (fp32 ? 1280 : 1536) : (fp32 ? 1536 : 2400);
+    } else if (l6) {
+        most = fp32 ? 2000 : 1536;
+    } else if (march_tile(L, kFire) == kStream32x16) {
+        long long planes;
+        z_chunk(L->lz, tile_columns(L, kStream32x16), L->numCUs, true, &planes);
+        most = one ? 310 * planes - 800 : 344 * planes - 682;
+    } else {
+        most = fp32 && one ? 1024 : 1280;
+    }
+    if (fp32 && 3 * L->lx <= kTileTX[kTile64x4]) most = std::max(most, 3600LL);
+    return tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ) <= most;
 }
 
 static bool takes_blocks(const qm_lattice* L, int mode) {
-    return L->tileOverride < 0 && L->zchunkOverride == 0 && block_sized(L, mode);
+    return L->tileOverride < 0 && L->zchunkOverride == 0 && blocks_pay(L, mode);
 }
 
 int qmin::active_tile(const qm_lattice* L, int mode) {
@@ -1158,13 +1213,6 @@ static void choose_zchunk(qm_lattice* L, int mode, int terms) {
         L->zchunk = L->zchunkOverride;
         return;
     }
-    if (L->numCUs == 0) {
-        int dev = 0;
-        hipDeviceProp_t prop;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-            L->numCUs = prop.multiProcessorCount;
-        if (L->numCUs <= 0) L->numCUs = 256;
-    }
     const int tile = active_tile(L, mode);
     if (tile == kBlock) {
         const int nbz = (L->lz + Block::BZ - 1) / Block::BZ;
@@ -1178,22 +1226,7 @@ static void choose_zchunk(qm_lattice* L, int mode, int terms) {
     else
         perCU = L->precision == QM_FP64 ? march_blocks_per_cu<double>(mode, terms, tile)
                                         : march_blocks_per_cu<float>(mode, terms, tile);
-    const long long columns = tile_columns(L, tile), slots = (long long)perCU * L->numCUs;
-    auto cost = [&](int zc) {
-        const long long groups = columns * ((L->lz + zc - 1) / zc);
-        return (double)((groups + slots - 1) / slots) * (zc + 4);   // a chunk of zc planes passes zc + 4
-    };
-    const long long chunks = std::max(1LL, slots / columns);
-    const int once = std::max(4, std::min((int)((L->lz + chunks - 1) / chunks), L->lz));
-    int best = once;
-    // The pass that keeps only Q and v has one work-group per CU: where one round
-    // of them would leave many CUs idle, several shorter ones are better (200^3
-    // FP64, 182 work-groups of 100 planes: 574 us; 455 of 40: 485; 192^3 399 and
-    // 388).  The marching passes gain nothing so (220^3 FP32: 394 and 437 us).
-    if (is_stream_tile(tile))
-        for (int zc = once - 1; zc >= 12; --zc)
-            if (cost(zc) < 0.95 * cost(once) && cost(zc) < cost(best)) best = zc;
-    L->zchunk = best;
+    L->zchunk = z_chunk(L->lz, tile_columns(L, tile), (long long)perCU * L->numCUs, is_stream_tile(tile));
 }
 
 static int march_blocks(const qm_lattice* L, int mode) {
@@ -1396,7 +1429,7 @@ int qm_lattice_autotune(qm_lattice* L, qm_ldg* f, int* tileOut, int* zchunkOut, 
 // work-group.  Iteration with boundary, FP64: 24^3, L1, 16.4 against 14.2 us,
 // 50^3, L3, 27.4 against 26.5, 64^3, L3, 33.1 against 38.8 (FP32: 17.4 against
 // 15.2, 23.6 against 22.3, 27.3 against 26.9; 80^3 38 against 46).
-constexpr long long kChainSites = 1 << 17;
+constexpr long long kChainSites = 1 << 17;   // of which all take blocks
 
 static bool chains_fire(const qm_lattice* L) { return active_tile(L, kFire) == kBlock && L->n <= kChainSites; }
 
@@ -1413,7 +1446,7 @@ int qmin::prepare(qm_lattice* L, const qm_ldg* f) {
     long long worst = 0;
     for (int t = 0; t < kNumTiles; ++t) worst = std::max(worst, tile_columns(L, t) * ((L->lz + 3) / 4));
     size_t need = 3 * (size_t)(worst + boundary_slots(L));
-    if (block_sized(L, kFire) || block_sized(L, kForce)) {
+    if (L->n <= kBlockSites) {
         const long long blocks = tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ);
         need = std::max(need, (L->n <= kChainSites ? 2 : 1) * 3 * (size_t)(blocks + boundary_slots(L)));
     }
