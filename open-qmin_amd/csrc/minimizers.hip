@@ -498,15 +498,19 @@ static int drive(VecMinimizer& s, qm_lattice* L, Enqueue&& enqueue) {
 // so only a pass that is known to be the last stores them (40 of the 201 B that
 // an FP64 Nesterov pass would move per site); where the tolerance stopped the run
 // before its limit, they are computed again from the Q they belong to.  A run of
-// a few iterations stores them always.  Nesterov, L1..L3, 192 x 150 x 130 in
-// FP64: 158 against 190 us per iteration.
-constexpr int kFewIterations = 4;
+// a few iterations stores them always, and one with a tolerance in its first two,
+// after which the passes have saved what that computation takes: Nesterov, L1..L3,
+// 150^3 in FP64, stopped after one iteration 817 us, with the computation 852.  Without
+// stores Nesterov, L1..L3, 192 x 150 x 130 in FP64 takes 158 us per iteration,
+// with them 190.
+constexpr int kFewIterations = 4, kFirstIterations = 2;
 template <typename Enqueue>
 static int drive_steps(VecMinimizer& s, qm_lattice* L, const qm_ldg* f, Enqueue&& enqueue) {
     const int begin = s.iterations;
-    const bool always = s.maxIter - begin <= kFewIterations;
-    const int rc = drive(s, L, [&](int iteration) { return enqueue(always || iteration + 1 >= s.maxIter); });
-    if (s.iterations > begin && s.iterations < s.maxIter && !always)
+    const int first = s.maxIter - begin <= kFewIterations ? kFewIterations : s.fc > 0 ? kFirstIterations : 0;
+    const int rc =
+        drive(s, L, [&](int iteration) { return enqueue(iteration - begin < first || iteration + 1 >= s.maxIter); });
+    if (s.iterations - begin > first && s.iterations < s.maxIter)
         if (int rc2 = last_step_force(L, f)) return rc ? rc : rc2;
     return rc;
 }
