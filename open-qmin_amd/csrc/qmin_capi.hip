@@ -205,20 +205,31 @@ int qmin::ensure_partials(qm_lattice* L, size_t count) {
 // transposition runs on the device, through LDS so that both sides are read and
 // written in whole lines, and the host copies straight from or to the caller's
 // array: forces, energy and defects of 128 x 112 x 96 sites take 6.5 ms, with the
-// transposition on the host 18.6 ms.
+// transposition on the host 18.6 ms.  Two ranges of sizes differ:
+//  * On small lattices the transposition is cheaper on the host than its launch
+//    and, in FP32, the doubles it moves.  Reading a field, on the host and on
+//    the device (us): FP64 12^3 40 and 53, 24^3 48 and 49, 36^3 185 and 140; FP32
+//    24^3 33 and 49, 36^3 90 and 140 (as floats 99), 60^3 470 and 470 (floats).
+//    Writing one: FP64 24^3 40 and 45, 36^3 119 and 95; FP32 36^3 68 and 95, 60^3
+//    280 and 280.
+//  * An FP32 field of up to a million sites is read as floats, a piece at a time
+//    through a buffer that stays in the host's cache: 60^3 470 us, as doubles
+//    630, 100^3 3.7 ms and 4.1; beyond, into an array that has been written
+//    before, 160^3 10.4 and 9.2.
+constexpr long long kHostSites[2] = {16384, 65536};   // transposed on the host: FP64, FP32
+constexpr long long kFloatSites = 1 << 20;
 constexpr int kTransposeSites = 256;   // sites, and threads, of a work-group
 
 static unsigned transpose_blocks(long long n) { return unsigned((n + kTransposeSites - 1) / kTransposeSites); }
 
-template <typename R>
-__global__ void __launch_bounds__(kTransposeSites) sites_from_planes_kernel(const R* planes, double* sites,
-                                                                           long long n) {
-    __shared__ double t[5 * kTransposeSites];
+template <typename R, typename S>
+__global__ void __launch_bounds__(kTransposeSites) sites_from_planes_kernel(const R* planes, S* sites, long long n) {
+    __shared__ S t[5 * kTransposeSites];
     const long long i0 = (long long)blockIdx.x * kTransposeSites;
     const int count = int(min((long long)kTransposeSites, n - i0)), tid = threadIdx.x;
     if (tid < count) {
 #pragma unroll
-        for (int c = 0; c < 5; ++c) t[5 * tid + c] = double(planes[c * n + i0 + tid]);
+        for (int c = 0; c < 5; ++c) t[5 * tid + c] = S(planes[c * n + i0 + tid]);
     }
     __syncthreads();
     for (int e = tid; e < 5 * count; e += kTransposeSites) sites[5 * i0 + e] = t[e];
@@ -243,9 +254,60 @@ __global__ void __launch_bounds__(kTransposeSites) planes_from_sites_kernel(cons
 // Users hold scratchMutex, as calls that only read a lattice may overlap.
 static double* scratch_reals(const qm_lattice* L) { return static_cast<double*>(L->dSet[L->hCtrl.cur ^ 1]); }
 
+template <typename R>
+static int upload_planes(qm_lattice* L, int which, const double* aos) {
+    const long long n = L->n;
+    R* const planes = static_cast<R*>(L->dSet[L->hCtrl.cur]) + which * 5 * n;
+    if (n <= kHostSites[sizeof(R) == 4]) {
+        std::vector<R> soa(5 * n);
+        for (long long i = 0; i < n; ++i)
+            for (int c = 0; c < 5; ++c) soa[c * n + i] = R(aos[5 * i + c]);
+        HIP_TRY(copy_on(L, planes, soa.data(), 5 * n * sizeof(R), hipMemcpyHostToDevice));
+        return QM_OK;
+    }
+    std::lock_guard<std::mutex> lock(L->scratchMutex);
+    double* tmp = scratch_reals(L);
+    HIP_TRY(copy_on(L, tmp, aos, 5 * n * sizeof(double), hipMemcpyHostToDevice));
+    planes_from_sites_kernel<R><<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(tmp, planes, n);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(L->stream));
+    return QM_OK;
+}
+
+template <typename R>
+static int download_planes(qm_lattice* L, int which, double* aos) {
+    const long long n = L->n;
+    const R* const planes = static_cast<const R*>(L->dSet[L->hCtrl.cur]) + which * 5 * n;
+    if (n <= kHostSites[sizeof(R) == 4]) {
+        std::vector<R> soa(5 * n);
+        HIP_TRY(copy_on(L, soa.data(), planes, 5 * n * sizeof(R), hipMemcpyDeviceToHost));
+        for (long long i = 0; i < n; ++i)
+            for (int c = 0; c < 5; ++c) aos[5 * i + c] = double(soa[c * n + i]);
+        return QM_OK;
+    }
+    std::lock_guard<std::mutex> lock(L->scratchMutex);
+    double* tmp = scratch_reals(L);
+    if (sizeof(R) == 4 && n <= kFloatSites) {
+        float* sites = reinterpret_cast<float*>(tmp);
+        sites_from_planes_kernel<<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(planes, sites, n);
+        HIP_TRY(hipGetLastError());
+        constexpr long long kPiece = 1 << 18;
+        std::vector<float> piece(std::min(kPiece, 5 * n));
+        for (long long k = 0; k < 5 * n; k += kPiece) {
+            const long long count = std::min(kPiece, 5 * n - k);
+            HIP_TRY(copy_on(L, piece.data(), sites + k, count * sizeof(float), hipMemcpyDeviceToHost));
+            for (long long j = 0; j < count; ++j) aos[k + j] = piece[j];
+        }
+        return QM_OK;
+    }
+    sites_from_planes_kernel<<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(planes, tmp, n);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(copy_on(L, aos, tmp, 5 * n * sizeof(double), hipMemcpyDeviceToHost));
+    return QM_OK;
+}
+
 // AoS host field -> SoA device plane set (current set)
 static int upload_field(qm_lattice* L, int which, const double* aos) {
-    const long long n = L->n;
     if (which == QM_FIELD_Q) {
         // The objects' FP64 Q, restored when an FP32 state converts back to
         // FP64.  On an FP32 lattice a value equal to the kept one in FP32 is the
@@ -262,33 +324,11 @@ static int upload_field(qm_lattice* L, int which, const double* aos) {
             }
         }
     }
-    std::lock_guard<std::mutex> lock(L->scratchMutex);
-    double* tmp = scratch_reals(L);
-    HIP_TRY(copy_on(L, tmp, aos, 5 * n * sizeof(double), hipMemcpyHostToDevice));
-    if (L->precision == QM_FP64)
-        planes_from_sites_kernel<double><<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(
-            tmp, static_cast<double*>(L->dSet[L->hCtrl.cur]) + which * 5 * n, n);
-    else
-        planes_from_sites_kernel<float><<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(
-            tmp, static_cast<float*>(L->dSet[L->hCtrl.cur]) + which * 5 * n, n);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(L->stream));
-    return QM_OK;
+    return L->precision == QM_FP64 ? upload_planes<double>(L, which, aos) : upload_planes<float>(L, which, aos);
 }
 
 static int download_field(qm_lattice* L, int which, double* aos) {
-    const long long n = L->n;
-    std::lock_guard<std::mutex> lock(L->scratchMutex);
-    double* tmp = scratch_reals(L);
-    if (L->precision == QM_FP64)
-        sites_from_planes_kernel<double><<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(
-            static_cast<const double*>(L->dSet[L->hCtrl.cur]) + which * 5 * n, tmp, n);
-    else
-        sites_from_planes_kernel<float><<<transpose_blocks(n), kTransposeSites, 0, L->stream>>>(
-            static_cast<const float*>(L->dSet[L->hCtrl.cur]) + which * 5 * n, tmp, n);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(copy_on(L, aos, tmp, 5 * n * sizeof(double), hipMemcpyDeviceToHost));
-    return QM_OK;
+    return L->precision == QM_FP64 ? download_planes<double>(L, which, aos) : download_planes<float>(L, which, aos);
 }
 
 // ------------------------------------------------------------------ lattice API
