@@ -1081,6 +1081,9 @@ static int compose(qm_lattice* L, const qm_ldg* f) {
 
 static int upload_weights(qm_lattice* L, const qm_ldg* f) {
     const double want[7] = {f->L1, f->L2, f->L3, f->L4, f->L6, (double)terms_of(f), (double)L->precision};
+    // calls that only read the lattice prepare it too, and may overlap: the
+    // constants noted and the operators composed stay those of one force
+    std::lock_guard<std::mutex> lock(L->composeMutex);
     bool same = true;
     for (int k = 0; k < 7; ++k) same = same && want[k] == L->composed[k];
     if (same) return QM_OK;

@@ -42,6 +42,7 @@ struct qm_lattice {
     // the constants dW and dTerms were composed for: L1, L2, L3, L4, L6, the
     // stencil variant and the precision (NaN: none yet)
     double composed[7] = {NAN, NAN, NAN, NAN, NAN, NAN, NAN};
+    std::mutex composeMutex;              // held while they are compared or replaced
     DevObject* dObjects = nullptr;
     void* dSet[2] = {nullptr, nullptr};   // each 15 n reals: Q, U, F planes
     int32_t* dSites = nullptr;            // compacted sites finished by the boundary pass
