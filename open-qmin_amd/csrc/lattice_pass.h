@@ -331,8 +331,9 @@ __device__ __forceinline__ void fire_partials(const double* part, long long tota
 // velocity mix v = ck u + cf F, (1, 0) when none is pending and (0, 0) after a
 // reset (energyMinimizerFIRE.cpp:117-144, velocityVerlet.cpp:8-40):
 //   q + dt v + dt^2/2 F = q + (du u + df F),  v + dt/2 F = vu u + vf F.
-// One rounding of q, and the products contracted by hand, so that every pass that
-// drifts a site rounds alike.
+// One rounding of q, and the products contracted by hand, so that the marching and
+// the block passes round alike.  (The pass that keeps only Q and v drifts in a
+// form of its own, fire_stream.hip, and rounds differently.)
 template <typename R>
 struct FireMove {
     R du, df, vu, vf, hdt;

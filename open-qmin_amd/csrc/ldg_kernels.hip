@@ -1,11 +1,13 @@
 // gfx950 kernels of the lattice Landau-de Gennes minimizer.
 //
-// Fused lattice pass (march_kernel): one work-group owns a 32 x 8 column of
-// sites and marches it along a z chunk.  Each step stages one halo-padded
-// plane of the new state into a 3-plane LDS ring: in FIRE mode the pending
-// FIRE velocity mix, the velocity-Verlet drift and the first half kick are
-// applied while loading (Q' = Q + dt v + dt^2/2 F, v' = v + dt/2 F), so the
-// force at Q' is computed from LDS without another pass over HBM.  Every
+// Fused lattice pass (march_kernel, march_wide_kernel): one work-group owns a
+// column of 32 x 8 to 64 x 8 sites and marches it along a z chunk.  Each step
+// stages one halo-padded plane of the new state into a 3-plane LDS ring: in FIRE
+// mode the pending FIRE velocity mix, the velocity-Verlet drift and the first
+// half kick are applied while loading (Q' = Q + dt v + dt^2/2 F, v' = v + dt/2 F),
+// so the force at Q' is computed from LDS without another pass over HBM.  On
+// small lattices (block_kernel) a work-group stages a block of 16 x 4 x 4 sites
+// with its halo at once instead.  Every
 // site's force needs only its 3x3x3 neighbourhood minus the corners: the
 // reference's stencils use neighbour derivatives transverse to the neighbour
 // direction only (src/forces/lcForces.h:66-1043).  The second half kick and
@@ -14,11 +16,11 @@
 // pass, which keeps the rarely-needed 27-case boundary stencils out of this
 // kernel's register budget.
 //
-// Boundary pass (boundary_kernel): one thread per site of the compacted t < 0
-// list; 27-case stencils, anchoring, fields and metric.  A one-work-group
-// kernel (fire_finalize_kernel) then sums all partials in a fixed order and
-// advances the FIRE scalars on the device (energyMinimizerFIRE.cpp:77-145): no
-// host round trip.
+// Boundary pass (boundary_kernel): eight lanes or one (boundary_lanes) per site
+// of the compacted t < 0 list; 27-case stencils, anchoring, fields and metric.  A
+// one-work-group kernel (fire_finalize_kernel), or on small lattices the next
+// block pass, then sums all partials in a fixed order and advances the FIRE
+// scalars on the device (energyMinimizerFIRE.cpp:77-145): no host round trip.
 #include "lattice_pass.h"
 
 namespace qmin {

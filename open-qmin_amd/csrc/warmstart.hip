@@ -105,10 +105,12 @@ constexpr int kFwdBlock = 16;                                 // row groups take
 // current one run.  Rows in LDS are padded (8 BF16 at 64 channels, 4 below), so
 // that the 16 sites of a fragment fall on different banks.
 //
-// Bound by LDS: at the full BF16 rate a wave's 64 x 64 products would read 128 B
-// per clock and CU from it, all that it gives, before any staging.  Gathering
-// every tap's operand from L2 instead, 27 reads of each site, left the kernel
-// waiting on those gathers.  At 128^3, before and now: 64 -> 64 channels 1.46
+// Bound by latency: with two work-groups per CU (72.7 KB of LDS each at 64
+// channels) the waves wait half of their time on operand reads and on the two
+// barriers of a step, while LDS is busy 40% of the clocks (bank conflicts 14%),
+// the matrix cores 28%, the vector units 26% and the L1 18% (64 -> 64, 128^3).
+// Gathering every tap's operand from L2 instead, 27 reads of each site, left the
+// kernel waiting on those gathers.  At 128^3, before and now: 64 -> 64 channels 1.46
 // and 0.65 ms (710 TFLOP/s), 64 -> 16 0.99 and 0.36, 32 -> 64 0.78 and 0.45,
 // 16 -> 32 0.43 and 0.13 ms.  Measured and not kept: 320 slots, with which the
 // 64 -> 16 kernel has two work-groups per CU instead of three (0.52 ms); three
@@ -116,8 +118,10 @@ constexpr int kFwdBlock = 16;                                 // row groups take
 // and a raised wave priority during the taps (no difference).
 template <int NT, int KT>
 __global__ void __launch_bounds__(kWsThreads, 2) conv_fwd_kernel(ConvArgs a) {
-    // K32: 32 input channels per matrix instruction (for 64 input channels; with
-    // 32, one such step per tap ran 9% slower at 128^3 than two 16-channel ones)
+    // K32: 32 input channels per matrix instruction, for 64 input channels.  (With
+    // 32 the 16-channel form was the faster one, by 9%, in the kernel that gathered
+    // its operands; in this one the other takes 394 us against 450, 32 -> 64 at
+    // 128^3, but needs inputs of 16-byte alignment.)
     constexpr bool K32 = KT == 4;
     constexpr int CO = NT * 16, CI = KT * 16, RS = CI + (K32 ? 8 : 4);   // LDS row stride in BF16
     constexpr int CPS = CI / 8;                                          // 16-byte pieces of a site
@@ -448,8 +452,9 @@ __device__ __forceinline__ v8bf raw_operand(const Raw<PC> (&r)[8], int c) {
 // fixed order through LDS.
 // 64 x 64 channels of 302k sites: 160 us (418 TFLOP/s); staged in LDS per tap and
 // transposed there by two-byte stores it took 770 us.  Bound by the operand
-// loads through the L1 (8 KB per wave and 32 sites) and the vector work beside
-// the 16 matrix instructions they feed.
+// loads through the L1 (8 KB per wave and 32 sites: one access in 73% of the
+// clocks) and the vector work beside the 16 matrix instructions they feed (51%;
+// the matrix cores 19%).
 template <int NT, int KT>
 __global__ void __launch_bounds__(kWgThreads) conv_wgrad_kernel(WgradArgs a) {
     constexpr int CO = NT * 16, CI = KT * 16;
