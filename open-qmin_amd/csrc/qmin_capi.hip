@@ -1130,46 +1130,52 @@ static int z_chunk(int lz, long long columns, long long slots, bool stream, long
     return best;
 }
 
-// Whether the block pass is the faster one, for a lattice of B blocks of 16 x 4 x 4
-// sites.  Its time grows with B (1024 run at once, in FP64 without L6 25 to 27 us a
-// FIRE iteration, 15 us more per further 1000), that of the marching passes
-// with the planes that their z chunks pass one after the other.  FIRE iterations
-// without boundary sites, in blocks and marching (us):
-//   FP64 L1     64^3 26 and 26, 70^3 33 and 30, 86^3 52 and 43, 96^3 62 and 54;
-//        L1..L3 64^3 27 and 31, 70^3 36 and 34, 86^3 54 and 45, 96^3 65 and 55;
-//        L1..L6 64^3 31 and 36, 80^3 50 and 47, 96^3 71 and 64
-//   FP32 L1     64^3 20 and 20, 70^3 27 and 24, 96^3 42 and 33;
-//        L1..L3 64^3 21 and 23, 80^3 30 and 31, 96^3 43 and 36;
-//        L1..L6 80^3 33 and 38, 86^3 44 and 44, 96^3 48 and 45
+// Whether the block pass is the faster one.  Its time grows with the blocks of 16 x
+// 4 x 4 sites, full or not (1024 run at once, in FP64 without L6 25 to 27 us a FIRE
+// iteration, 15 us more per further 1000), that of the marching passes with the
+// sites and with the threads that tiles of 32 or 64 sites a row leave idle on them.
+// So the line is a number of blocks that rises with those idle threads; kBlockLine
+// has it by least regret over 110 shapes without boundary sites, 131,072 to 1.2
+// million sites, rows of 3 to 512: on average within 0.7% of the better choice, at
+// worst 15% (always marching 18 to 76%, at worst a factor of five).
+// FIRE iterations in blocks and marching (us):
+//   FP64 L1     64^3 26 and 26, 86^3 52 and 43, 96^3 62 and 54, 7 x 355 x 355 59 and 101
+//        L1..L3 64^3 27 and 31, 86^3 54 and 45, 96^3 65 and 55
+//        L1..L6 64^3 31 and 36, 96^3 71 and 64, 33 x 110 x 110 47 and 59
+//   FP32 L1     64^3 20 and 20, 96^3 42 and 33, 17 x 150 x 150 29 and 38
+//        L1..L3 64^3 21 and 23, 80^3 30 and 31, 96^3 43 and 36
+//        L1..L6 80^3 33 and 38, 96^3 48 and 45, 20 x 300 x 100 45 and 63
+// and Nesterov, which the blocks' halo costs more:
+//   FP64 L1 70^3 23 and 22, L1..L3 76^3 29 and 31, L1..L6 80^3 37 and 41, 86^3 48 and 42
+//   FP32 L1 100 x 100 x 40 21 and 18, L1..L3 22 and 21, L1..L6 96^3 37 and 42
 // Against the FP64 FIRE pass that keeps only Q and v, which takes 4.7 (L1) and
 // 5.4 us per plane, the line moves with its planes: 256 x 256 x 13 (4096 blocks, 11
 // planes) L1..L3 76 and 60, 200 x 200 x 20 (3250, 14 planes) 61 and 75, 128 x 128 x
-// 32 (2048, 8) 44 and 47, L1 40 and 38.  FP32 marching tiles are 64 sites wide, of
-// which short rows leave most idle: 17 x 150 x 150 L1 29 and 38.
-// Adam and Nesterov, whose halo costs more in blocks: Nesterov FP64 L1 70^3 23 and
-// 22, L1..L3 76^3 29 and 31, 17 x 150 x 150 33 and 30, L1..L6 80^3 37 and 41,
-// 86^3 48 and 42, 96^3 54 and 57, 150 x 150 x 30 49 and 43; FP32 L1 100 x 100 x 40
-// 21 and 18, L1..L3 22 and 21, L1..L6 96^3 37 and 42, 512 x 512 x 3 36 and 29.
-constexpr long long kBlockSites = 900000, kBlockStepSites = 400000;   // the most measured
+// 32 (2048, 8) 44 and 47, L1 40 and 38.
+struct BlockLine {
+    double blocks, idle, sites;   // blocks + idle (idle threads / 1000) + sites (sites / 1000), 1280 at least
+};
+constexpr BlockLine kBlockLine[2][3][2] = {
+    // FP64, FP32; L1, L1..L4, L1..L6; FIRE, other passes
+    {{{1350, 5.7, -1.9}, {1160, 3.5, 0.6}}, {{1420, 3.8, -0.1}, {1360, 1.7, 2.4}}, {{60, 15.6, -0.1}, {240, 4.5, 3.6}}},
+    {{{630, 3.0, 0.0}, {860, 2.9, 0.6}}, {{1000, 2.9, 0.3}, {1160, 3.5, 2.7}}, {{2570, 8.5, -1.8}, {1770, 7.1, 1.9}}}};
+constexpr long long kBlockSites = 1200000;   // the most measured
 
 static bool blocks_pay(const qm_lattice* L, int mode) {
     if (L->n <= 1 << 17) return true;
-    const bool one = L->terms == kOneConstant, l6 = L->terms == kMultiL6, fp32 = L->precision == QM_FP32;
-    if (L->n > (mode == kFire || l6 ? kBlockSites : kBlockStepSites)) return false;
-    long long most;
-    if (mode != kFire) {
-        most = l6 ? (fp32 ? 3600 : 2000) : one ? (fp32 ? 1280 : 1536) : (fp32 ? 1536 : 2400);
-    } else if (l6) {
-        most = fp32 ? 2000 : 1536;
-    } else if (march_tile(L, kFire) == kStream32x16) {
+    const int model = L->terms == kOneConstant ? 0 : (L->terms == kMultiL6 ? 2 : 1);
+    if (L->n > (model == 2 ? kBlockSites : mode == kFire ? 900000 : 400000)) return false;
+    const int tile = march_tile(L, mode);
+    const long long blocks = tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ);
+    if (is_stream_tile(tile)) {
         long long planes;
-        z_chunk(L->lz, tile_columns(L, kStream32x16), L->numCUs, true, &planes);
-        most = one ? 310 * planes - 800 : 344 * planes - 682;
-    } else {
-        most = fp32 && one ? 1024 : 1280;
+        z_chunk(L->lz, tile_columns(L, tile), L->numCUs, true, &planes);
+        return blocks <= (model == 0 ? 310 * planes - 800 : 344 * planes - 682);
     }
-    if (fp32 && 3 * L->lx <= kTileTX[kTile64x4]) most = std::max(most, 3600LL);
-    return tile_columns(L, kBlock) * ((L->lz + Block::BZ - 1) / Block::BZ) <= most;
+    const BlockLine& line = kBlockLine[L->precision == QM_FP32][model][mode != kFire];
+    const long long threads = tile_columns(L, tile) * kTileTX[tile] * kTileTY[tile] * L->lz;
+    const double most = line.blocks + 1e-3 * (line.idle * double(threads - L->n) + line.sites * double(L->n));
+    return blocks <= std::max(1280.0, most);
 }
 
 static bool takes_blocks(const qm_lattice* L, int mode) {
